@@ -34,8 +34,9 @@
 //            only edges whose neighbour lies in another tile of 64 elements are
 //            written (a neighbour in the same tile is read from LDS), rotating
 //            as the quadrilateral path's: stage 1 T0->T1, 2 T1->T2, 3 T2->T0
-//   geo      [E][10]: r_x, r_y, s_x, s_y, then the face normal (as the face's
-//            left element sees it) of edges 0, 1, 2
+//   geo      [E][16]: r_x, r_y, s_x, s_y, then the face normal (as the face's
+//            left element sees it) of edges 0, 1, 2, |e|/(2J) of each edge and
+//            of the neighbour's side of each (0 on a boundary)
 //   links    [E][3] int2: x = neighbour element (-1 on a boundary), y = packed
 //            neighbour edge (or BC type) | role << 3 | BC data index << 6
 //   ops      constant memory, per order: Dr, Ds [Np][Np], interp [3(p+1)][Np],
@@ -45,6 +46,7 @@
 #include "zj_host_math.hpp"
 #include "zj_kernels.hpp"
 #include "zj_riemann_vjp.hpp"
+#include "zj_tri_frag.hpp"
 #include "zj_tri_ops.hpp"
 #include "zj_viscous.hpp"
 
@@ -71,7 +73,8 @@ struct TriShape {
 
 constexpr int TILE = BLOCK / NV;  // elements per workgroup (one lane per element and variable)
 constexpr int EB = 16;            // elements per block of the state and trace layouts
-constexpr int GEO = 10;           // geometry words per element
+constexpr int GEO = 16;           // geometry words per element
+constexpr int GEO_S = 10, GEO_SN = 13;  // edge factors within them: own, the neighbour's
 
 // Operator tables of order P in constant memory, laid out for wide scalar
 // loads in the kernels' loops:
@@ -125,6 +128,13 @@ template <typename R> __device__ __forceinline__ R clf(int k);
 template <> __device__ __forceinline__ double clf<double>(int k) { return c_lf64[k]; }
 template <> __device__ __forceinline__ float clf<float>(int k) { return c_lf32[k]; }
 
+// The same operators as matrix-core tables, in device memory (vector loads).
+__device__ double d_frag64[tri::frag_offset<double>(6)];
+__device__ float d_frag32[tri::frag_offset<float>(6)];
+template <typename R> __device__ __forceinline__ const R* frag_ops();
+template <> __device__ __forceinline__ const double* frag_ops<double>() { return d_frag64; }
+template <> __device__ __forceinline__ const float* frag_ops<float>() { return d_frag32; }
+
 template <typename R> __device__ __forceinline__ R cop(int k);
 template <> __device__ __forceinline__ double cop<double>(int k) { return c_ops64[k]; }
 template <> __device__ __forceinline__ float cop<float>(int k) { return c_ops32[k]; }
@@ -165,6 +175,7 @@ struct TriArgs {
     // and the family's face liftings in c_lf
     double mu, kappa, eta;
     int lf_off;
+    int family;           // of the correction: DG, SD = GA, HU
 };
 
 __device__ __forceinline__ int link_edge(int info) { return info & 7; }
@@ -410,25 +421,416 @@ __global__ __launch_bounds__(BLOCK, (TriWaves<R, P>::value)) void tri_stage_kern
 //       trace of grad U plus eta times the lifting of this face's jumps
 //       alone at the face's points (LF_k = interp . lift of edge k)
 //   dU/dt = -(Dr Fr + Ds Fs) - sum_j lift[:, j] (s_j F^I_j - Fn_j)
-// Lanes as in tri_stage_kernel (one per element and variable), but the point
-// values (U, then Q) live in LDS, and each lane reads the four variables of a
-// point from there: the per-lane registers hold only the divergence and the
-// normal-flux sums.  A tile holds TT elements, sized so that the trace arrays
-// (U, dU/dx, dU/dy) and the point arrays (U, Qx, Qy; later the flux
-// differences) fit the LDS.  Traces across tiles carry 12 words per flux
-// point ([E][3(p+1)][12]: U, dU/dx, dU/dy).
+// Lanes as zj_tri_frag.hpp has them: a wave owns G groups of four elements,
+// lane l holds row 4 b + l/16 (solution or flux point) of element (l/4) mod 4,
+// variable l mod 4.  The operators are matrix-core products over such
+// fragments; what needs the four variables of a point together (the fluxes)
+// takes one lane per point or face point through LDS.  Traces across tiles
+// carry 12 words per flux point ([E][3(p+1)][12]: U, dU/dx, dU/dy).
+//
+// What bounds it is the latency of LDS and memory at two (FP64) to four
+// waves per SIMD, then VALU issue (about 1,400 instructions per wave of
+// eight elements) beside 4,400 (FP64) cycles of matrix-core work.  Hence no
+// branches around loads (rows in excess, in-tile edges and elements beyond
+// the mesh read a valid address and select afterwards: branches had split
+// the LDS reads into some 60 waits a wave), the operator tables in LDS (read
+// from memory they took a quarter of the kernel's time), the neighbours'
+// traces fetched a phase ahead, and two element groups per wave per operator
+// word.  500,000 elements, P3, HLLC, us a stage, scalar operands and one lane
+// per element and variable -> this: FP64 670 / 771 / 771 -> 430, FP32
+// 354 / 390 / 384 -> 241 / 272 / 277 (1.9 TB/s of the stage's traffic).
 constexpr int TWV = 12;
 
+template <typename R, int P> constexpr bool tri_visc_scalar() { return P == 1 || (P == 2 && sizeof(R) == 4); }
+
+// The workgroup: WV waves of G groups each, 4 G WV elements.
+// LDS per element: the traces of U, then one region that holds U with the
+// corrected gradient, the point fluxes in its place, and at last both traces
+// of the BR2 gradient, whose x part the face fluxes replace.
 template <typename R, int P> struct TriViscTile {
-    static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1);
-    static constexpr int bytes(int tt) { return tt * (3 * NFP + 3 * NP) * NV * (int)sizeof(R); }
-    // within 120 KiB of LDS (gfx950 gives a workgroup up to 160 KiB)
-    static constexpr int value = bytes(64) <= 122880 ? 64 : (bytes(32) <= 122880 ? 32 : 16);
-    static_assert(bytes(16) <= 122880, "the smallest tile exceeds the LDS");
+    static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1), PB = (NP + 3) / 4, FB = (NFP + 3) / 4;
+    static constexpr bool BIG = sizeof(R) == 8 && P == 5;
+    static constexpr int G = BIG ? 1 : 2, WV = BIG ? 8 : 4;
+    static constexpr int value = tri_visc_scalar<R, P>() ? 64 : 4 * G * WV;
+    // rows of an element's region: Q_x, then F_r, at 0; Q_y, then F_s, at NP; U at RU; then the
+    // gradient traces x (later the common fluxes) at 0 and y at NFP, the partner's U traces at
+    // 2 NFP.  Arrays are stored whole blocks of four rows at a time, in the order of their rows,
+    // so that the next array overwrites the rows in excess.
+    static constexpr int RU = NP + 4 * PB;
+    static constexpr int ROWS = RU + 4 * PB > 2 * NFP + 4 * FB ? RU + 4 * PB : 2 * NFP + 4 * FB;
+    static constexpr int ESF = tri::elem_stride<R>(4 * FB), ESX = tri::elem_stride<R>(ROWS);
+    static_assert(value * (ESF + ESX) * (int)sizeof(R) <= 122880, "the tile exceeds the LDS");
 };
 
+template <typename R, int P, int MODE>
+__global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stage_kernel(TriArgs<R> a) {
+    using S = TriShape<P>;
+    using TV = TriViscTile<R, P>;
+    using FO = tri::FragOps<R, P>;
+    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP, PB = FO::PB, FB = FO::FB, CB = FO::CB;
+    constexpr int G = TV::G, NWV = TV::WV, NB = 64 * NWV, TT = TV::value, ESF = TV::ESF, ESX = TV::ESX;
+    constexpr int RU = TV::RU, RY = NFP, RO = 2 * NFP;  // rows of U, the y gradient traces, the partner's U traces
+    __shared__ R ops[FO::COMMON + FO::FAMILY];  // the operator tables
+    const R* const fam = ops + FO::COMMON;
+    __shared__ R sTu[TT * ESF];      // traces of U
+    __shared__ R sX[TT * ESX];
+    __shared__ double sred[NWV];
+    __shared__ R sGeo[TT * 4];       // r_x, r_y, s_x, s_y
+    __shared__ R sEw[TT * 3 * 4];    // per edge: jump weights x, y (outward normal times |e|/(2J)), the partner's
+                                     // weights of its face lifting x, y
+    __shared__ R sNs[TT * 3 * 4];    // per edge: face normal, own factor +-|e|/(2J), the partner's -+|e|/(2J)
+    __shared__ int4 sPa[TT * 3];     // per edge, where its partner's slots are (point f faces slot P - f): element
+                                     // and slot P of its edge in the tile (the edge's own if across tiles), the
+                                     // partner's edge if across tiles (else 3), the row of slot P in the trace array
+    __shared__ unsigned char sList[TT * 3];
+    __shared__ int sCnt[NWV];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane >> 4, v = lane & 3;
+    const int tile = tile_of_block(a.xcd_groups);
+    const int e0 = tile * TT;
+    const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
+    auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };  // this lane's element of group q
+    auto eg = [&](int q) { return min(e0 + elg(q), a.E - 1); };                // ... in the mesh, clamped to it
+    auto st = [](int elx, int j) { return elx * ESF + j * NV; };               // trace slots
+    auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };              // rows of the other region
+
+    // ---- 0: state, gradient, traces of U
+    double u[G][PB];
+    R ur[G][PB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) u[q][b] = a.U_in[blk(eg(q), min(4 * b + row, NP - 1), NP) + v];
+    {
+        const R* const src = frag_ops<R>() + tri::frag_offset<R>(P);
+        for (int t = 4 * tid; t < FO::COMMON + FO::FAMILY; t += 4 * NB) {
+            R w[4];
+            load4(src + (t < FO::COMMON ? t : t + a.family * FO::FAMILY), w);
+            store4(ops + t, w);
+        }
+    }
+    // one lane per edge of the tile; an in-tile face is solved by its left element only
+    static_assert(TT * 3 <= NB, "one lane per edge of the tile");
+    bool owned = false;
+    if (tid < TT * 3) {
+        const int el = tid / 3, k = tid - el * 3, e = min(e0 + el, a.E - 1);
+        const R* Ge = a.geo + (int64_t)e * GEO;
+        const int2 Lk = a.links[(int64_t)e * 3 + k];
+        const int nl = Lk.x - e0, ek = link_edge(Lk.y);
+        const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
+        const bool in = !live || (nl >= 0 && nl < TT);  // beyond the mesh: its own neighbour
+        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
+        const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, right ? sn : -sn};
+        store4(sEw + 4 * tid, we);
+        store4(sNs + 4 * tid, ns);
+        const bool self = !live || !in;
+        sPa[tid] = make_int4(self ? el : nl, (self ? k : ek) * FP + P, in ? 3 : ek,
+                             in ? P : (int)((unsigned)Lk.x * NFP + ek * FP + P));  // row < 2^32
+        owned = live && !(right && in);
+    }
+    if (tid < TT) {
+        R w[4];
+        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        store4(sGeo + 4 * tid, w);
+    }
+    const unsigned long long own_mask = __ballot(owned);
+    if (lane == 0) sCnt[wave] = __popcll(own_mask);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) {
+            ur[q][b] = 4 * b + row < NP ? R(u[q][b]) : R(0);
+            sX[sx_(elg(q), RU + 4 * b + row) + v] = ur[q][b];
+        }
+    __syncthreads();  // operators and edges in place
+    // the neighbours' U traces across tiles (lanes of in-tile edges read one line in common)
+    auto partner = [&](int q, int b) { return sPa[elg(q) * 3 + min(4 * b + row, NFP - 1) / FP]; };
+    auto remote = [&](int w, int b) { return ((int64_t)(unsigned)w - min(4 * b + row, NFP - 1) % FP) * TWV + v; };
+    R oth[G][FB];
+    unsigned edges = 0;  // two bits per slot: the partner's edge, 3 in the tile
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const int4 pa = partner(q, b);
+            edges |= (unsigned)pa.z << 2 * (q * FB + b);
+            oth[q][b] = a.T_in[remote(pa.w, b)];
+        }
+    auto edge_of = [&](int q, int b) { return (int)(edges >> 2 * (q * FB + b)) & 3; };
+    static_assert(G * FB <= 16, "two bits per slot");
+    R tu[G][FB], gd[G][2 * PB];
+    tri::frag_mma<true, R, G, FB, PB>(ops + FO::I, ur, tu);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) sTu[st(elg(q), 4 * b + row) + v] = tu[q][b];
+    tri::frag_mma<true, R, G, 2 * PB, PB>(ops + FO::D, ur, gd);
+    if (owned) {
+        int pos = __popcll(own_mask & ((1ull << lane) - 1));
+        for (int w = 0; w < wave; ++w) pos += sCnt[w];
+        sList[pos] = (unsigned char)tid;
+    }
+    __syncthreads();
+
+    // ---- 1: jumps, corrected gradient (the jumps' lifting along the outward normals)
+    R jmp[G][FB];
+    {
+        R jw[2 * G][FB], Q[2 * G][PB], ti[G][FB];
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const int4 pa = partner(q, b);
+                ti[q][b] = sTu[st(pa.x, pa.y - min(4 * b + row, NFP - 1) % FP) + v];
+            }
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            R ge[4];
+            load4(sGeo + 4 * elg(q), ge);
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                Q[2 * q][b] = ge[0] * gd[q][b] + ge[2] * gd[q][PB + b];
+                Q[2 * q + 1][b] = ge[1] * gd[q][b] + ge[3] * gd[q][PB + b];
+            }
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const int j = 4 * b + row;
+                const R* w = sEw + 4 * (elg(q) * 3 + min(j, NFP - 1) / FP);
+                oth[q][b] = edge_of(q, b) == 3 ? ti[q][b] : oth[q][b];
+                const R d = R(0.5) * (tu[q][b] + oth[q][b]) - tu[q][b];
+                jmp[q][b] = j < NFP ? d : R(0);
+                jw[2 * q][b] = w[0] * jmp[q][b];
+                jw[2 * q + 1][b] = w[1] * jmp[q][b];
+            }
+        }
+        tri::frag_mma<false, R, 2 * G, PB, FB>(fam + FO::L, jw, Q);
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) sX[sx_(elg(q), 4 * b + row) + v] = Q[2 * q][b];
+        tri::wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) sX[sx_(elg(q), NP + 4 * b + row) + v] = Q[2 * q + 1][b];
+    }
+    tri::wave_lds_fence();  // U and Q of the wave's elements in place
+
+    // ---- 2: contravariant total fluxes, one lane per point of the wave's
+    // elements, in place of Q; the partner's gradient traces on their way
+    R ox[G][FB], oy[G][FB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const R* T = a.T_in + remote(partner(q, b).w, b);
+            ox[q][b] = T[NV];
+            oy[q][b] = T[2 * NV];
+        }
+#pragma unroll 1
+    for (int t = lane; t < 4 * G * NP; t += 64) {
+        const int el = wave * 4 * G + t / NP, m = t % NP;
+        R U4[NV], X4[NV], Y4[NV], FR[NV], FS[NV], Fv[NV], Gv[NV], ge[4];
+        load4(sX + sx_(el, RU + m), U4);
+        load4(sX + sx_(el, m), X4);
+        load4(sX + sx_(el, NP + m), Y4);
+        load4(sGeo + 4 * el, ge);
+        const R inv = fast_rcp(U4[0]);
+        const R ux = U4[1] * inv, uy = U4[2] * inv;
+        const R p = (g - R(1)) * (U4[3] - R(0.5) * (U4[1] * ux + U4[2] * uy));
+        visc_flux(U4, X4, Y4, g, mu, kappa, Fv, Gv);
+        const R fx[NV] = {U4[1], U4[1] * ux + p, U4[1] * uy, (U4[3] + p) * ux};
+        const R fy[NV] = {U4[2], U4[2] * ux, U4[2] * uy + p, (U4[3] + p) * uy};
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            const R Fx = fx[w] - Fv[w], Fy = fy[w] - Gv[w];
+            FR[w] = ge[0] * Fx + ge[1] * Fy;
+            FS[w] = ge[2] * Fx + ge[3] * Fy;
+        }
+        store4(sX + sx_(el, m), FR);
+        store4(sX + sx_(el, NP + m), FS);
+    }
+    tri::wave_lds_fence();
+
+    // ---- 3: divergence and transformed normal fluxes; then the traces of
+    // the gradient plus the BR2 lifting of each edge's own jumps (across
+    // tiles the mean of both sides), in place of the point values
+    R dv[G][PB + FB];
+    {
+        R f[G][CB];
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < CB; ++b) {
+                const R w = sX[sx_(elg(q), 4 * b + row) + v];
+                f[q][b] = 4 * b + row < 2 * NP ? w : R(0);
+            }
+        tri::frag_mma<true, R, G, PB + FB, CB>(ops + FO::F, f, dv);
+    }
+    tri::wave_lds_fence();  // every read of the point fluxes done
+    {
+        R tg[G][2 * FB], lo[G][4][FB], gyv[G][FB];
+        tri::frag_mma<true, R, G, 2 * FB, PB>(ops + FO::G, ur, tg);
+        tri::diag_mma<R, P>(fam + FO::LF, jmp, lo);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int el = elg(q);
+            R ge[4];
+            load4(sGeo + 4 * el, ge);
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const int j = 4 * b + row, ek = edge_of(q, b);
+                R w[4];
+                load4(sEw + 4 * (el * 3 + min(j, NFP - 1) / FP), w);
+                const R own = eta * lo[q][0][b];
+                R gx = ge[0] * tg[q][b] + ge[2] * tg[q][FB + b] + w[0] * own;
+                R gy = ge[1] * tg[q][b] + ge[3] * tg[q][FB + b] + w[1] * own;
+                // the partner's jumps and outward normal are minus this side's
+                const R ln = ek == 0 ? lo[q][1][b] : (ek == 1 ? lo[q][2][b] : lo[q][3][b]);
+                gx = ek == 3 ? gx : R(0.5) * (gx + (ox[q][b] + w[2] * ln));
+                gy = ek == 3 ? gy : R(0.5) * (gy + (oy[q][b] + w[3] * ln));
+                sX[sx_(el, j) + v] = gx;
+                gyv[q][b] = gy;
+            }
+        }
+        tri::wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) sX[sx_(elg(q), RY + 4 * b + row) + v] = gyv[q][b];
+        tri::wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) sX[sx_(elg(q), RO + 4 * b + row) + v] = oth[q][b];
+    }
+    double u0[G][PB];
+    if (MODE == MODE_STAGE2 || MODE == MODE_STAGE3) {
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) u0[q][b] = a.U0[blk(eg(q), min(4 * b + row, NP - 1), NP) + v];
+    }
+    __syncthreads();
+    int nsolved = 0;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) nsolved += sCnt[w];
+
+    // ---- 4: common fluxes of the solved face points, scaled by each side's
+    // +-|e|/(2J): Riemann minus the BR2 viscous flux, in place of both sides'
+    // x gradient traces (each slot's is read by the lane that solves it
+    // alone).  Across tiles the partner's slot is the edge's own, which holds
+    // the mean, and whose flux is written last.
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
+        const int c = sList[t / FP], f = t - (t / FP) * FP;
+        const int el = c / 3, j = (c - el * 3) * FP + f;
+        const int4 pc = sPa[c];
+        const int so = sx_(el, j), sn = pc.z == 3 ? sx_(pc.x, pc.y - f) : so;
+        R own[NV], ot[NV], ns[4], Qbx[NV], Qby[NV], gx[NV], gy[NV];
+        load4(sTu + st(el, j), own);
+        load4(sX + sx_(el, RO + j), ot);
+        load4(sNs + 4 * c, ns);
+        load4(sX + so, Qbx);
+        load4(sX + sn, gx);
+        load4(sX + so + RY * NV, Qby);
+        load4(sX + sn + RY * NV, gy);
+        const bool right = ns[2] < R(0);
+        R Uc[NV], UL[NV], UR[NV], Fc[NV], Fv[NV], Gv[NV];
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            Uc[w] = R(0.5) * (own[w] + ot[w]);
+            Qbx[w] = R(0.5) * (Qbx[w] + gx[w]);
+            Qby[w] = R(0.5) * (Qby[w] + gy[w]);
+            UL[w] = right ? ot[w] : own[w];
+            UR[w] = right ? own[w] : ot[w];
+        }
+        visc_flux(Uc, Qbx, Qby, g, mu, kappa, Fv, Gv);
+        riemann_by_kind(a.riemann, UL, UR, ns[0], ns[1], g, Fc);
+        R d[NV], dn[NV];
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            Fc[w] -= Fv[w] * ns[0] + Gv[w] * ns[1];
+            d[w] = ns[2] * Fc[w];
+            dn[w] = ns[3] * Fc[w];
+        }
+        store4(sX + sn, dn);
+        tri::wave_lds_fence();
+        store4(sX + so, d);
+    }
+    __syncthreads();
+
+    // ---- 5: lifted flux differences, RK stage update
+    {
+        R d[G][FB], div[G][PB];
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const R w = sX[sx_(elg(q), 4 * b + row) + v];
+                d[q][b] = 4 * b + row < NFP ? w - dv[q][PB + b] : R(0);
+            }
+#pragma unroll
+            for (int b = 0; b < PB; ++b) div[q][b] = dv[q][b];
+        }
+        tri::frag_mma<false, R, G, PB, FB>(fam + FO::L, d, div);
+        const double dt = MODE == MODE_RESIDUAL ? 0.0 : *a.dt_ptr;
+        double l2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int e = e0 + elg(q);
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                const int i = 4 * b + row;
+                const bool ok = i < NP && e < a.E;
+                const double res = -double(div[q][b]);
+                double un = res;
+                if (MODE == MODE_STAGE1) un = u[q][b] + dt * res;
+                if (MODE == MODE_STAGE2) un = 0.75 * u0[q][b] + 0.25 * (u[q][b] + dt * res);
+                if (MODE == MODE_STAGE3) un = (1.0 / 3.0) * u0[q][b] + (2.0 / 3.0) * (u[q][b] + dt * res);
+                if (ok) (MODE == MODE_RESIDUAL ? a.R_out : a.U_out)[blk(e, i, NP) + v] = un;
+                if (MODE == MODE_RESIDUAL || MODE == MODE_STAGE3) l2 += ok ? res * res : 0.0;
+                ur[q][b] = i < NP ? R(un) : R(0);
+            }
+        }
+        if ((MODE == MODE_RESIDUAL || MODE == MODE_STAGE3) && a.l2_partial) {
+            const double s2 = block_reduce_n<OpSum, NWV>(l2, sred);
+            if (tid == 0) a.l2_partial[tile] = s2;
+        }
+    }
+    if (MODE == MODE_RESIDUAL) return;
+
+    // ---- 6: traces of the new stage state and of its gradient on edges
+    // another tile reads
+    R tn[G][FB], tg[G][2 * FB];
+    tri::frag_mma<true, R, G, FB, PB>(ops + FO::I, ur, tn);
+    tri::frag_mma<true, R, G, 2 * FB, PB>(ops + FO::G, ur, tg);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+        R ge[4];
+        load4(sGeo + 4 * elg(q), ge);
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            if (edge_of(q, b) == 3 || 4 * b + row >= NFP) continue;
+            R* T = a.T_out + ((int64_t)(e0 + elg(q)) * NFP + 4 * b + row) * TWV + v;
+            T[0] = tn[q][b];
+            T[NV] = ge[0] * tg[q][b] + ge[2] * tg[q][FB + b];
+            T[2 * NV] = ge[1] * tg[q][b] + ge[3] * tg[q][FB + b];
+        }
+    }
+}
+
+// The stage at the lowest orders (P1, and P2 in FP32): lanes as in
+// tri_stage_kernel, one per element and variable, the operators as scalar
+// operands.  A point has few operator entries there and padding to blocks of
+// four costs the matrix-core form a third of its rows: on 80,000 elements P1
+// takes 33 / 20 us a stage (FP64 / FP32) against 39 / 22, FP32 P2 34-37
+// against 36-38; FP64 P2 takes 85 against 59.  The point values (U, then Q)
+// live in LDS, each lane reads a point's four variables there.
 template <typename R, int P, int MODE, int TT>
-__global__ __launch_bounds__(TT * NV) void tri_visc_stage_kernel(TriArgs<R> a) {
+__global__ __launch_bounds__(TT * NV) void tri_visc_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
     constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
     constexpr int NB = TT * NV, NWV = NB / 64;
@@ -826,39 +1228,31 @@ __global__ __launch_bounds__(TT * NV) void tri_visc_stage_kernel(TriArgs<R> a) {
     }
 }
 
-// Traces of U and grad U on every edge (after a new state is set).
+// Traces of U and grad U on every edge (after a new state is set): one wave
+// per four elements.
 template <typename R, int P>
 __global__ __launch_bounds__(BLOCK) void tri_visc_trace_kernel(int E, const double* U, const R* geo, R* T_out) {
-    using S = TriShape<P>;
-    constexpr int NP = S::NP, NFP = S::NFP, O0 = ops_offset(P), CA = TriOps<P>::CA;
-    const int e = blockIdx.x * TILE + (threadIdx.x >> 2), v = threadIdx.x & 3;
-    if (e >= E) return;
-    const R* G = geo + (int64_t)e * GEO;
-    const R rx = G[0], ry = G[1], sx = G[2], sy = G[3];
-    R u[NP], gr[NP], gs[NP];
+    using FO = tri::FragOps<R, P>;
+    constexpr int NP = FO::NP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB;
+    const R* const ops = frag_ops<R>() + tri::frag_offset<R>(P);
+    const int lane = threadIdx.x & 63, row = lane >> 4, v = lane & 3;
+    const int e = (blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * 4 + ((lane >> 2) & 3);
+    const bool live = e < E;
+    R u[1][PB], t[1][FB], tg[1][2 * FB];
 #pragma unroll
-    for (int m = 0; m < NP; ++m) { u[m] = R(U[blk(e, m, NP) + v]); gr[m] = R(0); gs[m] = R(0); }
+    for (int b = 0; b < PB; ++b) u[0][b] = live && 4 * b + row < NP ? R(U[blk(e, 4 * b + row, NP) + v]) : R(0);
+    tri::frag_mma<true, R, 1, FB, PB>(ops + FO::I, u, t);
+    tri::frag_mma<true, R, 1, 2 * FB, PB>(ops + FO::G, u, tg);
+    if (!live) return;
+    const R* Ge = geo + (int64_t)e * GEO;
+    const R rx = Ge[0], ry = Ge[1], sx = Ge[2], sy = Ge[3];
 #pragma unroll
-    for (int m = 0; m < NP; ++m)
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            gr[i] = fmaR(cop<R>(O0 + m * CA + i), u[m], gr[i]);
-            gs[i] = fmaR(cop<R>(O0 + m * CA + NP + i), u[m], gs[i]);
-        }
-#pragma unroll 1
-    for (int j = 0; j < NFP; ++j) {
-        R tu = R(0), tx = R(0), ty = R(0);
-#pragma unroll
-        for (int m = 0; m < NP; ++m) {
-            const R w = cop<R>(O0 + m * CA + 2 * NP + j);
-            tu = fmaR(w, u[m], tu);
-            tx = fmaR(w, rx * gr[m] + sx * gs[m], tx);
-            ty = fmaR(w, ry * gr[m] + sy * gs[m], ty);
-        }
-        R* T = T_out + ((int64_t)e * NFP + j) * TWV;
-        T[v] = tu;
-        T[NV + v] = tx;
-        T[2 * NV + v] = ty;
+    for (int b = 0; b < FB; ++b) {
+        if (4 * b + row >= NFP) continue;
+        R* T = T_out + ((int64_t)e * NFP + 4 * b + row) * TWV + v;
+        T[0] = t[0][b];
+        T[NV] = rx * tg[0][b] + sx * tg[0][FB + b];
+        T[2 * NV] = ry * tg[0][b] + sy * tg[0][FB + b];
     }
 }
 
@@ -2055,16 +2449,26 @@ hipError_t tri_launch(int P, int mode, const TriArgs<R>& a, hipStream_t s) {
 
 template <typename R, int P>
 hipError_t tri_visc_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
-    constexpr int TT = TriViscTile<R, P>::value;
-    const int grid = (std::max(a.E, 1) + TT - 1) / TT;
-    const dim3 blk(TT * NV);
-    switch (mode) {
-    case MODE_RESIDUAL: klaunch(tri_visc_stage_kernel<R, P, MODE_RESIDUAL, TT>, grid, blk, 0, s, a); break;
-    case MODE_STAGE1: klaunch(tri_visc_stage_kernel<R, P, MODE_STAGE1, TT>, grid, blk, 0, s, a); break;
-    case MODE_STAGE2: klaunch(tri_visc_stage_kernel<R, P, MODE_STAGE2, TT>, grid, blk, 0, s, a); break;
-    default: klaunch(tri_visc_stage_kernel<R, P, MODE_STAGE3, TT>, grid, blk, 0, s, a); break;
+    if constexpr (std::is_same<R, double>::value && P == 4) {
+        return hipErrorInvalidValue;  // refused when the handle is made
+    } else {
+        constexpr int TT = TriViscTile<R, P>::value;
+        const int grid = (std::max(a.E, 1) + TT - 1) / TT;
+        auto launch = [&](auto m) {
+            constexpr int MODE = decltype(m)::value;
+            if constexpr (tri_visc_scalar<R, P>())
+                klaunch(tri_visc_scalar_kernel<R, P, MODE, TT>, grid, dim3(TT * NV), 0, s, a);
+            else
+                klaunch(tri_visc_stage_kernel<R, P, MODE>, grid, dim3(64 * TriViscTile<R, P>::WV), 0, s, a);
+        };
+        switch (mode) {
+        case MODE_RESIDUAL: launch(std::integral_constant<int, MODE_RESIDUAL>{}); break;
+        case MODE_STAGE1: launch(std::integral_constant<int, MODE_STAGE1>{}); break;
+        case MODE_STAGE2: launch(std::integral_constant<int, MODE_STAGE2>{}); break;
+        default: launch(std::integral_constant<int, MODE_STAGE3>{}); break;
+        }
+        return hipGetLastError();
     }
-    return hipGetLastError();
 }
 
 template <typename R>
@@ -2080,7 +2484,8 @@ hipError_t tri_visc_launch(int P, int mode, const TriArgs<R>& a, hipStream_t s) 
 
 template <typename R>
 hipError_t tri_visc_trace(int P, int E, const double* U, const R* geo, R* T, hipStream_t s) {
-    const int grid = (std::max(E, 1) + TILE - 1) / TILE;
+    constexpr int PER = BLOCK / 64 * 4;  // elements per workgroup
+    const int grid = (std::max(E, 1) + PER - 1) / PER;
     switch (P) {
     case 1: tri_visc_trace_kernel<R, 1><<<grid, BLOCK, 0, s>>>(E, U, geo, T); break;
     case 2: tri_visc_trace_kernel<R, 2><<<grid, BLOCK, 0, s>>>(E, U, geo, T); break;
@@ -2261,6 +2666,22 @@ hipError_t load_tri_ops(int device) {
                 for (int i = 0; i < np; ++i) dl[(size_t)jj * np + i] = F.lift[(size_t)i * nf + jj];
         }
     }
+    std::vector<double> fr64((size_t)tri::frag_offset<double>(6));
+    std::vector<float> fr32((size_t)tri::frag_offset<float>(6));
+    auto frags = [&](auto order) {
+        constexpr int P = decltype(order)::value;
+        tri::Operators F[3];
+        const int kinds[3] = {ZJ_CORR_DG, ZJ_CORR_SD, ZJ_CORR_HU};
+        for (int k = 0; k < 3; ++k)
+            if (!tri::operators(P, F[k], kinds[k])) return false;
+        tri::frag_build<double, P>(fr64.data() + tri::frag_offset<double>(P), F);
+        tri::frag_build<float, P>(fr32.data() + tri::frag_offset<float>(P), F);
+        return true;
+    };
+    if (!frags(std::integral_constant<int, 1>{}) || !frags(std::integral_constant<int, 2>{}) ||
+        !frags(std::integral_constant<int, 3>{}) || !frags(std::integral_constant<int, 4>{}) ||
+        !frags(std::integral_constant<int, 5>{}))
+        return hipErrorInvalidValue;
     std::vector<double> lf((size_t)LF_TOTAL, 0.0);
     for (int P = 1; P <= 5; ++P) {
         for (int fam = 0; fam < 3; ++fam) {
@@ -2289,6 +2710,10 @@ hipError_t load_tri_ops(int device) {
         e = hipMemcpyToSymbol(HIP_SYMBOL(c_lf64), lf.data(), lf.size() * sizeof(double), 0, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpyToSymbol(HIP_SYMBOL(c_lf32), lff.data(), lff.size() * sizeof(float), 0, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpyToSymbol(HIP_SYMBOL(d_frag64), fr64.data(), fr64.size() * sizeof(double), 0, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpyToSymbol(HIP_SYMBOL(d_frag32), fr32.data(), fr32.size() * sizeof(float), 0, hipMemcpyHostToDevice);
     if (e == hipSuccess && device >= 0 && device < 64) g_ops_loaded |= 1ull << device;
     return e;
 }
@@ -2460,7 +2885,11 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
     std::vector<double> geo((size_t)E * GEO, 0.0);
     for (int e = 0; e < E; ++e) {
         const int o = perm.empty() ? e : perm[(size_t)e];
-        for (int c = 0; c < 4; ++c) geo[(size_t)e * GEO + c] = met[(size_t)o * 4 + c];
+        double* ge = &geo[(size_t)e * GEO];
+        for (int c = 0; c < 4; ++c) ge[c] = met[(size_t)o * 4 + c];
+        ge[GEO_S] = std::sqrt(ge[2] * ge[2] + ge[3] * ge[3]);
+        ge[GEO_S + 1] = std::sqrt((ge[0] + ge[2]) * (ge[0] + ge[2]) + (ge[1] + ge[3]) * (ge[1] + ge[3]));
+        ge[GEO_S + 2] = std::sqrt(ge[0] * ge[0] + ge[1] * ge[1]);
     }
     std::vector<double> hcd((size_t)E);
     for (int e = 0; e < E; ++e) hcd[(size_t)e] = hc[(size_t)(perm.empty() ? e : perm[(size_t)e])];
@@ -2500,8 +2929,11 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
             L = make_int2(-1, bct | (ROLE_BOUNDARY << 3) | (bci << 6));
         }
     }
-    for (size_t k = 0; k < links.size(); ++k)
+    for (size_t k = 0; k < links.size(); ++k) {
         if (links[k].y == -1) return tfail(h, ZJ_ERR_ARG, "an element edge has no face");
+        if (links[k].x >= 0)
+            geo[k / 3 * GEO + GEO_SN + k % 3] = geo[(size_t)links[k].x * GEO + GEO_S + (links[k].y & 7)];
+    }
 
     ZJ_THIP(h, hipSetDevice(h->device));
     ZJ_THIP(h, load_tri_ops(h->device));
@@ -2555,6 +2987,7 @@ static TriArgs<R> tri_args(zj_tri* h, int mode) {
     a.kappa = h->kappa;
     a.eta = h->eta;
     a.lf_off = lf_family(h->corr) * lf_words(h->P);
+    a.family = lf_family(h->corr);
     R** T = (R**)h->T;
     switch (mode) {
     case MODE_RESIDUAL:
