@@ -7,6 +7,7 @@ increment is a few 1e-3 of the state at these time steps, so the state's
 rounding (1e-16 FP64) shows in it at 1e-13 and the bar holds for it too; the
 FP32-bulk increment carries the residual's own FP32 error.
 """
+import numpy as np
 import pytest
 
 from tests.test_gpu_parity import rel, say
@@ -31,3 +32,31 @@ def test_tri_viscous_tiles(p, precision, n):
     ri = rel(s.get_state() - U, o.advance(U, dt) - U)
     say(f"  rel L2 residual {r:.3e}, step increment {ri:.3e}")
     assert r < BAR[precision] and ri < BAR[precision]
+
+
+@pytest.mark.parametrize("n", [1, 4, 5])
+@pytest.mark.parametrize("p,precision", [(1, "fp64"), (2, "fp64"), (5, "fp64"), (2, "fp32bulk"), (4, "fp32bulk")])
+def test_tri_viscous_vjp_tiles(p, precision, n):
+    """One step backwards with dJ/d(dt) at the adjoint's tile edges (32 elements; 64 at P1, 16 at FP64 P5):
+    <g, dU1/dU v> and <g, dU1/d(dt)> against central differences of the oracle's step.  The difference
+    quotient's own error is eps^2 / 6 times the third derivative plus rounding / eps: 1e-8 at eps = 1e-5;
+    FP32-bulk carries its 1e-6 residual error into the product of a random g with the step."""
+    corr = {1: "ga", 4: "dg", 5: "hu"}[n]
+    say(f"case: triangle viscous step VJP, {2 * n * n} elements P{p} {precision} roe/{corr}")
+    s, o, m = _pair(n, p, "roe", corr, precision=precision, seed=n)
+    U = _state(m, p, 3 + n)
+    s.set_state(U)
+    dt, eps = 0.25 * s.dt_cfl(0.5), 1e-5
+    rng = np.random.default_rng(n)
+    g, v = rng.standard_normal(U.size), rng.standard_normal(U.size) * U
+    s.adjoint_set(g)
+    dtb = s.rk3_step_vjp(dt)
+    got, got_dt = float(s.adjoint_get() @ v), dtb
+    want = float(g @ (o.advance(U + eps * v, dt) - o.advance(U - eps * v, dt))) / (2 * eps)
+    h = 1e-4 * dt
+    want_dt = float(g @ (o.advance(U, dt + h) - o.advance(U, dt - h))) / (2 * h)
+    scale, scale_dt = np.linalg.norm(g) * np.linalg.norm(v), np.linalg.norm(g) * np.linalg.norm(o.residual(U))
+    r, rd = abs(got - want) / scale, abs(got_dt - want_dt) / scale_dt
+    say(f"  state {r:.3e}, time step {rd:.3e}")
+    bar = 1e-8 if precision == "fp64" else 1e-5
+    assert r < bar and rd < bar

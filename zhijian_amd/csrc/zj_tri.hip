@@ -1294,7 +1294,8 @@ struct TriVjpArgs {
     int xcd_groups;
     int lift_off;
     double mu, kappa, eta;  // Navier-Stokes terms (tri_visc_vjp_kernel)
-    int lf_off;
+    int family;             // of the correction: DG, SD = GA, HU
+    const double* R_in;     // residual at q, with dtb_partial (tri_visc_vjp_kernel)
 };
 
 template <typename R, int P, int MODE>
@@ -1657,703 +1658,551 @@ __global__ __launch_bounds__(BLOCK) void tri_complete_kernel(int E, const int2* 
 
 // ------------------------------------------------------------ adjoint, BR2
 // Vector-Jacobian product of one triangle stage with the Navier-Stokes terms
-// (tri_visc_stage_kernel), or of its residual alone.  The forward values are
-// recomputed as that kernel forms them (traces of U and of its gradient, the
-// corrected gradient, the point fluxes, the flux differences), with the point
-// fluxes kept apart from the corrected gradient; then, per lane (element,
-// variable) unless stated:
+// (tri_visc_stage_kernel), or of its residual alone; lanes and operator
+// products as there.  Of the forward values it recomputes the traces, the
+// corrected gradient and both sides' BR2 gradients; the residual, needed for
+// the time step's cotangent alone, comes from a residual launch (R_in).  Then
 //   R1  cotangent of u_out: its partial value plus, on cross-tile edges, the
 //       transposed traces of U and of its gradient; the RK combination
 //   R2  the lifting transposed: the flux differences' cotangents
 //   R4  the divergence and the interpolated normal fluxes transposed; then one
 //       lane per point (all four variables): the Euler and viscous flux VJPs,
 //       the cotangents of U and of the corrected gradient at the point
-//   R5  the corrected gradient's lifted jumps transposed: each edge point's
-//       jump cotangent
+//   R5  the corrected gradient's lifted jumps transposed
 //   R3  per solved face point: the common flux's cotangent, the Riemann and
-//       viscous flux VJPs at the face, the jump cotangents of both sides'
-//       corrected gradients; the cotangents of both sides' traces (of U and
-//       of the gradient) at their slots (LDS, or the cross-tile neighbour's
-//       slot in HBM, 12 words); then the face liftings transposed, gathered
-//       over the edge's points
-//   R6  the traces and the gradient transposed: cotangent of q
+//       viscous flux VJPs at the face, the cotangents of both sides' traces
+//       (of U and of the gradient) at their slots
+//   R7  the face liftings transposed; every edge point's jump cotangent
+//   R6  the traces and the gradient transposed: cotangent of q.  Across tiles
+//       the partner's 12 words go to its slot in memory
+// Bounds as the stage kernel's, with one (FP64) or two waves per SIMD.  80,000
+// elements, P3, us a launch (operators as scalar operands, the residual
+// recomputed in every launch -> this): FP64 480 -> 175, FP32 210 -> 90; a step
+// backwards 1719 -> 665 and 820 -> 356.
 template <typename R, int P> struct TriViscVjpTile {
-    static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1);
-    static constexpr int XW = 2 * (NP > NFP ? NP : NFP);  // the point fluxes, later the jump cotangents
-    static constexpr int words = 4 * NFP + 3 * NP + XW;    // per element and variable
-    static constexpr int bytes(int tt) { return tt * words * NV * (int)sizeof(R); }
-    static constexpr int value = bytes(64) <= 61440 ? 64 : (bytes(32) <= 61440 ? 32 : 16);
-    // gfx950 gives a workgroup up to 160 KiB of LDS: FP64 P4 and P5 take 69
-    // and 91 KiB at 16 elements (one workgroup per CU)
-    static constexpr bool fits = bytes(16) <= 122880;
+    static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1), PB = (NP + 3) / 4, FB = (NFP + 3) / 4;
+    static constexpr bool BIG = sizeof(R) == 8 && P == 5;
+    static constexpr int G = BIG ? 1 : 2, WV = P == 1 ? 8 : 4, value = 4 * G * WV;
+    // waves per SIMD asked for: in FP64 the face points' VJPs take more than the 256 VGPRs of two (P2:
+    // 584 us a step at one wave, 707 at two with scratch), P5's LDS allows one workgroup
+    static constexpr int WPE = (sizeof(R) == 8 ? P == 1 : P < 5) ? 2 : 1;
+    // rows of an element's region: Q_x, Q_y, the point fluxes' cotangents x, y, U (RU); later the
+    // gradient traces x and y, the partner's U traces and the flux differences' cotangents
+    static constexpr int RU = 3 * NP + 4 * PB;
+    static constexpr int ROWS = RU + 4 * PB > 3 * NFP + 4 * FB ? RU + 4 * PB : 3 * NFP + 4 * FB;
+    static constexpr int ESF = tri::elem_stride<R>(4 * FB), ESX = tri::elem_stride<R>(ROWS);
 };
 
-template <typename R, int P, int MODE, int TT>
-__global__ __launch_bounds__(TT * NV) void tri_visc_vjp_kernel(TriVjpArgs<R> a) {
+template <typename R, int P, int MODE>
+__global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R, P>::WPE)) void tri_visc_vjp_kernel(TriVjpArgs<R> a) {
     using S = TriShape<P>;
-    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
-    constexpr int NB = TT * NV, NWV = NB / 64;
-    static_assert(NB % 64 == 0, "tile layout");
-    using OP = TriOps<P>;
-    constexpr int O0 = ops_offset(P), CA = OP::CA, OI = O0 + OP::C;
-    constexpr int XW = TriViscVjpTile<R, P>::XW;
+    using TV = TriViscVjpTile<R, P>;
+    using FO = tri::FragOps<R, P>;
+    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP, PB = FO::PB, FB = FO::FB;
+    constexpr int G = TV::G, NWV = TV::WV, NB = 64 * NWV, TT = TV::value, ESF = TV::ESF, ESX = TV::ESX;
+    constexpr int RU = TV::RU, RA = 2 * NP, RB = 3 * NP;       // point rows
+    constexpr int RY = NFP, RO = 2 * NFP, RD = 3 * NFP;         // trace rows
     constexpr double ca = MODE == MODE_STAGE2 ? 0.75 : (MODE == MODE_STAGE3 ? 1.0 / 3.0 : 0.0);
     constexpr double cb = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
     constexpr double cc = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
-    const int OLT = O0 + a.lift_off;
-    const int LFO = lf_offset(P) + a.lf_off;
-    __shared__ R sTu[TT * NFP * NV];   // traces of U
-    __shared__ R sTx[TT * NFP * NV];   // traces of the gradient, then their cotangents
-    __shared__ R sTy[TT * NFP * NV];
-    __shared__ R sD[TT * NFP * NV];    // flux differences, their cotangents, then the U traces' cotangents
-    __shared__ R sU[TT * NP * NV];     // q, then the flux VJPs' cotangents of U at the points
-    __shared__ R sQx[TT * NP * NV];    // corrected gradient, then its cotangent
-    __shared__ R sQy[TT * NP * NV];
-    __shared__ R sX[TT * XW * NV];     // contravariant point fluxes, then their x / y cotangents;
-                                       // later the jump cotangents and the face liftings' seeds
+    constexpr int N0 = FO::F, N1 = FO::FAMILY, N2 = FO::ADJ, N3 = FO::ADJ_FAMILY;  // D, I, G; L, LF; FT, GT, DT; LT, LFT
+    __shared__ R ops[N0 + N1 + N2 + N3];
+    const R *const fam = ops + N0, *const adj = fam + N1, *const afam = adj + N2;
+    __shared__ R sTu[TT * ESF];      // traces of U; later, across tiles, the partner's U cotangents
+    __shared__ R sX[TT * ESX];
     __shared__ double sred[NWV];
-    __shared__ R sEdge[TT * 3];
-    __shared__ int2 sLink[TT * 3];
-    __shared__ R sNrm[TT * 3 * 2];
+    __shared__ R sGeo[TT * 4];
+    __shared__ R sEw[TT * 3 * 4];    // as in tri_visc_stage_kernel
+    __shared__ R sNs[TT * 3 * 4];    // (the partner's factor 0 across tiles)
+    __shared__ int4 sPa[TT * 3];
     __shared__ unsigned char sList[TT * 3];
     __shared__ int sCnt[NWV];
-    R* const sFR = sX;
-    R* const sFS = sX + TT * NP * NV;
-    R* const sJ = sX;
-    R* const sC = sX + TT * NFP * NV;
 
-    const int tid = threadIdx.x, el = tid >> 2, v = tid & 3;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane >> 4, v = lane & 3;
     const int tile = tile_of_block(a.xcd_groups);
-    const int e0 = tile * TT, e = e0 + el;
-    const bool live = e < a.E;
+    const int e0 = tile * TT;
     const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
-    const int64_t base = blk(e, 0, NP) + v;
-    auto sl = [](int elx, int j, int w) { return (elx * NFP + j) * NV + w; };
-    auto sp = [](int elx, int m, int w) { return (elx * NP + m) * NV + w; };
+    auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };
+    auto eg = [&](int q) { return min(e0 + elg(q), a.E - 1); };
+    auto st = [](int elx, int j) { return elx * ESF + j * NV; };
+    auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };
+    auto pt = [&](int q, int b) { return blk(eg(q), min(4 * b + row, NP - 1), NP) + v; };
 
-    // ---- forward 0: state, gradient, traces of U and of the gradient
-    R rx = R(0), ry = R(0), sx = R(0), sy = R(0);
-    R jwx[3] = {R(0), R(0), R(0)}, jwy[3] = {R(0), R(0), R(0)};  // each edge's jump weights
-    int2 L[3] = {make_int2(0, 0), make_int2(0, 0), make_int2(0, 0)};
-    if (live) {
+    // ---- 0: q, the incoming cotangent, operators and edges
+    R ur[G][PB];
+    double unb[G][PB], rin[G][PB];
 #pragma unroll
-        for (int m = 0; m < NP; ++m) sU[sp(el, m, v)] = R(a.U_in[base + (int64_t)m * EB * NV]);
-        const R* G = a.geo + (int64_t)e * GEO;
-        rx = G[0]; ry = G[1]; sx = G[2]; sy = G[3];
+    for (int q = 0; q < G; ++q)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) L[k] = a.links[(int64_t)e * 3 + k];
-        R se[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const R ax = k == 0 ? sx : (k == 1 ? rx + sx : rx), ay = k == 0 ? sy : (k == 1 ? ry + sy : ry);
-            se[k] = sqrtR(ax * ax + ay * ay);
-            const R sg = link_role(L[k].y) == ROLE_RIGHT ? R(-1) : R(1);
-            jwx[k] = sg * se[k] * G[4 + 2 * k];
-            jwy[k] = sg * se[k] * G[5 + 2 * k];
+        for (int b = 0; b < PB; ++b) {
+            ur[q][b] = R(a.U_in[pt(q, b)]);
+            unb[q][b] = a.Ub_in[pt(q, b)];
+            rin[q][b] = MODE != MODE_RESIDUAL && a.dtb_partial ? a.R_in[pt(q, b)] : 0.0;
         }
-        if (v < 3) {
-            sEdge[el * 3 + v] = se[v];
-            sLink[el * 3 + v] = L[v];
-            sNrm[(el * 3 + v) * 2] = G[4 + 2 * v];
-            sNrm[(el * 3 + v) * 2 + 1] = G[5 + 2 * v];
-        }
-        R gr[NP], gs[NP];
-#pragma unroll
-        for (int i = 0; i < NP; ++i) { gr[i] = R(0); gs[i] = R(0); }
-#pragma unroll
-        for (int m = 0; m < NP; ++m) {
-            const R um = sU[sp(el, m, v)];
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                gr[i] = fmaR(cop<R>(O0 + m * CA + i), um, gr[i]);
-                gs[i] = fmaR(cop<R>(O0 + m * CA + NP + i), um, gs[i]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            sQx[sp(el, i, v)] = rx * gr[i] + sx * gs[i];
-            sQy[sp(el, i, v)] = ry * gr[i] + sy * gs[i];
-        }
-#pragma unroll 1
-        for (int j = 0; j < NFP; ++j) {
-            R tu = R(0), tx = R(0), ty = R(0);
-#pragma unroll
-            for (int m = 0; m < NP; ++m) {
-                const R w = cop<R>(OI + j * NP + m);
-                tu = fmaR(w, sU[sp(el, m, v)], tu);
-                tx = fmaR(w, sQx[sp(el, m, v)], tx);
-                ty = fmaR(w, sQy[sp(el, m, v)], ty);
-            }
-            sTu[sl(el, j, v)] = tu;
-            sTx[sl(el, j, v)] = tx;
-            sTy[sl(el, j, v)] = ty;
+    {
+        const R* const src = frag_ops<R>() + tri::frag_offset<R>(P);
+        for (int t = 4 * tid; t < N0 + N1 + N2 + N3; t += 4 * NB) {
+            const int o = t < N0 ? t
+                          : t < N0 + N1 ? t - N0 + FO::COMMON + a.family * N1
+                          : t < N0 + N1 + N2 ? t - N0 - N1 + FO::ADJ0
+                                             : t - N0 - N1 - N2 + FO::ADJ_FAM0 + a.family * N3;
+            R w[4];
+            load4(src + o, w);
+            store4(ops + t, w);
         }
     }
+    static_assert(TT * 3 <= NB, "one lane per edge of the tile");
     bool owned = false;
-    if (live && v < 3) {
-        const int2 Lv = v == 0 ? L[0] : (v == 1 ? L[1] : L[2]);
-        const int nl = Lv.x - e0;
-        owned = !(link_role(Lv.y) == ROLE_RIGHT && nl >= 0 && nl < TT);
+    if (tid < TT * 3) {
+        const int el = tid / 3, k = tid - el * 3, e = min(e0 + el, a.E - 1);
+        const R* Ge = a.geo + (int64_t)e * GEO;
+        const int2 Lk = a.links[(int64_t)e * 3 + k];
+        const int nl = Lk.x - e0, ek = link_edge(Lk.y);
+        const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
+        const bool in = !live || (nl >= 0 && nl < TT);
+        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
+        const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, in ? (right ? sn : -sn) : R(0)};
+        store4(sEw + 4 * tid, we);
+        store4(sNs + 4 * tid, ns);
+        const bool self = !live || !in;
+        sPa[tid] = make_int4(self ? el : nl, (self ? k : ek) * FP + P, in ? 3 : ek,
+                             in ? P : (int)((unsigned)Lk.x * NFP + ek * FP + P));
+        owned = live && !(right && in);
+    }
+    if (tid < TT) {
+        R w[4];
+        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        store4(sGeo + 4 * tid, w);
     }
     const unsigned long long own_mask = __ballot(owned);
-    const int lane = tid & 63, wave = tid >> 6;
     if (lane == 0) sCnt[wave] = __popcll(own_mask);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) {
+            ur[q][b] = 4 * b + row < NP ? ur[q][b] : R(0);
+            sX[sx_(elg(q), RU + 4 * b + row) + v] = ur[q][b];
+        }
     __syncthreads();
-
-    // ---- forward 1: corrected gradient
-    if (live) {
-        R jx[NFP], jy[NFP];
+    auto partner = [&](int q, int b) { return sPa[elg(q) * 3 + min(4 * b + row, NFP - 1) / FP]; };
+    auto remote = [&](int w, int b) { return ((int64_t)(unsigned)w - min(4 * b + row, NFP - 1) % FP) * TWV + v; };
+    R oth[G][FB];
+    unsigned edges = 0;  // two bits per slot: the partner's edge, 3 in the tile
 #pragma unroll
-        for (int kk = 0; kk < 3; ++kk) {
-            const int2 Lk = L[kk];
-            const int nl = Lk.x - e0;
-            const bool in = nl >= 0 && nl < TT;
-            const int ek = link_edge(Lk.y);
+    for (int q = 0; q < G; ++q)
 #pragma unroll
-            for (int f = 0; f < FP; ++f) {
-                const int j = kk * FP + f, oj = ek * FP + (P - f);
-                const R own = sTu[sl(el, j, v)];
-                R oth;
-                if (in) oth = sTu[sl(nl, oj, v)];
-                else oth = a.T_in[((int64_t)Lk.x * NFP + oj) * TWV + v];
-                const R jmp = R(0.5) * (own + oth) - own;
-                jx[j] = jwx[kk] * jmp;
-                jy[j] = jwy[kk] * jmp;
-            }
+        for (int b = 0; b < FB; ++b) {
+            const int4 pa = partner(q, b);
+            edges |= (unsigned)pa.z << 2 * (q * FB + b);
+            oth[q][b] = a.T_in[remote(pa.w, b)];
         }
-#pragma unroll 1
-        for (int i = 0; i < NP; ++i) {
-            R qx = sQx[sp(el, i, v)], qy = sQy[sp(el, i, v)];
-#pragma unroll
-            for (int j = 0; j < NFP; ++j) {
-                const R l = cop<R>(OLT + j * NP + i);
-                qx = fmaR(l, jx[j], qx);
-                qy = fmaR(l, jy[j], qy);
-            }
-            sQx[sp(el, i, v)] = qx;
-            sQy[sp(el, i, v)] = qy;
-        }
-    }
+    auto edge_of = [&](int q, int b) { return (int)(edges >> 2 * (q * FB + b)) & 3; };
+    static_assert(G * FB <= 16, "two bits per slot");
     if (owned) {
         int pos = __popcll(own_mask & ((1ull << lane) - 1));
         for (int w = 0; w < wave; ++w) pos += sCnt[w];
-        sList[pos] = (unsigned char)(el * 3 + v);
+        sList[pos] = (unsigned char)tid;
     }
-    __syncthreads();
+    R tu[G][FB], gd[G][2 * PB];
+    tri::frag_mma<true, R, G, FB, PB>(ops + FO::I, ur, tu);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) sTu[st(elg(q), 4 * b + row) + v] = tu[q][b];
+    tri::frag_mma<true, R, G, 2 * PB, PB>(ops + FO::D, ur, gd);
 
-    // ---- forward 2: contravariant total fluxes at the points (points v, v + 4,
-    // ... of the element, four variables each), then this lane's divergence
-    // and interpolated normal fluxes
-    constexpr int MPL = (NP + NV - 1) / NV;
-    if (live) {
-#pragma unroll 1
-        for (int q = 0; q < MPL; ++q) {
-            const int m = v + NV * q;
-            if (m >= NP) break;
-            R U4[NV], X4[NV], Y4[NV];
+    // ---- R1, R2: cotangents of u_out, of the divergence and of the flux differences; R4: of the point fluxes
+    double qb[G][PB], rsum = 0.0;
+    R fx[G][2 * PB], db[G][FB];
+    {
+        if (MODE != MODE_RESIDUAL && a.Tb_in) {
+            R f[G][3 * FB], add[G][PB];
 #pragma unroll
-            for (int w = 0; w < NV; ++w) {
-                U4[w] = sU[sp(el, m, w)];
-                X4[w] = sQx[sp(el, m, w)];
-                Y4[w] = sQy[sp(el, m, w)];
-            }
-            const R inv = fast_rcp(U4[0]);
-            const R ux = U4[1] * inv, uy = U4[2] * inv;
-            const R p = (g - R(1)) * (U4[3] - R(0.5) * (U4[1] * ux + U4[2] * uy));
-            R Fv[NV], Gv[NV];
-            visc_flux(U4, X4, Y4, g, mu, kappa, Fv, Gv);
-            const R fx[NV] = {U4[1], U4[1] * ux + p, U4[1] * uy, (U4[3] + p) * ux};
-            const R fy[NV] = {U4[2], U4[2] * ux, U4[2] * uy + p, (U4[3] + p) * uy};
+            for (int q = 0; q < G; ++q) {
+                R ge[4];
+                load4(sGeo + 4 * elg(q), ge);
 #pragma unroll
-            for (int w = 0; w < NV; ++w) {
-                const R Fx = fx[w] - Fv[w], Fy = fy[w] - Gv[w];
-                sFR[sp(el, m, w)] = rx * Fx + ry * Fy;
-                sFS[sp(el, m, w)] = sx * Fx + sy * Fy;
+                for (int b = 0; b < FB; ++b) {
+                    // own slots across tiles (the others read the tile's first row in common)
+                    const int j = 4 * b + row;
+                    const bool on = edge_of(q, b) != 3 && j < NFP;
+                    const R* T = a.Tb_in + (on ? (int64_t)eg(q) * NFP + j : (int64_t)0) * TWV + v;
+                    const R tb = T[0], xb = T[NV], yb = T[2 * NV];
+                    f[q][b] = on ? tb : R(0);
+                    f[q][FB + b] = on ? ge[0] * xb + ge[1] * yb : R(0);
+                    f[q][2 * FB + b] = on ? ge[2] * xb + ge[3] * yb : R(0);
+                }
             }
+            tri::frag_mma<true, R, G, PB, 3 * FB>(adj + FO::GT, f, add);
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int b = 0; b < PB; ++b) unb[q][b] += double(add[q][b]);
         }
+        const double dt = MODE == MODE_RESIDUAL ? 0.0 : *a.dt_ptr;
+        R f[G][PB + FB], dvb[G][PB];
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                const bool ok = 4 * b + row < NP && e0 + elg(q) < a.E;
+                double rb = unb[q][b];
+                qb[q][b] = 0.0;
+                if (MODE != MODE_RESIDUAL) {
+                    if (MODE == MODE_STAGE3 && ok) a.U0b[pt(q, b)] = ca * unb[q][b];
+                    if (MODE == MODE_STAGE2 && ok) a.U0b[pt(q, b)] += ca * unb[q][b];
+                    qb[q][b] = cb * unb[q][b];
+                    rb = cc * dt * unb[q][b];
+                    rsum += ok ? cc * rin[q][b] * unb[q][b] : 0.0;
+                }
+                dvb[q][b] = 4 * b + row < NP ? R(-rb) : R(0);  // R = -div
+            }
+        tri::frag_mma<true, R, G, FB, PB>(afam + FO::LT, dvb, db);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+#pragma unroll
+            for (int b = 0; b < PB; ++b) f[q][b] = dvb[q][b];
+#pragma unroll
+            for (int b = 0; b < FB; ++b) f[q][PB + b] = db[q][b];
+        }
+        tri::frag_mma<true, R, G, 2 * PB, PB + FB>(adj + FO::FT, f, fx);
     }
-    __syncthreads();
-    R div[NP];
+    if (a.dtb_partial) {
+        const double s2 = block_reduce_n<OpSum, NWV>(rsum, sred);
+        if (tid == 0) a.dtb_partial[tile] = s2;
+    }
+    __syncthreads();  // traces of U in place
+
+    // ---- corrected gradient, as the stage forms it; with the flux cotangents to the point lanes
+    R jmp[G][FB];
+    {
+        R jw[2 * G][FB], Q[2 * G][PB], ti[G][FB], fy[G][PB];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) div[i] = R(0);
-    if (live) {
-        R fn[NFP];
+        for (int q = 0; q < G; ++q)
 #pragma unroll
-        for (int j = 0; j < NFP; ++j) fn[j] = R(0);
-#pragma unroll 1
-        for (int m = 0; m < NP; ++m) {
-            const R fr = sFR[sp(el, m, v)], fs = sFS[sp(el, m, v)], frs = fr + fs;
+            for (int b = 0; b < FB; ++b) {
+                const int4 pa = partner(q, b);
+                ti[q][b] = sTu[st(pa.x, pa.y - min(4 * b + row, NFP - 1) % FP) + v];
+            }
 #pragma unroll
-            for (int i = 0; i < NP; ++i)
-                div[i] = fmaR(cop<R>(O0 + m * CA + NP + i), fs, fmaR(cop<R>(O0 + m * CA + i), fr, div[i]));
+        for (int q = 0; q < G; ++q) {
+            R ge[4];
+            load4(sGeo + 4 * elg(q), ge);
 #pragma unroll
-            for (int j = 0; j < NFP; ++j)
-                fn[j] = fmaR(cop<R>(O0 + m * CA + 2 * NP + j), j < FP ? fs : (j < 2 * FP ? frs : fr), fn[j]);
+            for (int b = 0; b < PB; ++b) {
+                Q[2 * q][b] = ge[0] * gd[q][b] + ge[2] * gd[q][PB + b];
+                Q[2 * q + 1][b] = ge[1] * gd[q][b] + ge[3] * gd[q][PB + b];
+                fy[q][b] = ge[1] * fx[q][b] + ge[3] * fx[q][PB + b];   // cotangents of F_y, F_x (total fluxes)
+                fx[q][b] = ge[0] * fx[q][b] + ge[2] * fx[q][PB + b];
+            }
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const int j = 4 * b + row;
+                const R* w = sEw + 4 * (elg(q) * 3 + min(j, NFP - 1) / FP);
+                oth[q][b] = edge_of(q, b) == 3 ? ti[q][b] : oth[q][b];
+                const R d = R(0.5) * (tu[q][b] + oth[q][b]) - tu[q][b];
+                jmp[q][b] = j < NFP ? d : R(0);
+                jw[2 * q][b] = w[0] * jmp[q][b];
+                jw[2 * q + 1][b] = w[1] * jmp[q][b];
+            }
         }
+        tri::frag_mma<false, R, 2 * G, PB, FB>(fam + FO::L, jw, Q);
+        auto put = [&](int r, auto&& val) {
 #pragma unroll
-        for (int j = 0; j < NFP; ++j) sD[sl(el, j, v)] = (j >= FP && j < 2 * FP) ? fn[j] : -fn[j];
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int b = 0; b < PB; ++b) sX[sx_(elg(q), r + 4 * b + row) + v] = val(q, b);
+            tri::wave_lds_fence();
+        };
+        put(0, [&](int q, int b) { return Q[2 * q][b]; });
+        put(NP, [&](int q, int b) { return Q[2 * q + 1][b]; });
+        put(RA, [&](int q, int b) { return fx[q][b]; });
+        put(RB, [&](int q, int b) { return fy[q][b]; });
+    }
+    R ox[G][FB], oy[G][FB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const R* T = a.T_in + remote(partner(q, b).w, b);
+            ox[q][b] = T[NV];
+            oy[q][b] = T[2 * NV];
+        }
+#pragma unroll 1
+    for (int t = lane; t < 4 * G * NP; t += 64) {
+        const int el = wave * 4 * G + t / NP, m = t % NP;
+        R U4[NV], X4[NV], Y4[NV], A4[NV], B4[NV], Fb[NV], Gb[NV];
+        load4(sX + sx_(el, RU + m), U4);
+        load4(sX + sx_(el, m), X4);
+        load4(sX + sx_(el, NP + m), Y4);
+        load4(sX + sx_(el, RA + m), A4);
+        load4(sX + sx_(el, RB + m), B4);
+        R Ub4[NV] = {R(0), R(0), R(0), R(0)}, Xb4[NV] = {R(0), R(0), R(0), R(0)}, Yb4[NV] = {R(0), R(0), R(0), R(0)};
+#pragma unroll
+        for (int w = 0; w < NV; ++w) { Fb[w] = -A4[w]; Gb[w] = -B4[w]; }
+        euler_flux_vjp(U4, g, A4, B4, Ub4);
+        visc_flux_vjp(U4, X4, Y4, g, mu, kappa, Fb, Gb, Ub4, Xb4, Yb4);
+        store4(sX + sx_(el, RU + m), Ub4);
+        store4(sX + sx_(el, m), Xb4);
+        store4(sX + sx_(el, NP + m), Yb4);
+    }
+    tri::wave_lds_fence();
+
+    // ---- point cotangents back; R5: the lifted jumps backwards, R6: the gradient; the BR2 gradients of both
+    // sides of every edge
+    R Qb[2 * G][PB], jb[G][FB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) {
+            const R ub = sX[sx_(elg(q), RU + 4 * b + row) + v];
+            const R xb = sX[sx_(elg(q), 4 * b + row) + v], yb = sX[sx_(elg(q), NP + 4 * b + row) + v];
+            const bool ok = 4 * b + row < NP;
+            qb[q][b] += ok ? double(ub) : 0.0;
+            Qb[2 * q][b] = ok ? xb : R(0);
+            Qb[2 * q + 1][b] = ok ? yb : R(0);
+        }
+    tri::wave_lds_fence();
+    {
+        R f2[G][2 * PB], acc[G][PB];
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            R ge[4];
+            load4(sGeo + 4 * elg(q), ge);
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                f2[q][b] = ge[0] * Qb[2 * q][b] + ge[1] * Qb[2 * q + 1][b];
+                f2[q][PB + b] = ge[2] * Qb[2 * q][b] + ge[3] * Qb[2 * q + 1][b];
+            }
+        }
+        tri::frag_mma<true, R, G, PB, 2 * PB>(adj + FO::DT, f2, acc);
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) qb[q][b] += double(acc[q][b]);
+    }
+    {
+        R lq[2 * G][FB], tg[G][2 * FB], lo[G][4][FB], gyv[G][FB];
+        tri::frag_mma<true, R, 2 * G, FB, PB>(afam + FO::LT, Qb, lq);
+        tri::frag_mma<true, R, G, 2 * FB, PB>(ops + FO::G, ur, tg);
+        tri::diag_mma<R, P>(fam + FO::LF, jmp, lo);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            R ge[4];
+            load4(sGeo + 4 * elg(q), ge);
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const int j = 4 * b + row, ek = edge_of(q, b);
+                R w[4];
+                load4(sEw + 4 * (elg(q) * 3 + min(j, NFP - 1) / FP), w);
+                jb[q][b] = w[0] * lq[2 * q][b] + w[1] * lq[2 * q + 1][b];
+                const R own = eta * lo[q][0][b];
+                R gx = ge[0] * tg[q][b] + ge[2] * tg[q][FB + b] + w[0] * own;
+                R gy = ge[1] * tg[q][b] + ge[3] * tg[q][FB + b] + w[1] * own;
+                const R ln = ek == 0 ? lo[q][1][b] : (ek == 1 ? lo[q][2][b] : lo[q][3][b]);
+                gx = ek == 3 ? gx : R(0.5) * (gx + (ox[q][b] + w[2] * ln));
+                gy = ek == 3 ? gy : R(0.5) * (gy + (oy[q][b] + w[3] * ln));
+                sX[sx_(elg(q), j) + v] = gx;
+                gyv[q][b] = gy;
+            }
+        }
+        auto put = [&](int r, const R (&val)[G][FB]) {
+            tri::wave_lds_fence();
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int b = 0; b < FB; ++b) sX[sx_(elg(q), r + 4 * b + row) + v] = val[q][b];
+        };
+        put(RY, gyv);
+        put(RO, oth);
+        put(RD, db);
     }
     __syncthreads();
     int nsolved = 0;
 #pragma unroll
     for (int w = 0; w < NWV; ++w) nsolved += sCnt[w];
 
-    // the values of one solved face point (slot j of element elt, edge kk):
-    // both sides' traces, edge factors, the face liftings of the jumps and
-    // the averaged state and BR2 gradient
-    struct Face {
-        int elt, kk, j, ek, oj, nl;
-        bool in, right;
-        int2 Lk;
-        R nx, ny, so, sn;
-        R own[NV], oth[NV], Uc[NV], Qbx[NV], Qby[NV];
-    };
-    auto face_at = [&](int t, Face& F) __attribute__((always_inline)) {
+    // ---- R3: every solved face point backwards.  Across tiles the partner's
+    // slot is the edge's own, written last; each slot is read and written by
+    // the lane that solves it alone.
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
         const int c = sList[t / FP], f = t - (t / FP) * FP;
-        F.elt = c / 3;
-        F.kk = c - F.elt * 3;
-        F.j = F.kk * FP + f;
-        F.Lk = sLink[F.elt * 3 + F.kk];
-        F.right = link_role(F.Lk.y) == ROLE_RIGHT;
-        F.nx = sNrm[(F.elt * 3 + F.kk) * 2];
-        F.ny = sNrm[(F.elt * 3 + F.kk) * 2 + 1];
-        F.ek = link_edge(F.Lk.y);
-        F.oj = F.ek * FP + (P - f);
-        F.nl = F.Lk.x - e0;
-        F.in = F.nl >= 0 && F.nl < TT;
-        const R* Tn = a.T_in + (int64_t)F.Lk.x * NFP * TWV;
-        R gxo[NV], gyo[NV], gxn[NV], gyn[NV];
+        const int el = c / 3, j = (c - el * 3) * FP + f;
+        const int4 pc = sPa[c];
+        const int so = sx_(el, j), sn = pc.z == 3 ? sx_(pc.x, pc.y - f) : so;
+        R ns[4], Fcb[NV], ownb[NV], othb[NV], Uc[NV], Ucb[NV] = {R(0), R(0), R(0), R(0)};
+        load4(sNs + 4 * c, ns);
+        const bool right = ns[2] < R(0);
+        {
+            R dn[NV];
+            load4(sX + so + RD * NV, Fcb);
+            load4(sX + sn + RD * NV, dn);
 #pragma unroll
-        for (int w = 0; w < NV; ++w) {
-            F.own[w] = sTu[sl(F.elt, F.j, w)];
-            gxo[w] = sTx[sl(F.elt, F.j, w)];
-            gyo[w] = sTy[sl(F.elt, F.j, w)];
+            for (int w = 0; w < NV; ++w) Fcb[w] = ns[2] * Fcb[w] + ns[3] * dn[w];
         }
-        if (F.in) {
+        {
+            R own[NV], ot[NV], UL[NV], UR[NV];
+            load4(sTu + st(el, j), own);
+            load4(sX + so + RO * NV, ot);
+            R ULb[NV] = {R(0), R(0), R(0), R(0)}, URb[NV] = {R(0), R(0), R(0), R(0)};
 #pragma unroll
             for (int w = 0; w < NV; ++w) {
-                F.oth[w] = sTu[sl(F.nl, F.oj, w)];
-                gxn[w] = sTx[sl(F.nl, F.oj, w)];
-                gyn[w] = sTy[sl(F.nl, F.oj, w)];
+                Uc[w] = R(0.5) * (own[w] + ot[w]);
+                UL[w] = right ? ot[w] : own[w];
+                UR[w] = right ? own[w] : ot[w];
             }
-            F.sn = sEdge[F.nl * 3 + F.ek];
-        } else {
-            load4(Tn + (int64_t)F.oj * TWV, F.oth);
-            load4(Tn + (int64_t)F.oj * TWV + NV, gxn);
-            load4(Tn + (int64_t)F.oj * TWV + 2 * NV, gyn);
-            const R* Gn = a.geo + (int64_t)F.Lk.x * GEO;
-            const R ax = F.ek == 0 ? Gn[2] : (F.ek == 1 ? Gn[0] + Gn[2] : Gn[0]);
-            const R ay = F.ek == 0 ? Gn[3] : (F.ek == 1 ? Gn[1] + Gn[3] : Gn[1]);
-            F.sn = sqrtR(ax * ax + ay * ay);
-        }
-        F.so = sEdge[F.elt * 3 + F.kk];
-        R lo[NV] = {R(0), R(0), R(0), R(0)}, ln[NV] = {R(0), R(0), R(0), R(0)};
-#pragma unroll 1
-        for (int f2 = 0; f2 < FP; ++f2) {
-            const int j2 = F.kk * FP + f2, o2 = F.ek * FP + (P - f2);
-            R uo[NV], un[NV];
-#pragma unroll
-            for (int w = 0; w < NV; ++w) uo[w] = sTu[sl(F.elt, j2, w)];
-            if (F.in) {
-#pragma unroll
-                for (int w = 0; w < NV; ++w) un[w] = sTu[sl(F.nl, o2, w)];
-            } else {
-                load4(Tn + (int64_t)o2 * TWV, un);
-            }
-            const R wo = clf<R>(LFO + (F.kk * FP + f) * FP + f2);
-            const R wn = clf<R>(LFO + (F.ek * FP + (P - f)) * FP + (P - f2));
+            riemann_by_kind_vjp(a.riemann, UL, UR, ns[0], ns[1], g, Fcb, ULb, URb);
 #pragma unroll
             for (int w = 0; w < NV; ++w) {
-                const R jo = R(0.5) * (uo[w] + un[w]) - uo[w];
-                lo[w] = fmaR(wo, jo, lo[w]);
-                ln[w] = fmaR(wn, jo, ln[w]);
+                ownb[w] = right ? URb[w] : ULb[w];
+                othb[w] = right ? ULb[w] : URb[w];
             }
         }
-        const R sg = F.right ? R(-1) : R(1);
-        const R nox = sg * F.nx, noy = sg * F.ny;
-#pragma unroll
-        for (int w = 0; w < NV; ++w) {
-            F.Uc[w] = R(0.5) * (F.own[w] + F.oth[w]);
-            F.Qbx[w] = R(0.5) * ((gxo[w] + eta * F.so * nox * lo[w]) + (gxn[w] + eta * F.sn * nox * ln[w]));
-            F.Qby[w] = R(0.5) * ((gyo[w] + eta * F.so * noy * lo[w]) + (gyn[w] + eta * F.sn * noy * ln[w]));
-        }
-    };
-
-    // ---- forward 3: flux differences of both sides of every solved face point
-#pragma unroll 1
-    for (int t = tid; t < nsolved * FP; t += NB) {
-        Face F;
-        face_at(t, F);
-        R UL[NV], UR[NV], Fc[NV], Fv[NV], Gv[NV];
-#pragma unroll
-        for (int w = 0; w < NV; ++w) {
-            UL[w] = F.right ? F.oth[w] : F.own[w];
-            UR[w] = F.right ? F.own[w] : F.oth[w];
-        }
-        visc_flux(F.Uc, F.Qbx, F.Qby, g, mu, kappa, Fv, Gv);
-        riemann_by_kind(a.riemann, UL, UR, F.nx, F.ny, g, Fc);
-        const R sc = F.right ? -F.so : F.so;
-#pragma unroll
-        for (int w = 0; w < NV; ++w) {
-            const R fi = Fc[w] - (Fv[w] * F.nx + Gv[w] * F.ny);
-            sD[sl(F.elt, F.j, w)] = sc * fi - sD[sl(F.elt, F.j, w)];
-            if (F.in) sD[sl(F.nl, F.oj, w)] = -F.sn * fi - sD[sl(F.nl, F.oj, w)];
-        }
-    }
-    __syncthreads();
-
-    // ---- forward 4 and R1: residual; cotangent of u_out, RK combination
-    double rsum = 0.0;
-    R divb[NP];
-    double qb[NP];
-    if (live) {
-#pragma unroll 1
-        for (int j = 0; j < NFP; ++j) {
-            const R d = sD[sl(el, j, v)];
-#pragma unroll
-            for (int i = 0; i < NP; ++i) div[i] = fmaR(cop<R>(OLT + j * NP + i), d, div[i]);
-        }
-        double unb[NP];
-#pragma unroll
-        for (int i = 0; i < NP; ++i) unb[i] = a.Ub_in[base + (int64_t)i * EB * NV];
-        if (MODE != MODE_RESIDUAL && a.Tb_in) {
-            // edge cotangents of u_out's traces (U, gradient) left on this element's cross-tile edges
-            R tu[NFP], tx[NFP], ty[NFP];
-            bool any = false;
-#pragma unroll
-            for (int kk = 0; kk < 3; ++kk) {
-                const int nl = L[kk].x - e0;
-                const bool cross = !(nl >= 0 && nl < TT);
-                any = any || cross;
-#pragma unroll
-                for (int f = 0; f < FP; ++f) {
-                    const int j = kk * FP + f;
-                    const R* Tb = a.Tb_in + ((int64_t)e * NFP + j) * TWV;
-                    tu[j] = cross ? Tb[v] : R(0);
-                    tx[j] = cross ? Tb[NV + v] : R(0);
-                    ty[j] = cross ? Tb[2 * NV + v] : R(0);
-                }
-            }
-            if (any) {
-                R grb[NP], gsb[NP];
-#pragma unroll
-                for (int m = 0; m < NP; ++m) {
-                    R su = R(0), qx = R(0), qy = R(0);
-#pragma unroll
-                    for (int j = 0; j < NFP; ++j) {
-                        const R w = cop<R>(OI + j * NP + m);
-                        su = fmaR(w, tu[j], su);
-                        qx = fmaR(w, tx[j], qx);
-                        qy = fmaR(w, ty[j], qy);
-                    }
-                    unb[m] += double(su);
-                    grb[m] = rx * qx + ry * qy;
-                    gsb[m] = sx * qx + sy * qy;
-                }
-#pragma unroll
-                for (int m = 0; m < NP; ++m) {
-                    R acc = R(0);
-#pragma unroll
-                    for (int i = 0; i < NP; ++i)
-                        acc = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], acc));
-                    unb[m] += double(acc);
-                }
-            }
-        }
-        const double dt = MODE == MODE_RESIDUAL ? 0.0 : *a.dt_ptr;
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int64_t gi = base + (int64_t)i * EB * NV;
-            double rb;
-            if (MODE == MODE_RESIDUAL) {
-                rb = unb[i];
-                qb[i] = 0.0;
-            } else {
-                if (MODE == MODE_STAGE3) a.U0b[gi] = ca * unb[i];
-                if (MODE == MODE_STAGE2) a.U0b[gi] += ca * unb[i];
-                qb[i] = cb * unb[i];
-                rb = cc * dt * unb[i];
-                rsum += cc * (-double(div[i])) * unb[i];
-            }
-            divb[i] = R(-rb);  // R = -div
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NP; ++i) { divb[i] = R(0); qb[i] = 0.0; }
-    }
-    if (a.dtb_partial) {
-        const double s2 = block_reduce_n<OpSum, NWV>(rsum, sred);
-        if (tid == 0) a.dtb_partial[tile] = s2;
-    }
-    __syncthreads();
-
-    // ---- R2, R4: the lifting transposed; the divergence and normal fluxes
-    // transposed to the x / y flux cotangents at the points
-    if (live) {
-#pragma unroll 1
-        for (int j = 0; j < NFP; ++j) {
-            R acc = R(0);
-#pragma unroll
-            for (int i = 0; i < NP; ++i) acc = fmaR(cop<R>(OLT + j * NP + i), divb[i], acc);
-            sD[sl(el, j, v)] = acc;
-        }
-#pragma unroll 1
-        for (int m = 0; m < NP; ++m) {
-            R frb = R(0), fsb = R(0);
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                frb = fmaR(cop<R>(O0 + m * CA + i), divb[i], frb);
-                fsb = fmaR(cop<R>(O0 + m * CA + NP + i), divb[i], fsb);
-            }
-#pragma unroll
-            for (int j = 0; j < NFP; ++j) {
-                // d = sc F^I - Fn with Fn = -fn (edges 0, 2), +fn (edge 1); fn_j
-                // interpolates fs, fr + fs, fr on edges 0, 1, 2
-                const R im = cop<R>(O0 + m * CA + 2 * NP + j);
-                const R db = sD[sl(el, j, v)];
-                const R fnb = (j >= FP && j < 2 * FP) ? -db : db;
-                if (j >= FP) frb = fmaR(im, fnb, frb);
-                if (j < 2 * FP) fsb = fmaR(im, fnb, fsb);
-            }
-            sFR[sp(el, m, v)] = rx * frb + sx * fsb;  // cotangent of F_x = f_x - F_v
-            sFS[sp(el, m, v)] = ry * frb + sy * fsb;  // and of F_y
-        }
-    }
-    __syncthreads();
-    if (live) {
-#pragma unroll 1
-        for (int q = 0; q < MPL; ++q) {
-            const int m = v + NV * q;
-            if (m >= NP) break;
-            R U4[NV], X4[NV], Y4[NV], A4[NV], B4[NV], Fb[NV], Gb[NV];
+        R Qbx[NV], Qby[NV], Qxb[NV] = {R(0), R(0), R(0), R(0)}, Qyb[NV] = {R(0), R(0), R(0), R(0)};
+        {
+            R gx[NV], gy[NV];
+            load4(sX + so, Qbx);
+            load4(sX + sn, gx);
+            load4(sX + so + RY * NV, Qby);
+            load4(sX + sn + RY * NV, gy);
+            R Fvb[NV], Gvb[NV];
 #pragma unroll
             for (int w = 0; w < NV; ++w) {
-                U4[w] = sU[sp(el, m, w)];
-                X4[w] = sQx[sp(el, m, w)];
-                Y4[w] = sQy[sp(el, m, w)];
-                A4[w] = sFR[sp(el, m, w)];
-                B4[w] = sFS[sp(el, m, w)];
-                Fb[w] = -A4[w];
-                Gb[w] = -B4[w];
+                Qbx[w] = R(0.5) * (Qbx[w] + gx[w]);
+                Qby[w] = R(0.5) * (Qby[w] + gy[w]);
+                Fvb[w] = -Fcb[w] * ns[0];
+                Gvb[w] = -Fcb[w] * ns[1];
             }
-            R Ub4[NV] = {R(0), R(0), R(0), R(0)}, Xb4[NV] = {R(0), R(0), R(0), R(0)},
-              Yb4[NV] = {R(0), R(0), R(0), R(0)};
-            euler_flux_vjp(U4, g, A4, B4, Ub4);
-            visc_flux_vjp(U4, X4, Y4, g, mu, kappa, Fb, Gb, Ub4, Xb4, Yb4);
-#pragma unroll
-            for (int w = 0; w < NV; ++w) {
-                sU[sp(el, m, w)] = Ub4[w];
-                sQx[sp(el, m, w)] = Xb4[w];
-                sQy[sp(el, m, w)] = Yb4[w];
-            }
+            visc_flux_vjp(Uc, Qbx, Qby, g, mu, kappa, Fvb, Gvb, Ucb, Qxb, Qyb);
         }
-    }
-    __syncthreads();
-
-    // ---- R5: the corrected gradient's lifted jumps transposed
-    if (live) {
-#pragma unroll 1
-        for (int j = 0; j < NFP; ++j) {
-            R bx = R(0), by = R(0);
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const R l = cop<R>(OLT + j * NP + i);
-                bx = fmaR(l, sQx[sp(el, i, v)], bx);
-                by = fmaR(l, sQy[sp(el, i, v)], by);
-            }
-            const int kk = j / FP;
-            sJ[sl(el, j, v)] = (kk == 0 ? jwx[0] : (kk == 1 ? jwx[1] : jwx[2])) * bx +
-                               (kk == 0 ? jwy[0] : (kk == 1 ? jwy[1] : jwy[2])) * by;
-        }
-    }
-    __syncthreads();
-
-    // ---- R3: every solved face point backwards
-#pragma unroll 1
-    for (int t = tid; t < nsolved * FP; t += NB) {
-        Face F;
-        face_at(t, F);
-        R UL[NV], UR[NV], Fcb[NV], Fvb[NV], Gvb[NV];
-        const R sc = F.right ? -F.so : F.so;
 #pragma unroll
         for (int w = 0; w < NV; ++w) {
-            UL[w] = F.right ? F.oth[w] : F.own[w];
-            UR[w] = F.right ? F.own[w] : F.oth[w];
-            R fb = sc * sD[sl(F.elt, F.j, w)];
-            if (F.in) fb += -F.sn * sD[sl(F.nl, F.oj, w)];
-            Fcb[w] = fb;
-            Fvb[w] = -fb * F.nx;
-            Gvb[w] = -fb * F.ny;
-        }
-        R ULb[NV] = {R(0), R(0), R(0), R(0)}, URb[NV] = {R(0), R(0), R(0), R(0)};
-        riemann_by_kind_vjp(a.riemann, UL, UR, F.nx, F.ny, g, Fcb, ULb, URb);
-        R Ucb[NV] = {R(0), R(0), R(0), R(0)}, Qxb[NV] = {R(0), R(0), R(0), R(0)}, Qyb[NV] = {R(0), R(0), R(0), R(0)};
-        visc_flux_vjp(F.Uc, F.Qbx, F.Qby, g, mu, kappa, Fvb, Gvb, Ucb, Qxb, Qyb);
-        const R sg = F.right ? R(-1) : R(1);
-        const R nox = sg * F.nx, noy = sg * F.ny;
-        R ownb[NV], othb[NV];
-#pragma unroll
-        for (int w = 0; w < NV; ++w) {
-            const R jo = sJ[sl(F.elt, F.j, w)], jn = F.in ? sJ[sl(F.nl, F.oj, w)] : R(0);
-            ownb[w] = (F.right ? URb[w] : ULb[w]) + R(0.5) * Ucb[w] - R(0.5) * jo + R(0.5) * jn;
-            othb[w] = (F.right ? ULb[w] : URb[w]) + R(0.5) * Ucb[w] + R(0.5) * jo - R(0.5) * jn;
+            ownb[w] += R(0.5) * Ucb[w];
+            othb[w] += R(0.5) * Ucb[w];
             Qxb[w] *= R(0.5);
             Qyb[w] *= R(0.5);
-            sC[sl(F.elt, F.j, w)] = eta * (nox * Qxb[w] + noy * Qyb[w]);
-            sD[sl(F.elt, F.j, w)] = ownb[w];
-            sTx[sl(F.elt, F.j, w)] = Qxb[w];
-            sTy[sl(F.elt, F.j, w)] = Qyb[w];
         }
-        if (F.in) {
-#pragma unroll
-            for (int w = 0; w < NV; ++w) {
-                sD[sl(F.nl, F.oj, w)] = othb[w];
-                sTx[sl(F.nl, F.oj, w)] = Qxb[w];
-                sTy[sl(F.nl, F.oj, w)] = Qyb[w];
-            }
-        } else {
-            R* Tb = a.Tb_out + ((int64_t)F.Lk.x * NFP + F.oj) * TWV;
-            store4(Tb, othb);
-            store4(Tb + NV, Qxb);
-            store4(Tb + 2 * NV, Qyb);
-        }
-    }
-    __syncthreads();
-    // the face liftings transposed: the jump at this point from every point's
-    // lifting cotangents (the seeds c, times each side's edge factor)
-#pragma unroll 1
-    for (int t = tid; t < nsolved * FP; t += NB) {
-        const int c = sList[t / FP], f = t - (t / FP) * FP;
-        const int elt = c / 3, kk = c - elt * 3, j = kk * FP + f;
-        const int2 Lk = sLink[elt * 3 + kk];
-        const int ek = link_edge(Lk.y), oj = ek * FP + (P - f), nl = Lk.x - e0;
-        const bool in = nl >= 0 && nl < TT;
-        const R so = sEdge[elt * 3 + kk];
-        R sn;
-        if (in) {
-            sn = sEdge[nl * 3 + ek];
-        } else {
-            const R* Gn = a.geo + (int64_t)Lk.x * GEO;
-            const R ax = ek == 0 ? Gn[2] : (ek == 1 ? Gn[0] + Gn[2] : Gn[0]);
-            const R ay = ek == 0 ? Gn[3] : (ek == 1 ? Gn[1] + Gn[3] : Gn[1]);
-            sn = sqrtR(ax * ax + ay * ay);
-        }
-        R jb[NV] = {R(0), R(0), R(0), R(0)};
-#pragma unroll 1
-        for (int f1 = 0; f1 < FP; ++f1) {
-            const R w1 = so * clf<R>(LFO + (kk * FP + f1) * FP + f) +
-                         sn * clf<R>(LFO + (ek * FP + (P - f1)) * FP + (P - f));
-#pragma unroll
-            for (int w = 0; w < NV; ++w) jb[w] = fmaR(w1, sC[sl(elt, kk * FP + f1, w)], jb[w]);
-        }
-        // jump = (u_n - u_o) / 2 at this point
-#pragma unroll
-        for (int w = 0; w < NV; ++w) sD[sl(elt, j, w)] -= R(0.5) * jb[w];
-        if (in) {
-#pragma unroll
-            for (int w = 0; w < NV; ++w) sD[sl(nl, oj, w)] += R(0.5) * jb[w];
-        } else {
-            R* Tb = a.Tb_out + ((int64_t)Lk.x * NFP + oj) * TWV;
-#pragma unroll
-            for (int w = 0; w < NV; ++w) Tb[w] += R(0.5) * jb[w];
-        }
+        store4(sX + sn, Qxb);
+        store4(sX + sn + RY * NV, Qyb);
+        store4(sX + sn + RO * NV, othb);
+        store4(sTu + st(el, j), othb);
+        tri::wave_lds_fence();
+        store4(sX + so, Qxb);
+        store4(sX + so + RY * NV, Qyb);
+        store4(sX + so + RO * NV, ownb);
     }
     __syncthreads();
 
-    // ---- R6: traces and gradient transposed; cotangent of q
-    if (!live) return;
-    R grb[NP], gsb[NP];
-    double out[NP];
+    // ---- R7: the face liftings backwards; every edge point's jump cotangent, for both sides
+    R xh[G][FB], yh[G][FB], jt[G][FB];
+    {
+        R l[G][4][FB];
 #pragma unroll
-    for (int m = 0; m < NP; ++m) {
-        R su = R(0), qx = sQx[sp(el, m, v)], qy = sQy[sp(el, m, v)];
+        for (int q = 0; q < G; ++q)
 #pragma unroll
-        for (int j = 0; j < NFP; ++j) {
-            const R w = cop<R>(OI + j * NP + m);
-            su = fmaR(w, sD[sl(el, j, v)], su);
-            qx = fmaR(w, sTx[sl(el, j, v)], qx);
-            qy = fmaR(w, sTy[sl(el, j, v)], qy);
+            for (int b = 0; b < FB; ++b) {
+                const int j = 4 * b + row, ek = edge_of(q, b);
+                const R x = sX[sx_(elg(q), j) + v], y = sX[sx_(elg(q), RY + j) + v];
+                R w[4];
+                load4(sEw + 4 * (elg(q) * 3 + min(j, NFP - 1) / FP), w);
+                xh[q][b] = j < NFP ? x : R(0);
+                yh[q][b] = j < NFP ? y : R(0);
+                l[q][0][b] = eta * (w[0] * xh[q][b] + w[1] * yh[q][b]);
+                const R ln = w[2] * xh[q][b] + w[3] * yh[q][b];
+#pragma unroll
+                for (int o = 0; o < 3; ++o) l[q][o + 1][b] = ek == o ? ln : R(0);
+            }
+        tri::diag_mma_t<R, P>(afam + FO::LFT, l, jt);
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                jt[q][b] += jb[q][b];
+                sX[sx_(elg(q), RD + 4 * b + row) + v] = jt[q][b];
+            }
+    }
+    __syncthreads();
+
+    // ---- R6: traces backwards; cotangent of q
+    R f[G][3 * FB], acc[G][PB];
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+        R ge[4];
+        load4(sGeo + 4 * elg(q), ge);
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const int j = 4 * b + row;
+            const int4 pa = partner(q, b);
+            const R jn = sX[sx_(pa.x, RD + pa.y - min(j, NFP - 1) % FP) + v];
+            const R ub = sX[sx_(elg(q), RO + j) + v], pb = sTu[st(elg(q), j) + v];
+            // the partner's own jumps, in the tile; across tiles the other tile adds them there
+            const R tub = ub - R(0.5) * jt[q][b] + (pa.z == 3 ? R(0.5) * jn : R(0));
+            f[q][b] = j < NFP ? tub : R(0);
+            f[q][FB + b] = ge[0] * xh[q][b] + ge[1] * yh[q][b];
+            f[q][2 * FB + b] = ge[2] * xh[q][b] + ge[3] * yh[q][b];
+            if (pa.z != 3 && j < NFP) {
+                R* T = a.Tb_out + remote(pa.w, b);
+                T[0] = pb + R(0.5) * jt[q][b];
+                T[NV] = xh[q][b];
+                T[2 * NV] = yh[q][b];
+            }
         }
-        out[m] = qb[m] + double(sU[sp(el, m, v)]) + double(su);
-        grb[m] = rx * qx + ry * qy;
-        gsb[m] = sx * qx + sy * qy;
     }
+    tri::frag_mma<true, R, G, PB, 3 * FB>(adj + FO::GT, f, acc);
 #pragma unroll
-    for (int m = 0; m < NP; ++m) {
-        R acc = R(0);
+    for (int q = 0; q < G; ++q)
 #pragma unroll
-        for (int i = 0; i < NP; ++i)
-            acc = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], acc));
-        const int64_t gi = base + (int64_t)m * EB * NV;
-        double o = out[m] + double(acc);
-        if (MODE == MODE_STAGE1) o += a.U0b[gi];
-        a.Ub_out[gi] = o;
-    }
+        for (int b = 0; b < PB; ++b) {
+            if (4 * b + row >= NP || e0 + elg(q) >= a.E) continue;
+            double o = qb[q][b] + double(acc[q][b]);
+            if (MODE == MODE_STAGE1) o += a.U0b[pt(q, b)];
+            a.Ub_out[pt(q, b)] = o;
+        }
 }
 
 // Completion of a cotangent with the Navier-Stokes terms: U_bar plus the
 // transposed traces of U and of its gradient for the cross-tile edge
-// cotangents (12 words per point) that the last adjoint launch left.
+// cotangents (12 words per point) that the last adjoint launch left (tiles of
+// TT elements).  One wave per four elements.
 template <typename R, int P, int TT>
-__global__ __launch_bounds__(TT * NV) void tri_visc_complete_kernel(int E, const int2* __restrict__ links,
-                                                                    const R* __restrict__ geo,
-                                                                    const double* __restrict__ Ub,
-                                                                    const R* __restrict__ Tb,
-                                                                    double* __restrict__ out, int xcd_groups) {
-    using S = TriShape<P>;
-    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
-    constexpr int O0 = ops_offset(P), CA = TriOps<P>::CA, OI = O0 + TriOps<P>::C;
-    const int tid = threadIdx.x, el = tid >> 2, v = tid & 3;
-    const int e0 = tile_of_block(xcd_groups) * TT, e = e0 + el;
-    if (e >= E) return;
-    const int64_t base = blk(e, 0, NP) + v;
-    double acc[NP];
+__global__ __launch_bounds__(BLOCK) void tri_visc_complete_kernel(int E, const int2* __restrict__ links,
+                                                                  const R* __restrict__ geo,
+                                                                  const double* __restrict__ Ub,
+                                                                  const R* __restrict__ Tb,
+                                                                  double* __restrict__ out) {
+    using FO = tri::FragOps<R, P>;
+    constexpr int NP = FO::NP, FP = FO::FP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB;
+    const R* const ops = frag_ops<R>() + tri::frag_offset<R>(P) + FO::ADJ0;
+    const int lane = threadIdx.x & 63, row = lane >> 4, v = lane & 3;
+    const int e = (blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * 4 + ((lane >> 2) & 3), ec = min(e, E - 1);
+    R f[1][3 * FB], acc[1][PB];
+    const R* Ge = geo + (int64_t)ec * GEO;
+    const R rx = Ge[0], ry = Ge[1], sx = Ge[2], sy = Ge[3];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) acc[i] = Ub[base + (int64_t)i * EB * NV];
-    if (Tb) {
-        R tu[NFP], tx[NFP], ty[NFP];
-#pragma unroll
-        for (int kk = 0; kk < 3; ++kk) {
-            const int2 Lk = links[(int64_t)e * 3 + kk];
-            const int nl = Lk.x - e0;
-            const bool cross = !(nl >= 0 && nl < TT);
-#pragma unroll
-            for (int f = 0; f < FP; ++f) {
-                const int j = kk * FP + f;
-                const R* T = Tb + ((int64_t)e * NFP + j) * TWV;
-                tu[j] = cross ? T[v] : R(0);
-                tx[j] = cross ? T[NV + v] : R(0);
-                ty[j] = cross ? T[2 * NV + v] : R(0);
+    for (int b = 0; b < FB; ++b) {
+        const int j = 4 * b + row;
+        f[0][b] = f[0][FB + b] = f[0][2 * FB + b] = R(0);
+        if (Tb && j < NFP) {
+            const int n = links[(int64_t)ec * 3 + j / FP].x;
+            if (n / TT != ec / TT) {
+                const R* T = Tb + ((int64_t)ec * NFP + j) * TWV + v;
+                f[0][b] = T[0];
+                f[0][FB + b] = rx * T[NV] + ry * T[2 * NV];
+                f[0][2 * FB + b] = sx * T[NV] + sy * T[2 * NV];
             }
-        }
-        const R* G = geo + (int64_t)e * GEO;
-        const R rx = G[0], ry = G[1], sx = G[2], sy = G[3];
-        R grb[NP], gsb[NP];
-#pragma unroll
-        for (int m = 0; m < NP; ++m) {
-            R su = R(0), qx = R(0), qy = R(0);
-#pragma unroll
-            for (int j = 0; j < NFP; ++j) {
-                const R w = cop<R>(OI + j * NP + m);
-                su = fmaR(w, tu[j], su);
-                qx = fmaR(w, tx[j], qx);
-                qy = fmaR(w, ty[j], qy);
-            }
-            acc[m] += double(su);
-            grb[m] = rx * qx + ry * qy;
-            gsb[m] = sx * qx + sy * qy;
-        }
-#pragma unroll
-        for (int m = 0; m < NP; ++m) {
-            R s = R(0);
-#pragma unroll
-            for (int i = 0; i < NP; ++i)
-                s = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], s));
-            acc[m] += double(s);
         }
     }
+    tri::frag_mma<true, R, 1, PB, 3 * FB>(ops + FO::GT, f, acc);
+    if (e >= E) return;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) out[base + (int64_t)i * EB * NV] = acc[i];
+    for (int b = 0; b < PB; ++b)
+        if (4 * b + row < NP) {
+            const int64_t gi = blk(e, 4 * b + row, NP) + v;
+            out[gi] = Ub[gi] + double(acc[0][b]);
+        }
 }
 
 // Traces of U on every edge (after a new state is set).
@@ -2543,33 +2392,30 @@ hipError_t tri_complete(int P, int E, const int2* links, const double* Ub, const
     return hipGetLastError();
 }
 
-// The BR2 adjoint's elements per workgroup for an order and precision (0
-// where its LDS arrays would exceed 120 KiB at 16 elements: none at P1-P5).
+// The BR2 adjoint's elements per workgroup for an order and precision.
 int tri_visc_vjp_tile(int P, bool fp64) {
     switch (P) {
-#define ZJ_TV(PP)                                                                                           \
-    case PP:                                                                                                \
-        return fp64 ? (TriViscVjpTile<double, PP>::fits ? TriViscVjpTile<double, PP>::value : 0)            \
-                    : (TriViscVjpTile<float, PP>::fits ? TriViscVjpTile<float, PP>::value : 0);
-        ZJ_TV(1) ZJ_TV(2) ZJ_TV(3) ZJ_TV(4) ZJ_TV(5)
-#undef ZJ_TV
-    default: return 0;
+    case 1: return fp64 ? TriViscVjpTile<double, 1>::value : TriViscVjpTile<float, 1>::value;
+    case 2: return fp64 ? TriViscVjpTile<double, 2>::value : TriViscVjpTile<float, 2>::value;
+    case 3: return fp64 ? TriViscVjpTile<double, 3>::value : TriViscVjpTile<float, 3>::value;
+    case 4: return fp64 ? TriViscVjpTile<double, 4>::value : TriViscVjpTile<float, 4>::value;
+    default: return fp64 ? TriViscVjpTile<double, 5>::value : TriViscVjpTile<float, 5>::value;
     }
 }
 
 template <typename R, int P>
 hipError_t tri_visc_vjp_p(int mode, const TriVjpArgs<R>& a, hipStream_t s) {
-    if constexpr (!TriViscVjpTile<R, P>::fits) {
-        return hipErrorInvalidValue;
+    if constexpr (std::is_same<R, double>::value && P == 4) {
+        return hipErrorInvalidValue;  // refused when the handle is made
     } else {
         constexpr int TT = TriViscVjpTile<R, P>::value;
         const int grid = (std::max(a.E, 1) + TT - 1) / TT;
-        const dim3 blk(TT * NV);
+        const dim3 blk(64 * TriViscVjpTile<R, P>::WV);
         switch (mode) {
-        case MODE_RESIDUAL: klaunch(tri_visc_vjp_kernel<R, P, MODE_RESIDUAL, TT>, grid, blk, 0, s, a); break;
-        case MODE_STAGE1: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE1, TT>, grid, blk, 0, s, a); break;
-        case MODE_STAGE2: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE2, TT>, grid, blk, 0, s, a); break;
-        default: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE3, TT>, grid, blk, 0, s, a); break;
+        case MODE_RESIDUAL: klaunch(tri_visc_vjp_kernel<R, P, MODE_RESIDUAL>, grid, blk, 0, s, a); break;
+        case MODE_STAGE1: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE1>, grid, blk, 0, s, a); break;
+        case MODE_STAGE2: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE2>, grid, blk, 0, s, a); break;
+        default: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE3>, grid, blk, 0, s, a); break;
         }
         return hipGetLastError();
     }
@@ -2588,26 +2434,22 @@ hipError_t tri_visc_vjp(int P, int mode, const TriVjpArgs<R>& a, hipStream_t s) 
 
 template <typename R, int P>
 hipError_t tri_visc_complete_p(int E, const int2* links, const R* geo, const double* Ub, const R* Tb, double* out,
-                               int xcd, hipStream_t s) {
-    if constexpr (!TriViscVjpTile<R, P>::fits) {
-        return hipErrorInvalidValue;
-    } else {
-        constexpr int TT = TriViscVjpTile<R, P>::value;
-        const int grid = (std::max(E, 1) + TT - 1) / TT;
-        tri_visc_complete_kernel<R, P, TT><<<grid, TT * NV, 0, s>>>(E, links, geo, Ub, Tb, out, xcd);
-        return hipGetLastError();
-    }
+                               hipStream_t s) {
+    constexpr int PER = BLOCK / 64 * 4;  // elements per workgroup
+    tri_visc_complete_kernel<R, P, TriViscVjpTile<R, P>::value>
+        <<<(std::max(E, 1) + PER - 1) / PER, BLOCK, 0, s>>>(E, links, geo, Ub, Tb, out);
+    return hipGetLastError();
 }
 
 template <typename R>
 hipError_t tri_visc_complete(int P, int E, const int2* links, const R* geo, const double* Ub, const R* Tb, double* out,
-                             int xcd, hipStream_t s) {
+                             hipStream_t s) {
     switch (P) {
-    case 1: return tri_visc_complete_p<R, 1>(E, links, geo, Ub, Tb, out, xcd, s);
-    case 2: return tri_visc_complete_p<R, 2>(E, links, geo, Ub, Tb, out, xcd, s);
-    case 3: return tri_visc_complete_p<R, 3>(E, links, geo, Ub, Tb, out, xcd, s);
-    case 4: return tri_visc_complete_p<R, 4>(E, links, geo, Ub, Tb, out, xcd, s);
-    default: return tri_visc_complete_p<R, 5>(E, links, geo, Ub, Tb, out, xcd, s);
+    case 1: return tri_visc_complete_p<R, 1>(E, links, geo, Ub, Tb, out, s);
+    case 2: return tri_visc_complete_p<R, 2>(E, links, geo, Ub, Tb, out, s);
+    case 3: return tri_visc_complete_p<R, 3>(E, links, geo, Ub, Tb, out, s);
+    case 4: return tri_visc_complete_p<R, 4>(E, links, geo, Ub, Tb, out, s);
+    default: return tri_visc_complete_p<R, 5>(E, links, geo, Ub, Tb, out, s);
     }
 }
 
@@ -3243,10 +3085,7 @@ extern "C" int zj_tri_get_info(zj_tri_handle h, int64_t* n_dof, int* elems_per_b
 static int tensure_adjoint(zj_tri* h) {
     if (h->A_Ub) return ZJ_OK;
     int tt = TILE;
-    if (h->viscous) {
-        tt = tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64);
-        if (tt == 0) return tfail(h, ZJ_ERR_UNSUPPORTED, "the triangle adjoint's LDS arrays exceed the workgroup's");
-    }
+    if (h->viscous) tt = tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64);
     ZJ_THIP(h, hipSetDevice(h->device));
     h->A_blk = (h->E + tt - 1) / tt;
     const size_t eb = ((size_t)h->E + EB - 1) / EB * EB;
@@ -3274,44 +3113,55 @@ static TriVjpArgs<R> tvjp_args(zj_tri* h) {
     a.mu = h->mu;
     a.kappa = h->kappa;
     a.eta = h->eta;
-    a.lf_off = lf_family(h->corr) * lf_words(h->P);
+    a.family = lf_family(h->corr);
     return a;
 }
 
-// One step backwards: traces of U^n, stages 1 and 2 recomputed into A_W1 and
-// A_W2 (with their cross-tile traces), then the stage VJPs 3, 2, 1, each
+// One step backwards: stages 1 and 2 recomputed into A_W1 and A_W2 (with their
+// cross-tile traces), then the stage VJPs 3, 2, 1, each
 // consuming the edge cotangents the previous launch left.
 template <typename R>
 static hipError_t tri_adjoint_step(zj_tri* h, bool want_dt, hipStream_t s) {
     R** AT = (R**)h->A_T;
     R** Tb = (R**)h->A_Tb;
     const R* geo = (const R*)h->geo;
-    // With the viscous terms every edge's traces are formed after each
-    // recomputed stage: the adjoint's tiles can be smaller than the stage
-    // kernel's, whose own trace writes cover only the edges across its tiles.
-    hipError_t e = h->viscous ? tri_visc_trace<R>(h->P, h->E, h->U, geo, AT[0], s) : tri_trace<R>(h->P, h->E, h->U, AT[0], s);
+    // The Navier-Stokes adjoint's tiles are mostly the stage kernel's, whose
+    // traces (T[0] of the state, then each recomputed stage's) cover the edges
+    // across them; else every edge's traces are formed after each stage.
+    const bool same = h->viscous && tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64) == h->epb;
+    const bool retrace = h->viscous && !same;
+    const R* T[3] = {same ? (const R*)h->T[0] : AT[0], AT[1], AT[2]};
+    hipError_t e = hipSuccess;
+    if (!same)
+        e = h->viscous ? tri_visc_trace<R>(h->P, h->E, h->U, geo, AT[0], s) : tri_trace<R>(h->P, h->E, h->U, AT[0], s);
     if (e != hipSuccess) return e;
     TriArgs<R> f = tri_args<R>(h, MODE_STAGE1);
-    f.U_in = h->U; f.U_out = h->A_W1; f.T_in = AT[0]; f.T_out = AT[1]; f.l2_partial = nullptr;
+    f.U_in = h->U; f.U_out = h->A_W1; f.T_in = T[0]; f.T_out = AT[1]; f.l2_partial = nullptr;
     if ((e = h->viscous ? tri_visc_launch<R>(h->P, MODE_STAGE1, f, s) : tri_launch<R>(h->P, MODE_STAGE1, f, s)) != hipSuccess)
         return e;
-    if (h->viscous && (e = tri_visc_trace<R>(h->P, h->E, h->A_W1, geo, AT[1], s)) != hipSuccess) return e;
+    if (retrace && (e = tri_visc_trace<R>(h->P, h->E, h->A_W1, geo, AT[1], s)) != hipSuccess) return e;
     f = tri_args<R>(h, MODE_STAGE2);
     f.U0 = h->U; f.U_in = h->A_W1; f.U_out = h->A_W2; f.T_in = AT[1]; f.T_out = AT[2]; f.l2_partial = nullptr;
     if ((e = h->viscous ? tri_visc_launch<R>(h->P, MODE_STAGE2, f, s) : tri_launch<R>(h->P, MODE_STAGE2, f, s)) != hipSuccess)
         return e;
-    if (h->viscous && (e = tri_visc_trace<R>(h->P, h->E, h->A_W2, geo, AT[2], s)) != hipSuccess) return e;
+    if (retrace && (e = tri_visc_trace<R>(h->P, h->E, h->A_W2, geo, AT[2], s)) != hipSuccess) return e;
     for (int st = 3; st >= 1; --st) {
         TriVjpArgs<R> a = tvjp_args<R>(h);
         a.U_in = st == 3 ? h->A_W2 : (st == 2 ? h->A_W1 : h->U);
         a.U0 = h->U;
-        a.T_in = AT[st - 1];
+        a.T_in = T[st - 1];
         a.Ub_in = h->A_Ub;
         a.Ub_out = h->A_Ub;
         a.Tb_in = h->A_has_tb ? Tb[h->A_cur] : nullptr;
         a.Tb_out = Tb[1 - h->A_cur];
         a.U0b = h->A_U0b;
         a.dtb_partial = want_dt ? h->A_dtb + (size_t)(3 - st) * h->A_blk : nullptr;
+        if (h->viscous && want_dt) {  // the residual at q, of which the time step's cotangent is made
+            f = tri_args<R>(h, MODE_RESIDUAL);
+            f.U_in = a.U_in; f.T_in = a.T_in; f.l2_partial = nullptr;
+            if ((e = tri_visc_launch<R>(h->P, MODE_RESIDUAL, f, s)) != hipSuccess) return e;
+            a.R_in = h->Rres;
+        }
         if ((e = h->viscous ? tri_visc_vjp<R>(h->P, st, a, s) : tri_vjp<R>(h->P, st, a, s)) != hipSuccess) return e;
         h->A_cur = 1 - h->A_cur;
         h->A_has_tb = true;
@@ -3351,9 +3201,9 @@ extern "C" int zj_tri_adjoint_get_device(zj_tri_handle h, double* d_ubar_aos, vo
     if (h->viscous)
         e = h->prec == ZJ_PREC_FP64
                 ? tri_visc_complete<double>(h->P, h->E, h->links, (const double*)h->geo, h->A_Ub, (const double*)tb,
-                                            h->Rres, h->xcd_groups, s)
+                                            h->Rres, s)
                 : tri_visc_complete<float>(h->P, h->E, h->links, (const float*)h->geo, h->A_Ub, (const float*)tb,
-                                           h->Rres, h->xcd_groups, s);
+                                           h->Rres, s);
     else
         e = h->prec == ZJ_PREC_FP64
                 ? tri_complete<double>(h->P, h->E, h->links, h->A_Ub, (const double*)tb, h->Rres, h->xcd_groups, s)
@@ -3409,7 +3259,7 @@ static hipError_t tri_residual_vjp(zj_tri* h, hipStream_t s) {
     a.Tb_out = tb;
     if (h->viscous) {
         if ((e = tri_visc_vjp<R>(h->P, MODE_RESIDUAL, a, s)) != hipSuccess) return e;
-        return tri_visc_complete<R>(h->P, h->E, h->links, geo, h->Rres, tb, h->W, h->xcd_groups, s);
+        return tri_visc_complete<R>(h->P, h->E, h->links, geo, h->Rres, tb, h->W, s);
     }
     if ((e = tri_vjp<R>(h->P, MODE_RESIDUAL, a, s)) != hipSuccess) return e;
     return tri_complete<R>(h->P, h->E, h->links, h->Rres, tb, h->W, h->xcd_groups, s);

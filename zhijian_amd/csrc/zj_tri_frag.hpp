@@ -167,6 +167,61 @@ __device__ __forceinline__ void diag_mma(const R* t, const R (&b)[G][FB], R (&ac
     }
 }
 
+// The sum of the four operators' transposes, each of its own columns:
+// acc[g] = sum_o operator_o^T . b[g][o].  FP64: the kept 4 x 4 blocks as
+// [row block][column block][operator][16]; FP32: whole tiles of rows.
+template <typename R, int P> struct DiagTTab {
+    using T = DiagTab<P>;
+    static constexpr bool F64 = std::is_same<R, double>::value;
+    static constexpr int FB = T::FB, WORDS = F64 ? 4 * 16 * T::before(FB, 0) : FragTab<R, FB, 4 * FB>::WORDS;
+};
+template <typename R, int P, typename F> void diag_fill_t(R* t, F&& at) {
+    using T = DiagTab<P>;
+    constexpr int FB = T::FB;
+    auto tr = [&](int row, int o, int col) { return at(o, col, row); };
+    if constexpr (DiagTTab<R, P>::F64) {
+        for (int m = 0; m < FB; ++m)
+            for (int k = 0; k < FB; ++k)
+                for (int l = 0; l < 64 && T::nz(m, k); ++l)
+                    t[T::before(m, k) * 64 + l] = R(tr(4 * m + l % 4, l / 16, 4 * k + l / 4 % 4));
+    } else {
+        frag_fill<R, FB, 4 * FB>(t, [&](int row, int c) { return tr(row, c / (4 * FB), c % (4 * FB)); });
+    }
+}
+template <typename R, int P, int G, int FB>
+__device__ __forceinline__ void diag_mma_t(const R* t, const R (&b)[G][4][FB], R (&acc)[G][FB]) {
+    using T = DiagTab<P>;
+    if constexpr (DiagTTab<R, P>::F64) {
+        const int lane = threadIdx.x & 63;
+        const R* s = t + (lane >> 4) * 4 + (lane & 3);
+#pragma unroll
+        for (int m = 0; m < FB; ++m) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) acc[g][m] = R(0);
+#pragma unroll
+            for (int k = 0; k < FB; ++k) {
+                if (!T::nz(m, k)) continue;
+#pragma unroll
+                for (int o = 0; o < 4; ++o) {
+                    const R a = s[T::before(m, k) * 64 + o * 16];
+#pragma unroll
+                    for (int g = 0; g < G; ++g)
+                        acc[g][m] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b[g][o][k], acc[g][m], 0, 0, 0);
+                }
+            }
+        }
+    } else {
+        R f[G][4 * FB];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+#pragma unroll
+                for (int k = 0; k < FB; ++k) f[g][o * FB + k] = b[g][o][k];
+        frag_mma<true, R, G, FB, 4 * FB>(t, f, acc);
+    }
+}
+
 // Orders LDS writes of a wave's lanes before its other lanes' later reads (a
 // wave's LDS operations execute in order; the compiler must keep them so).
 __device__ __forceinline__ void wave_lds_fence() {
@@ -196,6 +251,13 @@ template <typename R> constexpr int elem_stride(int rows) {
 //       at that edge's own points, and, for each of a neighbour's edges 0, 1,
 //       2, the neighbour's face lifting of the same jumps by this side's
 //       points (slots run the other way along a shared edge)
+// and for the adjoint (after the families, its own family parts last):
+//   FT  F backwards: cotangents of F_r, F_s (PB blocks each) from those of
+//       the divergence and of the flux differences      2 PB x (PB + FB)
+//   GT  traces of U and of its gradient's r and s parts backwards  PB x 3 FB
+//   DT  gradient backwards                                       PB x 2 PB
+//   LT  lifting backwards                                          FB x PB
+//   LFT face liftings backwards
 template <typename R, int P> struct FragOps {
     static constexpr int NP = (P + 1) * (P + 2) / 2, FP = P + 1, NFP = 3 * FP;
     static constexpr int PB = (NP + 3) / 4, FB = (NFP + 3) / 4, CB = (2 * NP + 3) / 4;
@@ -207,7 +269,17 @@ template <typename R, int P> struct FragOps {
     static constexpr int L = 0;
     static constexpr int LF = L + FragTab<R, PB, FB>::WORDS;
     static constexpr int FAMILY = LF + DiagTab<P>::WORDS;
-    static constexpr int WORDS = COMMON + 3 * FAMILY;
+    static constexpr int FT = 0;
+    static constexpr int GT = FT + FragTab<R, 2 * PB, PB + FB>::WORDS;
+    static constexpr int DT = GT + FragTab<R, PB, 3 * FB>::WORDS;
+    static constexpr int ADJ = DT + FragTab<R, PB, 2 * PB>::WORDS;
+    static constexpr int LT = 0;
+    static constexpr int LFT = LT + FragTab<R, FB, PB>::WORDS;
+    static constexpr int ADJ_FAMILY = LFT + DiagTTab<R, P>::WORDS;
+    static constexpr int ADJ0 = COMMON + 3 * FAMILY;          // where they begin
+    static constexpr int ADJ_FAM0 = ADJ0 + ADJ;
+    static constexpr int WORDS = ADJ_FAM0 + 3 * ADJ_FAMILY;
+    static_assert(F % 4 == 0 && ADJ % 4 == 0 && ADJ_FAMILY % 4 == 0, "copied by four words");
     static_assert(COMMON % 4 == 0 && FAMILY % 4 == 0, "copied by four words");
 };
 template <typename R> constexpr int frag_offset(int P) {
@@ -249,11 +321,29 @@ template <typename R, int P> void frag_build(R* t, const Operators* fam) {
         };
         auto same = [&](int a, int b) { return a < NFP && b < NFP && a / FP == b / FP; };
         frag_fill<R, PB, FB>(f + O::L, lift);
-        diag_fill<R, P>(f + O::LF, [&](int o, int a, int b) {
+        auto faces = [&](int o, int a, int b) {
             if (!same(a, b)) return 0.0;
             return o == 0 ? lf(a, b) : lf((o - 1) * FP + (P - a % FP), (o - 1) * FP + (P - b % FP));
-        });
+        };
+        diag_fill<R, P>(f + O::LF, faces);
+        R* fa = t + O::ADJ_FAM0 + k * O::ADJ_FAMILY;
+        frag_fill<R, FB, PB>(fa + O::LT, [&](int j, int i) { return lift(i, j); });
+        diag_fill_t<R, P>(fa + O::LFT, faces);
     }
+    R* ad = t + O::ADJ0;
+    frag_fill<R, 2 * PB, PB + FB>(ad + O::FT, [&](int r, int c) {
+        const bool s = r >= 4 * PB;  // a row of F_s
+        const int m = s ? r - 4 * PB : r;
+        if (c < 4 * PB) return s ? ds(c, m) : dr(c, m);
+        const int j = c - 4 * PB;  // flux difference = scaled common flux minus normal flux
+        if (j < FP) return s ? in(j, m) : 0.0;
+        return j < 2 * FP ? -in(j, m) : (s ? 0.0 : in(j, m));
+    });
+    frag_fill<R, PB, 3 * FB>(ad + O::GT, [&](int m, int c) {
+        const int j = c % (4 * FB);
+        return c < 4 * FB ? in(j, m) : in_d(c < 8 * FB, j, m);
+    });
+    frag_fill<R, PB, 2 * PB>(ad + O::DT, [&](int m, int c) { return c < 4 * PB ? dr(c, m) : ds(c - 4 * PB, m); });
 }
 
 }  // namespace tri
