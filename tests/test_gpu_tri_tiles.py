@@ -10,8 +10,11 @@ FP32-bulk increment carries the residual's own FP32 error.
 import numpy as np
 import pytest
 
+from oracle import tri_oracle as T
 from tests.test_gpu_parity import rel, say
 from tests.test_gpu_tri_viscous import _pair, _state
+from zhijian_amd import cases
+from zhijian_amd.tri import TriSolver
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +35,46 @@ def test_tri_viscous_tiles(p, precision, n):
     ri = rel(s.get_state() - U, o.advance(U, dt) - U)
     say(f"  rel L2 residual {r:.3e}, step increment {ri:.3e}")
     assert r < BAR[precision] and ri < BAR[precision]
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 9])
+@pytest.mark.parametrize("p", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("precision", ["fp64", "fp32bulk"])
+def test_tri_euler_tiles(p, precision, n):
+    corr = {1: "dg", 4: "ga", 5: "hu", 9: "sd"}[n]
+    say(f"case: triangle stage, {2 * n * n} elements P{p} {precision} hllc/{corr}")
+    m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
+    s = TriSolver(m.xy, m.tris, p, periodic=(1.0, 1.0), riemann="hllc", precision=precision, corr=corr)
+    o = T.TriTextbook(p, m.xy, m.tris, s.faces, s.normals, riemann="hllc", corr=corr)
+    U = _state(m, p, 7 + n)
+    s.set_state(U)
+    dt = 0.5 * s.dt_cfl(0.5)
+    r = rel(s.residual(), o.residual(U))
+    s.rk3_step(dt)
+    ri = rel(s.get_state() - U, o.advance(U, dt) - U)
+    say(f"  rel L2 residual {r:.3e}, step increment {ri:.3e}")
+    assert r < BAR[precision] and ri < BAR[precision]
+
+
+@pytest.mark.parametrize("p,n,viscous,precision", [(1, 110, False, "fp64"), (1, 111, False, "fp64"), (1, 110, True, "fp64"),
+                                                   (1, 111, True, "fp64"), (2, 127, True, "fp32bulk"),
+                                                   (2, 128, True, "fp32bulk"), (2, 180, False, "fp64"),
+                                                   (2, 182, False, "fp64")])
+def test_tri_form_by_size(p, n, viscous, precision):
+    """Both sides of the element counts (24,576 at P1, 32,768 and 65,536 at P2) from which large meshes take
+    the scalar form of the stage kernels."""
+    say(f"case: triangle stage {'viscous' if viscous else 'inviscid'}, {2 * n * n} elements P{p} {precision}")
+    m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
+    kw = dict(viscous=True, Re=100.0) if viscous else {}
+    s = TriSolver(m.xy, m.tris, p, periodic=(1.0, 1.0), riemann="roe", precision=precision, corr="ga", **kw)
+    o = T.TriTextbook(p, m.xy, m.tris, s.faces, s.normals, riemann="roe", corr="ga")
+    if viscous:
+        o.set_viscous(100.0)
+    U = _state(m, p, n)
+    s.set_state(U)
+    r = rel(s.residual(), o.residual(U))
+    say(f"  rel L2 {r:.3e}, tiles of {s.info()['elems_per_block']}")
+    assert r < BAR[precision]
 
 
 @pytest.mark.parametrize("n", [1, 4, 5])

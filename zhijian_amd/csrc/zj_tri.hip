@@ -17,8 +17,10 @@
 //   Fn_j = interpolated transformed normal flux: -Fs, Fr + Fs, -Fr on edges 0, 1, 2
 //   F^I_j = Riemann flux along the face normal, outward on each side
 //
-// Work mapping: one lane per (element, conservative variable); the four lanes
-// of an element form a DPP quad.  A lane keeps its variable at every solution
+// Work mapping: the stage and the Navier-Stokes kernels apply the operators on
+// the matrix cores (zj_tri_frag.hpp).  The scalar forms (large P1 and P2
+// meshes) and the inviscid adjoint take one lane per (element, conservative
+// variable); the four lanes of an element form a DPP quad.  A lane keeps its variable at every solution
 // point in registers and applies the dense operators as sums of outer
 // products whose entries are wave-uniform, read from constant memory through
 // scalar loads: no operator or state traffic through LDS.  The Euler flux of
@@ -53,6 +55,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -153,6 +156,32 @@ __device__ __forceinline__ int64_t blk(int e, int j, int n) {
 // array: the p+1 points of an edge share one 128-byte line (FP64, p = 3)
 __device__ __forceinline__ int64_t trix(int e, int j, int n) { return ((int64_t)e * n + j) * NV; }
 
+// A wave's rows of point values in the [E/16][NP][16][4] layout, G groups of
+// four elements from element e0 + 4 G wave: at(p, q, b) is row 4 b + lane/16 of
+// this lane's element and variable in group q.  The base is uniform, the
+// lane's part 32 bits (a scalar base and an offset in the load, instead of
+// 64-bit address arithmetic per value).  Rows and groups beyond the mesh are
+// clamped to the last ones; elements beyond it in the last group of four are
+// the layout's padding.
+template <int NP, int G> struct PointRows {
+    static constexpr int PB = (NP + 3) / 4;
+    int first, last;   // this wave's first element, the mesh's last group of four
+    unsigned lo, hi;   // byte offsets of the lane: rows of a whole block, of the last block
+    __device__ __forceinline__ PointRows(int e0, int wave, int lane, int E) {
+        first = e0 + __builtin_amdgcn_readfirstlane(wave) * 4 * G;
+        last = (E - 1) & ~3;
+        const int row = lane >> 4;
+        lo = (unsigned)(row * EB * NV + (lane & 15)) * 8u;
+        hi = (unsigned)(min(4 * (PB - 1) + row, NP - 1) * EB * NV + (lane & 15)) * 8u;
+    }
+    template <typename T> __device__ __forceinline__ T* at(T* p, int q, int b) const {
+        static_assert(sizeof(T) == 8, "state arrays are FP64");
+        using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+        C* const base = reinterpret_cast<C*>(p + blk(min(first + 4 * q, last), 0, NP));
+        return reinterpret_cast<T*>(base + (b < PB - 1 ? 4 * b * EB * NV * 8 + lo : hi));
+    }
+};
+
 template <typename R>
 struct TriArgs {
     int E;
@@ -188,13 +217,14 @@ template <typename R> __device__ __forceinline__ R fast_rcp(R x);
 template <> __device__ __forceinline__ double fast_rcp<double>(double x) { return rcp_refined(x); }
 template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// Waves per SIMD the stage kernel is compiled for: the FP64 P3 kernel fits
-// three (at most 168 VGPRs) without scratch; the rest is left to the compiler.
-template <typename R, int P> struct TriWaves { static constexpr int value = 1; };
-template <> struct TriWaves<double, 3> { static constexpr int value = 3; };
-
+// The stage of large meshes at P1 and P2: lanes one per (element, variable),
+// the operators as scalar operands (see the file's head); higher orders and
+// small meshes take tri_stage_kernel below.  us a stage, this / that: P1 FP64
+// 51,200 elements 11.7 / 15.7, 16,200 7.6 / 7.2, 7,200 7.5 / 5.5; P2 FP64
+// 500,000 166 / 182, 51,200 24 / 21; P2 FP32 80,000 17 / 18, 51,200 14 / 14,
+// 32,768 11 / 9.5.
 template <typename R, int P, int MODE>
-__global__ __launch_bounds__(BLOCK, (TriWaves<R, P>::value)) void tri_stage_kernel(TriArgs<R> a) {
+__global__ __launch_bounds__(BLOCK) void tri_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
     constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
     constexpr int NW = NP > NFP ? NP : NFP;
@@ -410,6 +440,264 @@ __global__ __launch_bounds__(BLOCK, (TriWaves<R, P>::value)) void tri_stage_kern
     }
 }
 
+// The stage on the matrix cores: lanes as zj_tri_frag.hpp has them (a wave
+// owns G groups of four elements, one point row per lane), one lane per point
+// for the Euler fluxes and one per solved face point for the common fluxes,
+// through LDS; loads carry no branches.  Bounded by LDS latency and VALU
+// issue, then memory.  500,000 elements, P3, HLLC, us a stage, one lane per
+// element and variable with scalar operands -> this: FP64
+// 214 / 260 / 264 -> 225 / 232 / 238, FP32 123 / 162 / 167 -> 127 / 150 / 155;
+// on 7,200, whose tiles of 64 left half the CUs idle, 17 -> 7.8 and 14 -> 6.2.
+template <typename R, int P> struct TriTile {
+    static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1);
+    static constexpr int PB = (NP + 3) / 4, FB = (NFP + 3) / 4, CB = (2 * NP + 3) / 4;
+    static constexpr bool BIG = sizeof(R) == 8 && P == 5;
+    static constexpr int G = BIG ? 1 : 2, WV = BIG ? 8 : 4, value = 4 * G * WV, WPE = sizeof(R) == 8 && P >= 4 ? 2 : 3;
+    // rows of an element: traces of U; then U, later F_r, and F_s, later the common fluxes and the
+    // other tiles' traces
+    // P1 and P2 meshes of at least this many elements take the scalar form
+    static constexpr int SCALAR_FROM = P == 1 ? 24576 : (P == 2 ? 65536 : INT_MAX);
+    static constexpr int tile(int E) { return E >= SCALAR_FROM ? TILE : value; }
+    static constexpr int RU = 4 * FB, RO = RU + NFP;
+    static constexpr int ROWS = RU + 4 * CB > RO + 4 * FB ? RU + 4 * CB : RO + 4 * FB;
+    static constexpr int ESX = tri::elem_stride<R>(ROWS);
+};
+
+template <typename R, int P, int MODE>
+__global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) void tri_stage_kernel(TriArgs<R> a) {
+    using TV = TriTile<R, P>;
+    using FO = tri::FragOps<R, P>;
+    constexpr int NP = FO::NP, FP = FO::FP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB, CB = FO::CB;
+    constexpr int G = TV::G, NWV = TV::WV, NB = 64 * NWV, TT = TV::value, ESX = TV::ESX, RU = TV::RU, RO = TV::RO;
+    constexpr int OI = 0, OF = tri::FragTab<R, FB, PB>::WORDS, OL = OF + tri::FragTab<R, PB + FB, CB>::WORDS, OW = OL + tri::FragTab<R, PB, FB>::WORDS;
+    __shared__ R ops[OW];            // the operator tables I, F, L
+    __shared__ R sX[TT * ESX];
+    __shared__ double sred[NWV];
+    __shared__ R sGeo[TT * 4];       // r_x, r_y, s_x, s_y
+    __shared__ R sNs[TT * 3 * 4];    // per edge: face normal, own factor +-|e|/(2J), the partner's -+|e|/(2J)
+    __shared__ int4 sPa[TT * 3];     // per edge: partner's element and slot P of its edge in the tile (the edge's own
+                                     // else); 0 in the tile, 1 across tiles, 2 boundary; then the row of slot P in
+                                     // the trace array, or BC type and data index
+    __shared__ unsigned char sList[TT * 3];
+    __shared__ int sCnt[NWV];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane >> 4, v = lane & 3;
+    const int tile = tile_of_block(a.xcd_groups);
+    const int e0 = tile * TT;
+    const R g = R(a.gamma);
+    auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };  // this lane's element of group q
+        auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };
+
+    const PointRows<NP, G> rows(e0, wave, lane, a.E);
+
+    // ---- 0: state, operators, edges
+    double u[G][PB];
+    R ur[G][PB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) u[q][b] = *rows.at(a.U_in, q, b);
+    {
+        const R* const src = frag_ops<R>() + tri::frag_offset<R>(P);
+        for (int t = 4 * tid; t < OW; t += 4 * NB) {
+            R w[4];
+            load4(src + (t < OF ? FO::I + t : t < OL ? FO::F + t - OF : FO::COMMON + a.family * FO::FAMILY + t - OL), w);
+            store4(ops + t, w);
+        }
+    }
+    static_assert(TT * 3 <= NB, "one lane per edge of the tile");
+    bool owned = false;
+    if (tid < TT * 3) {
+        const int el = tid / 3, k = tid - el * 3, e = min(e0 + el, a.E - 1);
+        const R* Ge = a.geo + (int64_t)e * GEO;
+        const int2 Lk = a.links[(int64_t)e * 3 + k];
+        const int nl = Lk.x - e0, ek = link_edge(Lk.y), role = link_role(Lk.y);
+        const bool right = role == ROLE_RIGHT, live = e0 + el < a.E, bnd = role == ROLE_BOUNDARY;
+        const bool in = !bnd && nl >= 0 && nl < TT;
+        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R ns[4] = {nx, ny, right ? -s : s, right ? sn : -sn};
+        store4(sNs + 4 * tid, ns);
+        const bool self = !live || !in;
+        sPa[tid] = make_int4(self ? el : nl, (self ? k : ek) * FP + P, !live || in ? 0 : (bnd ? 2 : 1),
+                             !live || in ? P : (bnd ? ek | link_bc(Lk.y) << 3 : (int)((unsigned)Lk.x * NFP + ek * FP + P)));
+        owned = live && !(right && in);
+    }
+    if (tid < TT) {
+        R w[4];
+        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        store4(sGeo + 4 * tid, w);
+    }
+    const unsigned long long own_mask = __ballot(owned);
+    if (lane == 0) sCnt[wave] = __popcll(own_mask);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) {
+            ur[q][b] = 4 * b + row < NP ? R(u[q][b]) : R(0);
+            sX[sx_(elg(q), RU + 4 * b + row) + v] = ur[q][b];
+        }
+    __syncthreads();  // operators and edges in place
+
+    // ---- 1: the other tiles' traces on their way, own traces, contravariant
+    // fluxes (one lane per point of the wave's elements, in place of U)
+    R oth[G][FB];
+    unsigned cross = 0;  // one bit per slot: an edge another tile reads
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const int j = min(4 * b + row, NFP - 1);
+            const int4 pa = sPa[elg(q) * 3 + j / FP];
+            cross |= (unsigned)(pa.z == 1 && 4 * b + row < NFP) << (q * FB + b);
+            oth[q][b] = a.T_in[(pa.z == 1 ? (int64_t)(unsigned)pa.w - j % FP : (int64_t)0) * NV + v];
+        }
+    {
+        R tu[G][FB];
+        tri::frag_mma<true, R, G, FB, PB>(ops + OI, ur, tu);
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) sX[sx_(elg(q), 4 * b + row) + v] = tu[q][b];
+    }
+    if (owned) {
+        int pos = __popcll(own_mask & ((1ull << lane) - 1));
+        for (int w = 0; w < wave; ++w) pos += sCnt[w];
+        sList[pos] = (unsigned char)tid;
+    }
+    tri::wave_lds_fence();
+#pragma unroll 1
+    for (int t = lane; t < 4 * G * NP; t += 64) {
+        const int el = wave * 4 * G + t / NP, m = t % NP;
+        R U4[NV], FR[NV], FS[NV], ge[4];
+        load4(sX + sx_(el, RU + m), U4);
+        load4(sGeo + 4 * el, ge);
+        const R inv = fast_rcp(U4[0]);
+        const R ux = U4[1] * inv, uy = U4[2] * inv;
+        const R p = (g - R(1)) * (U4[3] - R(0.5) * (U4[1] * ux + U4[2] * uy));
+        const R fx[NV] = {U4[1], U4[1] * ux + p, U4[1] * uy, (U4[3] + p) * ux};
+        const R fy[NV] = {U4[2], U4[2] * ux, U4[2] * uy + p, (U4[3] + p) * uy};
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            FR[w] = ge[0] * fx[w] + ge[1] * fy[w];
+            FS[w] = ge[2] * fx[w] + ge[3] * fy[w];
+        }
+        store4(sX + sx_(el, RU + m), FR);
+        store4(sX + sx_(el, RU + NP + m), FS);
+    }
+    tri::wave_lds_fence();
+
+    // ---- 2: divergence and transformed normal fluxes
+    R dv[G][PB + FB];
+    {
+        R f[G][CB];
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < CB; ++b) {
+                const R w = sX[sx_(elg(q), RU + 4 * b + row) + v];
+                f[q][b] = 4 * b + row < 2 * NP ? w : R(0);
+            }
+        tri::frag_mma<true, R, G, PB + FB, CB>(ops + OF, f, dv);
+    }
+    tri::wave_lds_fence();  // every read of the point fluxes done
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) sX[sx_(elg(q), RO + 4 * b + row) + v] = oth[q][b];
+    double u0[G][PB];
+    if (MODE == MODE_STAGE2 || MODE == MODE_STAGE3) {
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) u0[q][b] = *rows.at(a.U0, q, b);
+    }
+    __syncthreads();
+    int nsolved = 0;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) nsolved += sCnt[w];
+
+    // ---- 3: common fluxes of the solved face points, scaled by each side's
+    // +-|e|/(2J), at both sides' slots (an in-tile face by its left element;
+    // without a partner in the tile both are the edge's own, written last)
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
+        const int c = sList[t / FP], f = t - (t / FP) * FP;
+        const int el = c / 3, j = (c - el * 3) * FP + f;
+        const int4 pc = sPa[c];
+        R own[NV], ot[NV], ns[4], UL[NV], UR[NV], Fc[NV], d[NV], dn[NV];
+        load4(sX + sx_(el, j), own);
+        load4(sX + (pc.z == 0 ? sx_(pc.x, pc.y - f) : sx_(el, RO + j)), ot);
+        load4(sNs + 4 * c, ns);
+        if (pc.z == 2) ghost_state(own, ns[0], ns[1], pc.w & 7, a.bc_data + (int64_t)(pc.w >> 3) * 8, g, ot);
+        const bool right = ns[2] < R(0);
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            UL[w] = right ? ot[w] : own[w];
+            UR[w] = right ? own[w] : ot[w];
+        }
+        riemann_by_kind(a.riemann, UL, UR, ns[0], ns[1], g, Fc);
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            d[w] = ns[2] * Fc[w];
+            dn[w] = ns[3] * Fc[w];
+        }
+        store4(sX + (pc.z == 0 ? sx_(pc.x, RU + pc.y - f) : sx_(el, RU + j)), dn);
+        tri::wave_lds_fence();
+        store4(sX + sx_(el, RU + j), d);
+    }
+    __syncthreads();
+
+    // ---- 4: lifted flux differences, RK stage update
+    {
+        R d[G][FB], div[G][PB];
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                const R w = sX[sx_(elg(q), RU + 4 * b + row) + v];
+                d[q][b] = 4 * b + row < NFP ? w - dv[q][PB + b] : R(0);
+            }
+#pragma unroll
+            for (int b = 0; b < PB; ++b) div[q][b] = dv[q][b];
+        }
+        tri::frag_mma<false, R, G, PB, FB>(ops + OL, d, div);
+        const double dt = MODE == MODE_RESIDUAL ? 0.0 : *a.dt_ptr;
+        double l2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int e = e0 + elg(q);
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                const int i = 4 * b + row;
+                const bool ok = i < NP && e < a.E;
+                const double res = -double(div[q][b]);
+                double un = res;
+                if (MODE == MODE_STAGE1) un = u[q][b] + dt * res;
+                if (MODE == MODE_STAGE2) un = 0.75 * u0[q][b] + 0.25 * (u[q][b] + dt * res);
+                if (MODE == MODE_STAGE3) un = (1.0 / 3.0) * u0[q][b] + (2.0 / 3.0) * (u[q][b] + dt * res);
+                if (ok) *rows.at(MODE == MODE_RESIDUAL ? a.R_out : a.U_out, q, b) = un;
+                if (MODE == MODE_RESIDUAL || MODE == MODE_STAGE3) l2 += ok ? res * res : 0.0;
+                ur[q][b] = i < NP ? R(un) : R(0);
+            }
+        }
+        if ((MODE == MODE_RESIDUAL || MODE == MODE_STAGE3) && a.l2_partial) {
+            const double s2 = block_reduce_n<OpSum, NWV>(l2, sred);
+            if (tid == 0) a.l2_partial[tile] = s2;
+        }
+    }
+    if (MODE == MODE_RESIDUAL) return;
+
+    // ---- 5: traces of the new stage state on edges another tile reads
+    R tn[G][FB];
+    tri::frag_mma<true, R, G, FB, PB>(ops + OI, ur, tn);
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < FB; ++b)
+            if (cross >> (q * FB + b) & 1) a.T_out[trix(e0 + elg(q), 4 * b + row, NFP) + v] = tn[q][b];
+}
+
 // ------------------------------------------------------------ Navier-Stokes terms
 // The stage with the compressible Navier-Stokes viscous terms, BR2 (textbook
 // scheme; Bassi-Rebay 2 on the triangle's FR correction field), periodic
@@ -441,8 +729,6 @@ __global__ __launch_bounds__(BLOCK, (TriWaves<R, P>::value)) void tri_stage_kern
 // 354 / 390 / 384 -> 241 / 272 / 277 (1.9 TB/s of the stage's traffic).
 constexpr int TWV = 12;
 
-template <typename R, int P> constexpr bool tri_visc_scalar() { return P == 1 || (P == 2 && sizeof(R) == 4); }
-
 // The workgroup: WV waves of G groups each, 4 G WV elements.
 // LDS per element: the traces of U, then one region that holds U with the
 // corrected gradient, the point fluxes in its place, and at last both traces
@@ -451,7 +737,10 @@ template <typename R, int P> struct TriViscTile {
     static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1), PB = (NP + 3) / 4, FB = (NFP + 3) / 4;
     static constexpr bool BIG = sizeof(R) == 8 && P == 5;
     static constexpr int G = BIG ? 1 : 2, WV = BIG ? 8 : 4;
-    static constexpr int value = tri_visc_scalar<R, P>() ? 64 : 4 * G * WV;
+    static constexpr int value = 4 * G * WV;
+    // P1 and FP32 P2 meshes of at least this many elements take the scalar form, in tiles of 64
+    static constexpr int SCALAR_FROM = P == 1 ? 24576 : (P == 2 && sizeof(R) == 4 ? 32768 : INT_MAX);
+    static constexpr int tile(int E) { return E >= SCALAR_FROM ? TILE : value; }
     // rows of an element's region: Q_x, then F_r, at 0; Q_y, then F_s, at NP; U at RU; then the
     // gradient traces x (later the common fluxes) at 0 and y at NFP, the partner's U traces at
     // 2 NFP.  Arrays are stored whole blocks of four rows at a time, in the order of their rows,
@@ -491,9 +780,10 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
     const int e0 = tile * TT;
     const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
     auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };  // this lane's element of group q
-    auto eg = [&](int q) { return min(e0 + elg(q), a.E - 1); };                // ... in the mesh, clamped to it
-    auto st = [](int elx, int j) { return elx * ESF + j * NV; };               // trace slots
+        auto st = [](int elx, int j) { return elx * ESF + j * NV; };               // trace slots
     auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };              // rows of the other region
+
+    const PointRows<NP, G> rows(e0, wave, lane, a.E);
 
     // ---- 0: state, gradient, traces of U
     double u[G][PB];
@@ -501,7 +791,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
 #pragma unroll
     for (int q = 0; q < G; ++q)
 #pragma unroll
-        for (int b = 0; b < PB; ++b) u[q][b] = a.U_in[blk(eg(q), min(4 * b + row, NP - 1), NP) + v];
+        for (int b = 0; b < PB; ++b) u[q][b] = *rows.at(a.U_in, q, b);
     {
         const R* const src = frag_ops<R>() + tri::frag_offset<R>(P);
         for (int t = 4 * tid; t < FO::COMMON + FO::FAMILY; t += 4 * NB) {
@@ -711,7 +1001,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
 #pragma unroll
         for (int q = 0; q < G; ++q)
 #pragma unroll
-            for (int b = 0; b < PB; ++b) u0[q][b] = a.U0[blk(eg(q), min(4 * b + row, NP - 1), NP) + v];
+            for (int b = 0; b < PB; ++b) u0[q][b] = *rows.at(a.U0, q, b);
     }
     __syncthreads();
     int nsolved = 0;
@@ -790,7 +1080,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
                 if (MODE == MODE_STAGE1) un = u[q][b] + dt * res;
                 if (MODE == MODE_STAGE2) un = 0.75 * u0[q][b] + 0.25 * (u[q][b] + dt * res);
                 if (MODE == MODE_STAGE3) un = (1.0 / 3.0) * u0[q][b] + (2.0 / 3.0) * (u[q][b] + dt * res);
-                if (ok) (MODE == MODE_RESIDUAL ? a.R_out : a.U_out)[blk(e, i, NP) + v] = un;
+                if (ok) *rows.at(MODE == MODE_RESIDUAL ? a.R_out : a.U_out, q, b) = un;
                 if (MODE == MODE_RESIDUAL || MODE == MODE_STAGE3) l2 += ok ? res * res : 0.0;
                 ur[q][b] = i < NP ? R(un) : R(0);
             }
@@ -822,13 +1112,15 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
     }
 }
 
-// The stage at the lowest orders (P1, and P2 in FP32): lanes as in
-// tri_stage_kernel, one per element and variable, the operators as scalar
-// operands.  A point has few operator entries there and padding to blocks of
-// four costs the matrix-core form a third of its rows: on 80,000 elements P1
-// takes 33 / 20 us a stage (FP64 / FP32) against 39 / 22, FP32 P2 34-37
-// against 36-38; FP64 P2 takes 85 against 59.  The point values (U, then Q)
-// live in LDS, each lane reads a point's four variables there.
+// The stage of large meshes at the lowest orders (P1, and P2 in FP32): lanes
+// as in tri_scalar_kernel, one per element and variable, the operators as
+// scalar operands.  A point has few operator entries there, and padding to
+// blocks of four costs the matrix-core form a third of its rows; but its
+// tiles of 64 leave a small mesh's CUs idle.  us a stage, this / matrix cores:
+// P1 FP64 32,768 elements 13 / 17, 16,200 10.5 / 9.5, 7,200 10 / 7; P1 FP32
+// 80,000 20 / 22, 16,200 9 / 7; P2 FP32 80,000 36 / 37, 32,768 16.7 / 17.1,
+// 16,200 14 / 10 (P2 FP64 80,000 85 / 59).  The point values (U, then Q) live
+// in LDS, each lane reads a point's four variables there.
 template <typename R, int P, int MODE, int TT>
 __global__ __launch_bounds__(TT * NV) void tri_visc_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
@@ -1724,10 +2016,9 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
     const int e0 = tile * TT;
     const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
     auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };
-    auto eg = [&](int q) { return min(e0 + elg(q), a.E - 1); };
     auto st = [](int elx, int j) { return elx * ESF + j * NV; };
     auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };
-    auto pt = [&](int q, int b) { return blk(eg(q), min(4 * b + row, NP - 1), NP) + v; };
+    const PointRows<NP, G> rows(e0, wave, lane, a.E);
 
     // ---- 0: q, the incoming cotangent, operators and edges
     R ur[G][PB];
@@ -1736,9 +2027,9 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
     for (int q = 0; q < G; ++q)
 #pragma unroll
         for (int b = 0; b < PB; ++b) {
-            ur[q][b] = R(a.U_in[pt(q, b)]);
-            unb[q][b] = a.Ub_in[pt(q, b)];
-            rin[q][b] = MODE != MODE_RESIDUAL && a.dtb_partial ? a.R_in[pt(q, b)] : 0.0;
+            ur[q][b] = R(*rows.at(a.U_in, q, b));
+            unb[q][b] = *rows.at(a.Ub_in, q, b);
+            rin[q][b] = MODE != MODE_RESIDUAL && a.dtb_partial ? *rows.at(a.R_in, q, b) : 0.0;
         }
     {
         const R* const src = frag_ops<R>() + tri::frag_offset<R>(P);
@@ -1828,7 +2119,7 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
                     // own slots across tiles (the others read the tile's first row in common)
                     const int j = 4 * b + row;
                     const bool on = edge_of(q, b) != 3 && j < NFP;
-                    const R* T = a.Tb_in + (on ? (int64_t)eg(q) * NFP + j : (int64_t)0) * TWV + v;
+                    const R* T = a.Tb_in + (on ? (int64_t)(e0 + elg(q)) * NFP + j : (int64_t)0) * TWV + v;
                     const R tb = T[0], xb = T[NV], yb = T[2 * NV];
                     f[q][b] = on ? tb : R(0);
                     f[q][FB + b] = on ? ge[0] * xb + ge[1] * yb : R(0);
@@ -1851,8 +2142,8 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
                 double rb = unb[q][b];
                 qb[q][b] = 0.0;
                 if (MODE != MODE_RESIDUAL) {
-                    if (MODE == MODE_STAGE3 && ok) a.U0b[pt(q, b)] = ca * unb[q][b];
-                    if (MODE == MODE_STAGE2 && ok) a.U0b[pt(q, b)] += ca * unb[q][b];
+                    if (MODE == MODE_STAGE3 && ok) *rows.at(a.U0b, q, b) = ca * unb[q][b];
+                    if (MODE == MODE_STAGE2 && ok) *rows.at(a.U0b, q, b) += ca * unb[q][b];
                     qb[q][b] = cb * unb[q][b];
                     rb = cc * dt * unb[q][b];
                     rsum += ok ? cc * rin[q][b] * unb[q][b] : 0.0;
@@ -2158,8 +2449,8 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
         for (int b = 0; b < PB; ++b) {
             if (4 * b + row >= NP || e0 + elg(q) >= a.E) continue;
             double o = qb[q][b] + double(acc[q][b]);
-            if (MODE == MODE_STAGE1) o += a.U0b[pt(q, b)];
-            a.Ub_out[pt(q, b)] = o;
+            if (MODE == MODE_STAGE1) o += *rows.at(a.U0b, q, b);
+            *rows.at(a.Ub_out, q, b) = o;
         }
 }
 
@@ -2275,12 +2566,22 @@ __global__ __launch_bounds__(BLOCK) void tri_dt_kernel(const double* __restrict_
 
 template <typename R, int P>
 hipError_t tri_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
-    const int grid = (std::max(a.E, 1) + TILE - 1) / TILE;
+    using TV = TriTile<R, P>;
+    const int TT = TV::tile(a.E), grid = (std::max(a.E, 1) + TT - 1) / TT;
+    auto launch = [&](auto m) {
+        constexpr int MODE = decltype(m)::value;
+        if constexpr (TV::SCALAR_FROM < INT_MAX)
+            if (a.E >= TV::SCALAR_FROM) {
+                klaunch(tri_scalar_kernel<R, P, MODE>, grid, dim3(BLOCK), 0, s, a);
+                return;
+            }
+        klaunch(tri_stage_kernel<R, P, MODE>, grid, dim3(64 * TV::WV), 0, s, a);
+    };
     switch (mode) {
-    case MODE_RESIDUAL: klaunch(tri_stage_kernel<R, P, MODE_RESIDUAL>, grid, dim3(BLOCK), 0, s, a); break;
-    case MODE_STAGE1: klaunch(tri_stage_kernel<R, P, MODE_STAGE1>, grid, dim3(BLOCK), 0, s, a); break;
-    case MODE_STAGE2: klaunch(tri_stage_kernel<R, P, MODE_STAGE2>, grid, dim3(BLOCK), 0, s, a); break;
-    default: klaunch(tri_stage_kernel<R, P, MODE_STAGE3>, grid, dim3(BLOCK), 0, s, a); break;
+    case MODE_RESIDUAL: launch(std::integral_constant<int, MODE_RESIDUAL>{}); break;
+    case MODE_STAGE1: launch(std::integral_constant<int, MODE_STAGE1>{}); break;
+    case MODE_STAGE2: launch(std::integral_constant<int, MODE_STAGE2>{}); break;
+    default: launch(std::integral_constant<int, MODE_STAGE3>{}); break;
     }
     return hipGetLastError();
 }
@@ -2301,14 +2602,16 @@ hipError_t tri_visc_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
     if constexpr (std::is_same<R, double>::value && P == 4) {
         return hipErrorInvalidValue;  // refused when the handle is made
     } else {
-        constexpr int TT = TriViscTile<R, P>::value;
-        const int grid = (std::max(a.E, 1) + TT - 1) / TT;
+        using TV = TriViscTile<R, P>;
+        const int TT = TV::tile(a.E), grid = (std::max(a.E, 1) + TT - 1) / TT;
         auto launch = [&](auto m) {
             constexpr int MODE = decltype(m)::value;
-            if constexpr (tri_visc_scalar<R, P>())
-                klaunch(tri_visc_scalar_kernel<R, P, MODE, TT>, grid, dim3(TT * NV), 0, s, a);
-            else
-                klaunch(tri_visc_stage_kernel<R, P, MODE>, grid, dim3(64 * TriViscTile<R, P>::WV), 0, s, a);
+            if constexpr (TV::SCALAR_FROM < INT_MAX)
+                if (a.E >= TV::SCALAR_FROM) {
+                    klaunch(tri_visc_scalar_kernel<R, P, MODE, TILE>, grid, dim3(BLOCK), 0, s, a);
+                    return;
+                }
+            klaunch(tri_visc_stage_kernel<R, P, MODE>, grid, dim3(64 * TV::WV), 0, s, a);
         };
         switch (mode) {
         case MODE_RESIDUAL: launch(std::integral_constant<int, MODE_RESIDUAL>{}); break;
@@ -2345,13 +2648,23 @@ hipError_t tri_visc_trace(int P, int E, const double* U, const R* geo, R* T, hip
     return hipGetLastError();
 }
 
-int tri_visc_tile(int P, bool fp64) {
+int tri_visc_tile(int P, bool fp64, int E) {
     switch (P) {
-    case 1: return fp64 ? TriViscTile<double, 1>::value : TriViscTile<float, 1>::value;
-    case 2: return fp64 ? TriViscTile<double, 2>::value : TriViscTile<float, 2>::value;
-    case 3: return fp64 ? TriViscTile<double, 3>::value : TriViscTile<float, 3>::value;
-    case 4: return fp64 ? TriViscTile<double, 4>::value : TriViscTile<float, 4>::value;
-    default: return fp64 ? TriViscTile<double, 5>::value : TriViscTile<float, 5>::value;
+    case 1: return fp64 ? TriViscTile<double, 1>::tile(E) : TriViscTile<float, 1>::tile(E);
+    case 2: return fp64 ? TriViscTile<double, 2>::tile(E) : TriViscTile<float, 2>::tile(E);
+    case 3: return fp64 ? TriViscTile<double, 3>::tile(E) : TriViscTile<float, 3>::tile(E);
+    case 4: return fp64 ? TriViscTile<double, 4>::tile(E) : TriViscTile<float, 4>::tile(E);
+    default: return fp64 ? TriViscTile<double, 5>::tile(E) : TriViscTile<float, 5>::tile(E);
+    }
+}
+
+int tri_tile(int P, bool fp64, int E) {
+    switch (P) {
+    case 1: return fp64 ? TriTile<double, 1>::tile(E) : TriTile<float, 1>::tile(E);
+    case 2: return fp64 ? TriTile<double, 2>::tile(E) : TriTile<float, 2>::tile(E);
+    case 3: return fp64 ? TriTile<double, 3>::tile(E) : TriTile<float, 3>::tile(E);
+    case 4: return fp64 ? TriTile<double, 4>::tile(E) : TriTile<float, 4>::tile(E);
+    default: return fp64 ? TriTile<double, 5>::tile(E) : TriTile<float, 5>::tile(E);
     }
 }
 
@@ -2690,7 +3003,7 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
         h->kappa = h->mu * p->gamma / ((p->gamma - 1.0) * p->Pr);
         h->eta = p->br2_eta > 0.0 ? p->br2_eta : 2.0;
     }
-    h->epb = h->viscous ? tri_visc_tile(P, h->prec == ZJ_PREC_FP64) : TILE;
+    h->epb = h->viscous ? tri_visc_tile(P, h->prec == ZJ_PREC_FP64, h->E) : tri_tile(P, h->prec == ZJ_PREC_FP64, h->E);
     h->nblk = (h->E + h->epb - 1) / h->epb;
     const int E = h->E;
 
@@ -3125,10 +3438,11 @@ static hipError_t tri_adjoint_step(zj_tri* h, bool want_dt, hipStream_t s) {
     R** AT = (R**)h->A_T;
     R** Tb = (R**)h->A_Tb;
     const R* geo = (const R*)h->geo;
-    // The Navier-Stokes adjoint's tiles are mostly the stage kernel's, whose
-    // traces (T[0] of the state, then each recomputed stage's) cover the edges
-    // across them; else every edge's traces are formed after each stage.
-    const bool same = h->viscous && tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64) == h->epb;
+    // The Navier-Stokes adjoint's tiles are mostly whole tiles of the stage
+    // kernel, whose traces (T[0] of the state, then each recomputed stage's)
+    // cover the edges across them; else every edge's traces are formed after
+    // each stage.
+    const bool same = h->viscous && tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64) % h->epb == 0;
     const bool retrace = h->viscous && !same;
     const R* T[3] = {same ? (const R*)h->T[0] : AT[0], AT[1], AT[2]};
     hipError_t e = hipSuccess;
