@@ -133,3 +133,25 @@ def test_viscous_multi_step_vjp():
     rr = abs(dre - refd) / abs(refd)
     say(f"  dJ/dRe: adjoint {dre:.12e}  Richardson FD {refd:.12e}  rel {rr:.2e}")
     assert rr < TOL
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 7])
+@pytest.mark.parametrize("precision", ["fp64", "fp32bulk"])
+@pytest.mark.parametrize("p", [1, 2, 3, 4, 5])
+def test_viscous_vjp_tiles(p, precision, n):
+    """Faces of one tile, which are solved backwards once for both sides, against faces across tiles, which each
+    side solves: an element that is its own neighbour (1 x 1), pairs that share two faces (2 x 2), one tile of P3 (4 x 4), several
+    tiles with a remainder (7 x 7).  Bars as above: FP64 is held to the finite difference's own
+    error; an FP32-bulk VJP carries FP32 rounding (6e-8) over some hundreds of terms a cotangent."""
+    say(f"case: viscous VJP tiles, TGV {n}x{n} P{p} hllc/dg Re 100 {precision}")
+    s, tb, t = _pair(cases.tgv_mesh(n), p, "hllc", "dg", precision=precision)
+    U = _state(t, 90 + p)
+    w = np.random.default_rng(91 + n).standard_normal(U.shape)
+    v = direction(U, 92 + n)
+    tol = TOL if precision == "fp64" else 2e-4
+    s.set_state(U)
+    assert dot_check(float(w @ fd(tb.residual, U, v)), float(s.residual_vjp(w) @ v), "residual") < tol
+    dt = 1e-3
+    s.adjoint_set(w)
+    s.rk3_step_vjp(dt)
+    assert dot_check(float(w @ fd(lambda X: tb.advance(X, dt, False), U, v)), float(s.adjoint_get() @ v), "step") < tol

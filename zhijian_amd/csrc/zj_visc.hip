@@ -545,68 +545,31 @@ __global__ __launch_bounds__(BLOCK) void visc_trace_kernel(int E, const double* 
 //       fluxes, the metric, the Euler and viscous flux VJPs, which give the
 //       cotangent of the corrected gradient Q; its correction terms
 //       transposed onto the jumps
-//   R4  per face point, as the forward solves it (both sides solve each
-//       face): the Riemann and viscous common-flux VJPs, the BR2 gradients
+//   R4  per face point, once for both sides in the tile (the common flux's
+//       cotangent sums both flux differences'; across tiles each side takes
+//       its own): the Riemann and viscous common-flux VJPs, the BR2 gradients
 //       and jumps backwards, to this side's trace and gradient-trace
 //       cotangents and the partner's (LDS in the tile, HBM across tiles)
 //   R5  the transposed traces; the gradient's cotangent through the
 //       transposed gradient operator; the cotangent of q
 // Traces and their cotangents across tiles carry 12 words per face point:
 // U, dU/dx, dU/dy.
+// Bound by waiting: LDS round trips and FP64 chains between nine barriers, so
+// what counts is the waves per SIMD.  Four point and four trace arrays whose
+// roles follow one another (66 KB at FP64 P3) let two workgroups share a CU
+// where one array per quantity (123 KB) let one; the registers are held to
+// the same (256) by reading a face's traces again behind its Riemann VJP and
+// by keeping the cotangent of q in LDS over R4.  Solving an in-tile face once
+// halves R4's flux VJPs.  128x128 P3 FP64, a checkpointed gradient over 32
+// steps (96 forward stages and 96 of these): 9.40 -> 7.09 ms.  A step
+// backwards at 128x128, us, P1..P5: FP64 143, 273, 297, 500, 694 -> 118, 209,
+// 228, 383, 506; FP32-bulk 105, 234, 167, 287, 377 -> 91, 153, 163, 247, 318.
 template <typename R, int P>
 constexpr int visc_adj_epb() {
-    using Y = Lay<R, P>;
-    constexpr int full = BLOCK / ((P + 1) * (P + 1));
-    // LDS within 120 KiB (gfx950 gives a workgroup up to 160 KiB): every
-    // order's full tile at both precisions
-    constexpr int cap = 122880 / ((6 * Y::UE + 9 * Y::TE) * (int)sizeof(R));
-    return cap < 1 ? 1 : (cap < full ? cap : full);
-}
-
-// Both traces and both BR2 lifting coefficients of one face point of
-// element el2 (edge k, point f), the partner read from LDS or HBM.
-template <typename R, int P>
-struct ViscFacePoint {
-    R own[NV], oth[NV], gxo[NV], gyo[NV], gxn[NV], gyn[NV];
-    R ax, ay, bx, by;
-};
-
-template <typename R, int P>
-__device__ __forceinline__ void visc_face_point(ViscFacePoint<R, P>& F, const R* sU, const R* sGx, const R* sGy,
-                                                const R* sTr, const R* sLm, const R* sLp, const R* T_in,
-                                                const R* Jinv, int e0, int epb, int el2, int e2, int k, int f,
-                                                const EdgeLink& L, R eta, R gLe, R gRe) {
-    using Y = Lay<R, P>;
-    constexpr int FP = P + 1;
-    const int nl = L.nbr - e0;
-    const bool inside = nl >= 0 && nl < epb;
-    const int oslot = P - f;
-    const TraceLine tl = trace_line<P>(k, f);
-    const TraceLine tn = trace_line<P>(L.nbr_edge, oslot);
-    const R* T = T_in + (((int64_t)L.nbr * 4 + L.nbr_edge) * FP + oslot) * TW;
-    const R* Jo = Jinv + (int64_t)e2 * 4;
-    const R* Jn = Jinv + (int64_t)L.nbr * 4;
-    const bool oxi = (k & 1) != 0, nxi = (L.nbr_edge & 1) != 0;
-    const R go = eta * ((k == 0 || k == 3) ? gLe : gRe);
-    const R gn = eta * ((L.nbr_edge == 0 || L.nbr_edge == 3) ? gLe : gRe);
-    F.ax = go * (oxi ? Jo[0] : Jo[2]); F.ay = go * (oxi ? Jo[1] : Jo[3]);
-    F.bx = gn * (nxi ? Jn[0] : Jn[2]); F.by = gn * (nxi ? Jn[1] : Jn[3]);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        F.own[v] = sTr[Y::tr(el2, k, f, v)];
-        if (inside) {
-            F.oth[v] = sTr[Y::tr(nl, L.nbr_edge, oslot, v)];
-            F.gxn[v] = trace_point<R, P>(sGx + nl * Y::UE + v * Y::UV, tn, sLm, sLp);
-            F.gyn[v] = trace_point<R, P>(sGy + nl * Y::UE + v * Y::UV, tn, sLm, sLp);
-        } else {
-            F.oth[v] = T[v];
-            F.gxn[v] = T[NV + v];
-            F.gyn[v] = T[2 * NV + v];
-        }
-        F.gxo[v] = trace_point<R, P>(sGx + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
-        F.gyo[v] = trace_point<R, P>(sGy + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
-    }
-    (void)sU;
+    // one point and one face point per thread: 32 and 21 elements at P1 and P2,
+    // 16, 10 and 7 at P3-P5.  That is within the 80 KiB of LDS of which two
+    // workgroups fit on a CU at both precisions.
+    return BLOCK / (4 * (P + 1)) < BLOCK / ((P + 1) * (P + 1)) ? BLOCK / (4 * (P + 1)) : BLOCK / ((P + 1) * (P + 1));
 }
 
 template <typename R, int P, int EPB, int MODE, int NTHR>
@@ -617,18 +580,22 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
     constexpr bool HAS_U0 = MODE == MODE_STAGE2 || MODE == MODE_STAGE3;
     constexpr int N1 = P + 1, S = N1 * N1, FP = N1;
     constexpr int NT = EPB * S, NF = EPB * 4 * FP;
-    static_assert(NT <= NTHR, "tile exceeds the workgroup");
+    static_assert(NT <= NTHR && EPB * 4 <= NTHR, "tile exceeds the workgroup");
     constexpr double ca = MODE == MODE_STAGE2 ? 0.75 : (MODE == MODE_STAGE3 ? 1.0 / 3.0 : 0.0);
     constexpr double cb = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
     constexpr double cc = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
-    __shared__ R sU[EPB * Y::UE], sGx[EPB * Y::UE], sGy[EPB * Y::UE];
+    __shared__ R sA[EPB * (Y::UE > Y::TE ? Y::UE : Y::TE)];                  // q, then the jumps
     __shared__ R sW1[EPB * Y::UE], sW2[EPB * Y::UE], sW3[EPB * Y::UE];
-    __shared__ R sTr[EPB * Y::TE], sJ[EPB * Y::TE], sFI[EPB * Y::TE];
-    __shared__ R sAu[EPB * Y::TE], sAx[EPB * Y::TE], sAy[EPB * Y::TE];  // incoming, then own-side cotangents
-    __shared__ R sNu[EPB * Y::TE], sNx[EPB * Y::TE], sNy[EPB * Y::TE];  // cotangents from in-tile partners
+    __shared__ R sTr[EPB * Y::TE];                                           // traces of q
+    // incoming edge cotangents of U and grad U; then flux differences (their
+    // cotangents) and traces of grad U; then the traces' cotangents
+    __shared__ R sFI[EPB * Y::TE], sTGx[EPB * Y::TE], sTGy[EPB * Y::TE];
     __shared__ R sD[N1 * N1], sLm[N1], sLp[N1], sC[2 * N1];
-    __shared__ unsigned char sIn[EPB * 4];
+    __shared__ unsigned short sList[EPB * 4];  // edges whose face points this tile solves backwards
+    __shared__ int sCnt[NTHR / 64];
     __shared__ double sRed[BLOCK / 64];
+    R* const sU = sA;
+    R* const sJ = sA;
 
     const int tid = threadIdx.x;
     const int e0 = tile * EPB;
@@ -648,149 +615,51 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
     // the forward residual is needed only for the dt cotangent
     const bool need_res = MODE != MODE_RESIDUAL && a.dtb_partial != nullptr;
 
-    // ---- forward A: stage input
-    double q[NV], u0[NV];
+    // ---- 0: stage input; incoming edge cotangents; the solved edges (an
+    // in-tile face by its left element, for both sides)
+    R Uq[NV] = {R(1), R(0), R(0), R(1)};
     R jx = R(0), jy = R(0), kx = R(0), ky = R(0);
     if (active) {
         jx = a.Jinv[(int64_t)e * 4]; jy = a.Jinv[(int64_t)e * 4 + 1];
         kx = a.Jinv[(int64_t)e * 4 + 2]; ky = a.Jinv[(int64_t)e * 4 + 3];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            u0[v] = HAS_U0 ? a.U0[v * PS + gi] : 0.0;
-            q[v] = (INC && HAS_U0) ? u0[v] + double(a.dW_in[v * PS + gi]) : a.U_in[v * PS + gi];
-            sU[ub + v * Y::UV] = R(q[v]);
+            const double q = (INC && HAS_U0) ? a.U0[v * PS + gi] + double(a.dW_in[v * PS + gi]) : a.U_in[v * PS + gi];
+            Uq[v] = R(q);
+            sU[ub + v * Y::UV] = Uq[v];
         }
     }
-    __syncthreads();
-
-    // ---- forward B1: gradient, own traces; incoming edge cotangents
-    if (active) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-            point_gradient<R, P>(sU + el * Y::UE + v * Y::UV, sD, i, j, jx, jy, kx, ky, sGx[ub + v * Y::UV],
-                                 sGy[ub + v * Y::UV]);
-    }
-    for (int t = tid; t < NF; t += NTHR) {
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        const int e2 = e0 + el2;
-        if (e2 >= a.E) continue;
-        const TraceLine tl = trace_line<P>(k, f);
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-            sTr[Y::tr(el2, k, f, v)] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
-        const EdgeLink L = a.links[(int64_t)e2 * 4 + k];
+    bool owned = false;
+    if (tid < EPB * 4 && e0 + tid / 4 < a.E) {
+        const EdgeLink L = a.links[(int64_t)e0 * 4 + tid];
         const int nl = L.nbr - e0;
-        const bool inside = nl >= 0 && nl < EPB;
-        if (f == 0) sIn[el2 * 4 + k] = inside;
-        R tb[TW];
-#pragma unroll
-        for (int w = 0; w < TW; ++w) tb[w] = R(0);
-        if (incoming && !inside) {
-            const R* src = a.Tb_in + (((int64_t)e2 * 4 + k) * FP + f) * TW;
-            load4(src, tb);
-            load4(src + NV, tb + NV);
-            load4(src + 2 * NV, tb + 2 * NV);
-        }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            sAu[Y::tr(el2, k, f, v)] = tb[v];
-            sAx[Y::tr(el2, k, f, v)] = tb[NV + v];
-            sAy[Y::tr(el2, k, f, v)] = tb[2 * NV + v];
-        }
+        owned = !(L.role == ROLE_RIGHT && nl >= 0 && nl < EPB);
     }
-    __syncthreads();
-
-    // ---- forward B2: jumps, common fluxes (viscous and Riemann), outward and scaled
-    for (int t = tid; t < NF; t += NTHR) {
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        const int e2 = e0 + el2;
-        if (e2 >= a.E) continue;
-        const EdgeLink L = a.links[(int64_t)e2 * 4 + k];
-        const R nx = a.normals[((int64_t)e2 * 4 + k) * 2], ny = a.normals[((int64_t)e2 * 4 + k) * 2 + 1];
-        ViscFacePoint<R, P> F;
-        visc_face_point<R, P>(F, sU, sGx, sGy, sTr, sLm, sLp, a.T_in, a.Jinv, e0, EPB, el2, e2, k, f, L, eta, gLe,
-                              gRe);
-        R qx[NV], qy[NV], Um[NV], Fv[NV], Gv[NV], UL[NV], UR[NV], Fc[NV];
-        const bool right = L.role == ROLE_RIGHT;
+    const unsigned long long own_mask = __ballot(owned);
+    if ((tid & 63) == 0) sCnt[tid >> 6] = __popcll(own_mask);
+    if (incoming)
+        for (int t = tid; t < NF; t += NTHR) {
+            const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+            const int e2 = e0 + el2;
+            if (e2 >= a.E) continue;
+            const int nl = a.links[(int64_t)e2 * 4 + k].nbr - e0;
+            R tb[TW];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const R uc = R(0.5) * (F.own[v] + F.oth[v]);
-            const R jo = uc - F.own[v], jn = uc - F.oth[v];
-            sJ[Y::tr(el2, k, f, v)] = jo;
-            qx[v] = R(0.5) * ((F.gxo[v] + F.ax * jo) + (F.gxn[v] + F.bx * jn));
-            qy[v] = R(0.5) * ((F.gyo[v] + F.ay * jo) + (F.gyn[v] + F.by * jn));
-            Um[v] = uc;
-            UL[v] = right ? F.oth[v] : F.own[v];
-            UR[v] = right ? F.own[v] : F.oth[v];
-        }
-        if (!need_res) continue;  // the jumps are all the reverse phases use
-        visc_flux(Um, qx, qy, g, mu, kappa, Fv, Gv);
-        riemann_by_kind(a.riemann, UL, UR, nx, ny, g, Fc);
-        const R ef = a.edge_f[(int64_t)e2 * 4 + k];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const R fc = Fc[v] - (Fv[v] * nx + Gv[v] * ny);
-            sFI[Y::tr(el2, k, f, v)] = ef * (right ? -fc : fc);
-        }
-    }
-    __syncthreads();
-
-    // ---- forward C: corrected gradient; contravariant total fluxes
-    auto corrected = [&](int v, R& Qx, R& Qy) {
-        const R cxi = sC[i] * sJ[Y::tr(el, 3, P - j, v)] + sC[N1 + i] * sJ[Y::tr(el, 1, j, v)];
-        const R ceta = sC[j] * sJ[Y::tr(el, 0, i, v)] + sC[N1 + j] * sJ[Y::tr(el, 2, P - i, v)];
-        Qx = sGx[ub + v * Y::UV] + jx * cxi + kx * ceta;
-        Qy = sGy[ub + v * Y::UV] + jy * cxi + ky * ceta;
-    };
-    if (active && need_res) {
-        R Uq[NV], Qx[NV], Qy[NV], fx[NV], fy[NV], Fv[NV], Gv[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            Uq[v] = sU[ub + v * Y::UV];
-            corrected(v, Qx[v], Qy[v]);
-        }
-        euler_flux(Uq, g, fx, fy);
-        visc_flux(Uq, Qx, Qy, g, mu, kappa, Fv, Gv);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const R Fx = fx[v] - Fv[v], Fy = fy[v] - Gv[v];
-            sW1[ub + v * Y::UV] = jx * Fx + jy * Fy;
-            sW2[ub + v * Y::UV] = kx * Fx + ky * Fy;
-        }
-    }
-    __syncthreads();
-
-    // ---- forward D: flux differences (in place of the common fluxes)
-    for (int t = tid; need_res && t < NF; t += NTHR) {
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        if (e0 + el2 >= a.E) continue;
-        const TraceLine tl = trace_line<P>(k, f);
-        const R* Fb = ((k & 1) ? sW1 : sW2) + el2 * Y::UE;
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-            sFI[Y::tr(el2, k, f, v)] = sFI[Y::tr(el2, k, f, v)] - trace_point<R, P>(Fb + v * Y::UV, tl, sLm, sLp);
-    }
-    __syncthreads();
-
-    // ---- forward E: residual
-    double res[NV] = {0.0, 0.0, 0.0, 0.0};
-    if (active && need_res) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const R* Fx = sW1 + el * Y::UE + v * Y::UV;
-            const R* Fy = sW2 + el * Y::UE + v * Y::UV;
-            R dxi = 0, deta = 0;
-#pragma unroll
-            for (int m = 0; m < N1; ++m) {
-                dxi += sD[i * N1 + m] * Fx[j * N1 + m];
-                deta += sD[j * N1 + m] * Fy[m * N1 + i];
+            for (int w = 0; w < TW; ++w) tb[w] = R(0);
+            if (!(nl >= 0 && nl < EPB)) {
+                const R* src = a.Tb_in + (((int64_t)e2 * 4 + k) * FP + f) * TW;
+                load4(src, tb);
+                load4(src + NV, tb + NV);
+                load4(src + 2 * NV, tb + 2 * NV);
             }
-            const R c = sFI[Y::tr(el, 3, P - j, v)] * sC[i] + sFI[Y::tr(el, 1, j, v)] * sC[N1 + i] +
-                        sFI[Y::tr(el, 0, i, v)] * sC[j] + sFI[Y::tr(el, 2, P - i, v)] * sC[N1 + j];
-            res[v] = double(-(dxi + deta + c));
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                sFI[Y::tr(el2, k, f, v)] = tb[v];
+                sTGx[Y::tr(el2, k, f, v)] = tb[NV + v];
+                sTGy[Y::tr(el2, k, f, v)] = tb[2 * NV + v];
+            }
         }
-    }
-    __syncthreads();  // the fluxes in sW1, sW2 are read
+    __syncthreads();
 
     // transposed traces (edges 0..3 at this point's slots) of a trace array
     auto trace_t = [&](const R* A, int v) -> R {
@@ -807,20 +676,40 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
         return acc;
     };
 
-    // ---- R1a: incoming gradient-trace cotangents onto the reference derivatives
-    if (incoming && active) {
+    // ---- forward: gradient, own traces; R1a: incoming gradient-trace
+    // cotangents onto the reference derivatives
+    R gx[NV], gy[NV];
+    if (active) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const R gbx = trace_t(sAx, v), gby = trace_t(sAy, v);
-            sW1[ub + v * Y::UV] = jx * gbx + jy * gby;
-            sW2[ub + v * Y::UV] = kx * gbx + ky * gby;
+            point_gradient<R, P>(sU + el * Y::UE + v * Y::UV, sD, i, j, jx, jy, kx, ky, gx[v], gy[v]);
+            if (incoming) {
+                const R gbx = trace_t(sTGx, v), gby = trace_t(sTGy, v);
+                sW1[ub + v * Y::UV] = jx * gbx + jy * gby;
+                sW2[ub + v * Y::UV] = kx * gbx + ky * gby;
+            }
         }
     }
+    for (int t = tid; t < NF; t += NTHR) {
+        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+        if (e0 + el2 >= a.E) continue;
+        const TraceLine tl = trace_line<P>(k, f);
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+            sTr[Y::tr(el2, k, f, v)] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+    }
+    if (owned) {
+        int pos = __popcll(own_mask & ((1ull << (tid & 63)) - 1));
+        for (int w = 0; w < tid >> 6; ++w) pos += sCnt[w];
+        sList[pos] = (unsigned short)tid;
+    }
     __syncthreads();
+    int nsolved = 0;
+#pragma unroll
+    for (int w = 0; w < NTHR / 64; ++w) nsolved += sCnt[w];
 
     // ---- R1b: cotangent of the stage output, RK combination
-    double rsum = 0.0;
-    double qb[NV] = {0.0, 0.0, 0.0, 0.0};
+    double qb[NV] = {0.0, 0.0, 0.0, 0.0}, runb[NV] = {0.0, 0.0, 0.0, 0.0};
     if (active) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
@@ -830,49 +719,197 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
             } else {
                 const double dt = *a.dt_ptr;
                 double unb = a.Ub_in[v * PS + gi];
-                if (incoming) unb += double(trace_t(sAu, v)) + double(grad_t(v));
+                if (incoming) unb += double(trace_t(sFI, v)) + double(grad_t(v));
                 if (MODE == MODE_STAGE3) a.U0b[v * PS + gi] = ca * unb;
                 if (MODE == MODE_STAGE2) a.U0b[v * PS + gi] += ca * unb;
                 qb[v] = cb * unb;
                 rb = cc * dt * unb;
-                rsum += cc * res[v] * unb;
+                runb[v] = cc * unb;
             }
             sW3[ub + v * Y::UV] = R(rb);
         }
     }
-    if (a.dtb_partial) {
-        const double s = block_reduce_n<OpSum, NTHR / 64>(rsum, sRed);
-        if (tid == 0) a.dtb_partial[tile] = s;
-    }
-    __syncthreads();
-
-    // ---- R2: cotangents of the flux differences (in place)
-    for (int t = tid; t < NF; t += NTHR) {
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        if (e0 + el2 >= a.E) continue;
-        const R* Rb = sW3 + el2 * Y::UE;
-        const bool odd = (k & 1) != 0;
-        const int line = (k == 0 || k == 1) ? f : P - f;
-        const R* gw = sC + ((k == 1 || k == 2) ? N1 : 0);
+    if (incoming) __syncthreads();
+    if (active) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            R acc = R(0);
-#pragma unroll
-            for (int m = 0; m < N1; ++m) acc -= gw[m] * Rb[v * Y::UV + (odd ? line * N1 + m : m * N1 + line)];
-            sFI[Y::tr(el2, k, f, v)] = acc;
+            sW1[ub + v * Y::UV] = gx[v];
+            sW2[ub + v * Y::UV] = gy[v];
         }
     }
     __syncthreads();
 
+    // ---- forward: traces of the gradient, jumps; R2: cotangents of the flux differences
+    auto flux_difference_cotangents = [&]() {
+        for (int t = tid; t < NF; t += NTHR) {
+            const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+            if (e0 + el2 >= a.E) continue;
+            const R* Rb = sW3 + el2 * Y::UE;
+            const bool odd = (k & 1) != 0;
+            const int line = (k == 0 || k == 1) ? f : P - f;
+            const R* gw = sC + ((k == 1 || k == 2) ? N1 : 0);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                R acc = R(0);
+#pragma unroll
+                for (int m = 0; m < N1; ++m) acc -= gw[m] * Rb[v * Y::UV + (odd ? line * N1 + m : m * N1 + line)];
+                sFI[Y::tr(el2, k, f, v)] = acc;
+            }
+        }
+    };
+    for (int t = tid; t < NF; t += NTHR) {
+        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+        const int e2 = e0 + el2;
+        if (e2 >= a.E) continue;
+        const TraceLine tl = trace_line<P>(k, f);
+        const EdgeLink L = a.links[(int64_t)e2 * 4 + k];
+        const int nl = L.nbr - e0, oslot = P - f;
+        const bool inside = nl >= 0 && nl < EPB;
+        R oth[NV];
+        if (!inside) load4(a.T_in + (((int64_t)L.nbr * 4 + L.nbr_edge) * FP + oslot) * TW, oth);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            sTGx[Y::tr(el2, k, f, v)] = trace_point<R, P>(sW1 + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+            sTGy[Y::tr(el2, k, f, v)] = trace_point<R, P>(sW2 + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+            const R own = sTr[Y::tr(el2, k, f, v)];
+            if (inside) oth[v] = sTr[Y::tr(nl, L.nbr_edge, oslot, v)];
+            sJ[Y::tr(el2, k, f, v)] = R(0.5) * (own + oth[v]) - own;
+        }
+    }
+    if (!need_res) flux_difference_cotangents();
+    __syncthreads();
+
+    // both sides' traces of one face point
+    auto face_traces = [&](int el2, int k, int f, const EdgeLink& L, R* own, R* oth) __attribute__((always_inline)) {
+        const int nl = L.nbr - e0, oslot = P - f;
+        const bool inside = nl >= 0 && nl < EPB;
+        R far[NV] = {R(0), R(0), R(0), R(0)};
+        if (!inside) load4(a.T_in + (((int64_t)L.nbr * 4 + L.nbr_edge) * FP + oslot) * TW, far);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            own[v] = sTr[Y::tr(el2, k, f, v)];
+            const R near = sTr[Y::tr(inside ? nl : el2, L.nbr_edge, oslot, v)];
+            oth[v] = inside ? near : far[v];
+        }
+    };
+    // its common state and BR2 gradient, with both sides' lifting coefficients
+    auto face_gradient = [&](int el2, int k, int f, const EdgeLink& L, const R* own, const R* oth, R* uc, R* qx, R* qy,
+                             R& ax, R& ay, R& bx, R& by) __attribute__((always_inline)) {
+        const int e2 = e0 + el2, nl = L.nbr - e0, oslot = P - f;
+        const bool inside = nl >= 0 && nl < EPB;
+        const R* Jo = a.Jinv + (int64_t)e2 * 4;
+        const R* Jn = a.Jinv + (int64_t)L.nbr * 4;
+        const bool oxi = (k & 1) != 0, nxi = (L.nbr_edge & 1) != 0;
+        const R go = eta * ((k == 0 || k == 3) ? gLe : gRe);
+        const R gn = eta * ((L.nbr_edge == 0 || L.nbr_edge == 3) ? gLe : gRe);
+        ax = go * Jo[oxi ? 0 : 2]; ay = go * Jo[oxi ? 1 : 3];
+        bx = gn * Jn[nxi ? 0 : 2]; by = gn * Jn[nxi ? 1 : 3];
+        R gxn[NV] = {R(0), R(0), R(0), R(0)}, gyn[NV] = {R(0), R(0), R(0), R(0)};
+        if (!inside) {
+            const R* T = a.T_in + (((int64_t)L.nbr * 4 + L.nbr_edge) * FP + oslot) * TW;
+            load4(T + NV, gxn);
+            load4(T + 2 * NV, gyn);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int s = Y::tr(inside ? nl : el2, L.nbr_edge, oslot, v);
+            gxn[v] = inside ? sTGx[s] : gxn[v];
+            gyn[v] = inside ? sTGy[s] : gyn[v];
+            uc[v] = R(0.5) * (own[v] + oth[v]);
+            const R jo = uc[v] - own[v], jn = uc[v] - oth[v];
+            qx[v] = R(0.5) * ((sTGx[Y::tr(el2, k, f, v)] + ax * jo) + (gxn[v] + bx * jn));
+            qy[v] = R(0.5) * ((sTGy[Y::tr(el2, k, f, v)] + ay * jo) + (gyn[v] + by * jn));
+        }
+    };
+    auto corrected = [&](int v, R& Qx, R& Qy) {
+        const R cxi = sC[i] * sJ[Y::tr(el, 3, P - j, v)] + sC[N1 + i] * sJ[Y::tr(el, 1, j, v)];
+        const R ceta = sC[j] * sJ[Y::tr(el, 0, i, v)] + sC[N1 + j] * sJ[Y::tr(el, 2, P - i, v)];
+        Qx = gx[v] + jx * cxi + kx * ceta;
+        Qy = gy[v] + jy * cxi + ky * ceta;
+    };
+
+    // ---- forward residual, for the time step's cotangent alone: common fluxes
+    // (outward and scaled), contravariant total fluxes, flux differences
+    if (need_res) {
+        for (int t = tid; t < NF; t += NTHR) {
+            const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+            const int e2 = e0 + el2;
+            if (e2 >= a.E) continue;
+            const EdgeLink L = a.links[(int64_t)e2 * 4 + k];
+            const R nx = a.normals[((int64_t)e2 * 4 + k) * 2], ny = a.normals[((int64_t)e2 * 4 + k) * 2 + 1];
+            R own[NV], oth[NV], uc[NV], qx[NV], qy[NV], ax, ay, bx, by, Fv[NV], Gv[NV], UL[NV], UR[NV], Fc[NV];
+            face_traces(el2, k, f, L, own, oth);
+            face_gradient(el2, k, f, L, own, oth, uc, qx, qy, ax, ay, bx, by);
+            const bool right = L.role == ROLE_RIGHT;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                UL[v] = right ? oth[v] : own[v];
+                UR[v] = right ? own[v] : oth[v];
+            }
+            visc_flux(uc, qx, qy, g, mu, kappa, Fv, Gv);
+            riemann_by_kind(a.riemann, UL, UR, nx, ny, g, Fc);
+            const R ef = a.edge_f[(int64_t)e2 * 4 + k];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const R fc = Fc[v] - (Fv[v] * nx + Gv[v] * ny);
+                sFI[Y::tr(el2, k, f, v)] = ef * (right ? -fc : fc);
+            }
+        }
+        if (active) {
+            R Qx[NV], Qy[NV], fx[NV], fy[NV], Fv[NV], Gv[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) corrected(v, Qx[v], Qy[v]);
+            euler_flux(Uq, g, fx, fy);
+            visc_flux(Uq, Qx, Qy, g, mu, kappa, Fv, Gv);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const R Fx = fx[v] - Fv[v], Fy = fy[v] - Gv[v];
+                sW1[ub + v * Y::UV] = jx * Fx + jy * Fy;
+                sW2[ub + v * Y::UV] = kx * Fx + ky * Fy;
+            }
+        }
+        __syncthreads();
+        for (int t = tid; t < NF; t += NTHR) {
+            const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+            if (e0 + el2 >= a.E) continue;
+            const TraceLine tl = trace_line<P>(k, f);
+            const R* Fb = ((k & 1) ? sW1 : sW2) + el2 * Y::UE;
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                sFI[Y::tr(el2, k, f, v)] = sFI[Y::tr(el2, k, f, v)] - trace_point<R, P>(Fb + v * Y::UV, tl, sLm, sLp);
+        }
+        __syncthreads();
+        double rsum = 0.0;
+        if (active) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const R* Fx = sW1 + el * Y::UE + v * Y::UV;
+                const R* Fy = sW2 + el * Y::UE + v * Y::UV;
+                R dxi = 0, deta = 0;
+#pragma unroll
+                for (int m = 0; m < N1; ++m) {
+                    dxi += sD[i * N1 + m] * Fx[j * N1 + m];
+                    deta += sD[j * N1 + m] * Fy[m * N1 + i];
+                }
+                const R c = sFI[Y::tr(el, 3, P - j, v)] * sC[i] + sFI[Y::tr(el, 1, j, v)] * sC[N1 + i] +
+                            sFI[Y::tr(el, 0, i, v)] * sC[j] + sFI[Y::tr(el, 2, P - i, v)] * sC[N1 + j];
+                rsum += double(-(dxi + deta + c)) * runb[v];
+            }
+        }
+        const double s = block_reduce_n<OpSum, NTHR / 64>(rsum, sRed);
+        if (tid == 0) a.dtb_partial[tile] = s;
+        __syncthreads();  // the flux differences are read
+        flux_difference_cotangents();
+        __syncthreads();
+    }
+
     // ---- R3: fluxes at the points backwards; the corrected gradient's cotangent
-    R Qxb[NV] = {R(0), R(0), R(0), R(0)}, Qyb[NV] = {R(0), R(0), R(0), R(0)};
     double musum = 0.0;  // <cotangent of F_v, F_v> over this thread's points and face points
     if (active) {
         const R* rbp = sW3 + el * Y::UE;
-        R Uq[NV], Qx[NV], Qy[NV], Fxb[NV], Fyb[NV];
+        R Qx[NV], Qy[NV], Fxb[NV], Fyb[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            Uq[v] = sU[ub + v * Y::UV];
             corrected(v, Qx[v], Qy[v]);
             const R* rv = rbp + v * Y::UV;
             // the flux traces enter the differences negatively
@@ -886,7 +923,8 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
             Fxb[v] = jx * ftb + kx * gtb;
             Fyb[v] = jy * ftb + ky * gtb;
         }
-        R ubq[NV] = {R(0), R(0), R(0), R(0)}, nFx[NV], nFy[NV];
+        R ubq[NV] = {R(0), R(0), R(0), R(0)}, Qxb[NV] = {R(0), R(0), R(0), R(0)}, Qyb[NV] = {R(0), R(0), R(0), R(0)};
+        R nFx[NV], nFy[NV];
         euler_flux_vjp(Uq, g, Fxb, Fyb, ubq);
 #pragma unroll
         for (int v = 0; v < NV; ++v) { nFx[v] = -Fxb[v]; nFy[v] = -Fyb[v]; }
@@ -906,50 +944,54 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
     }
     __syncthreads();
 
-    // ---- R4: face points backwards
-    for (int t = tid; t < NF; t += NTHR) {
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        const int e2 = e0 + el2;
-        if (e2 >= a.E) continue;
+    if constexpr (!INC)  // registers for R4, whose Riemann VJP holds the most live values
+        if (active) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) sW3[ub + v * Y::UV] = R(qb[v]);
+        }
+
+    // ---- R4: the solved face points backwards, with the flux differences'
+    // cotangents of both sides in the tile.  A slot is read and then written
+    // by the thread that solves its face alone.
+    for (int t = tid; t < nsolved * FP; t += NTHR) {
+        const int c = sList[t / FP], f = t - (t / FP) * FP;
+        const int el2 = c / 4, k = c - el2 * 4, e2 = e0 + el2;
         const EdgeLink L = a.links[(int64_t)e2 * 4 + k];
         const R nx = a.normals[((int64_t)e2 * 4 + k) * 2], ny = a.normals[((int64_t)e2 * 4 + k) * 2 + 1];
-        const int nl = L.nbr - e0;
+        const int nl = L.nbr - e0, oslot = P - f;
         const bool inside = nl >= 0 && nl < EPB;
-        const int oslot = P - f;
-        // the jump's cotangent from the correction terms of the points on this slot's line
-        const bool odd = (k & 1) != 0;
-        const int line = (k == 0 || k == 1) ? f : P - f;
-        const R* gw = sC + ((k == 1 || k == 2) ? N1 : 0);
-        const R* Cb = (odd ? sW1 : sW2) + el2 * Y::UE;
-        ViscFacePoint<R, P> F;
-        visc_face_point<R, P>(F, sU, sGx, sGy, sTr, sLm, sLp, a.T_in, a.Jinv, e0, EPB, el2, e2, k, f, L, eta, gLe,
-                              gRe);
         const bool right = L.role == ROLE_RIGHT;
-        R Jb[NV], uc[NV], jo[NV], jn[NV], qx[NV], qy[NV], UL[NV], UR[NV], Fcb[NV], Fvb[NV], Gvb[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
+        // a jump's cotangent from the correction terms of the points on its slot's line
+        auto jump_cotangent = [&](int elx, int kx_, int fx_, int v) {
+            const bool odd = (kx_ & 1) != 0;
+            const int line = (kx_ == 0 || kx_ == 1) ? fx_ : P - fx_;
+            const R* gw = sC + ((kx_ == 1 || kx_ == 2) ? N1 : 0);
+            const R* Cb = (odd ? sW1 : sW2) + elx * Y::UE + v * Y::UV + (odd ? line * N1 : line);
             R acc = R(0);
 #pragma unroll
-            for (int m = 0; m < N1; ++m) acc += gw[m] * Cb[v * Y::UV + (odd ? line * N1 + m : m * N1 + line)];
-            Jb[v] = acc;
-            uc[v] = R(0.5) * (F.own[v] + F.oth[v]);
-            jo[v] = uc[v] - F.own[v];
-            jn[v] = uc[v] - F.oth[v];
-            qx[v] = R(0.5) * ((F.gxo[v] + F.ax * jo[v]) + (F.gxn[v] + F.bx * jn[v]));
-            qy[v] = R(0.5) * ((F.gyo[v] + F.ay * jo[v]) + (F.gyn[v] + F.by * jn[v]));
-            UL[v] = right ? F.oth[v] : F.own[v];
-            UR[v] = right ? F.own[v] : F.oth[v];
-        }
+            for (int m = 0; m < N1; ++m) acc += gw[m] * Cb[odd ? m : m * N1];
+            return acc;
+        };
+        R own[NV], oth[NV], UL[NV], UR[NV], Fcb[NV];
+        face_traces(el2, k, f, L, own, oth);
         const R ef = a.edge_f[(int64_t)e2 * 4 + k];
+        const R en = inside ? a.edge_f[(int64_t)L.nbr * 4 + L.nbr_edge] : R(0);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const R d = sFI[Y::tr(el2, k, f, v)];
-            Fcb[v] = ef * (right ? -d : d);
-            Fvb[v] = -Fcb[v] * nx;
-            Gvb[v] = -Fcb[v] * ny;
+            UL[v] = right ? oth[v] : own[v];
+            UR[v] = right ? own[v] : oth[v];
+            Fcb[v] = ef * sFI[Y::tr(el2, k, f, v)];
+            if (inside) Fcb[v] -= en * sFI[Y::tr(nl, L.nbr_edge, oslot, v)];
+            if (right) Fcb[v] = -Fcb[v];
         }
         R ULb[NV] = {R(0), R(0), R(0), R(0)}, URb[NV] = {R(0), R(0), R(0), R(0)};
         riemann_by_kind_vjp(a.riemann, UL, UR, nx, ny, g, Fcb, ULb, URb);
+        asm volatile("" ::: "memory");  // the viscous part's loads stay behind the Riemann part (registers)
+        face_traces(el2, k, f, L, own, oth);
+        R uc[NV], qx[NV], qy[NV], ax, ay, bx, by, Fvb[NV], Gvb[NV];
+        face_gradient(el2, k, f, L, own, oth, uc, qx, qy, ax, ay, bx, by);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) { Fvb[v] = -Fcb[v] * nx; Gvb[v] = -Fcb[v] * ny; }
         R ucb[NV] = {R(0), R(0), R(0), R(0)}, qxb[NV] = {R(0), R(0), R(0), R(0)}, qyb[NV] = {R(0), R(0), R(0), R(0)};
         visc_flux_vjp(uc, qx, qy, g, mu, kappa, Fvb, Gvb, ucb, qxb, qyb);
         if (a.mub_partial) {
@@ -958,24 +1000,28 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
 #pragma unroll
             for (int v = 1; v < NV; ++v) musum += double(Fvb[v] * Fv[v] + Gvb[v] * Gv[v]);
         }
+        asm volatile("" ::: "memory");
         R nb[TW];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const R job = Jb[v] + R(0.5) * (F.ax * qxb[v] + F.ay * qyb[v]);
-            const R jnb = R(0.5) * (F.bx * qxb[v] + F.by * qyb[v]);
+            const R job = jump_cotangent(el2, k, f, v) + R(0.5) * (ax * qxb[v] + ay * qyb[v]);
+            const R jnb = (inside ? jump_cotangent(nl, L.nbr_edge, oslot, v) : R(0)) +
+                          R(0.5) * (bx * qxb[v] + by * qyb[v]);
             const R uct = ucb[v] + job + jnb;
             const R ownb = (right ? URb[v] : ULb[v]) + R(0.5) * uct - job;
             nb[v] = (right ? ULb[v] : URb[v]) + R(0.5) * uct - jnb;
             nb[NV + v] = R(0.5) * qxb[v];
             nb[2 * NV + v] = R(0.5) * qyb[v];
-            sAu[Y::tr(el2, k, f, v)] = ownb;
-            sAx[Y::tr(el2, k, f, v)] = R(0.5) * qxb[v];
-            sAy[Y::tr(el2, k, f, v)] = R(0.5) * qyb[v];
             if (inside) {
-                sNu[Y::tr(nl, L.nbr_edge, oslot, v)] = nb[v];
-                sNx[Y::tr(nl, L.nbr_edge, oslot, v)] = nb[NV + v];
-                sNy[Y::tr(nl, L.nbr_edge, oslot, v)] = nb[2 * NV + v];
+                const int s = Y::tr(nl, L.nbr_edge, oslot, v);
+                sFI[s] = nb[v];
+                sTGx[s] = nb[NV + v];
+                sTGy[s] = nb[2 * NV + v];
             }
+            const int s = Y::tr(el2, k, f, v);
+            sFI[s] = ownb;
+            sTGx[s] = nb[NV + v];
+            sTGy[s] = nb[2 * NV + v];
         }
         if (!inside) {
             R* dst = a.Tb_out + (((int64_t)L.nbr * 4 + L.nbr_edge) * FP + oslot) * TW;
@@ -989,25 +1035,18 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
     // ---- R5: transposed traces of U and grad U; the gradient's cotangent onto
     // the reference derivatives
     if (active) {
-        // a partner's slot is read only where the partner is in this tile
-        // (elsewhere it holds no value: selected, never multiplied by 0)
-        const bool in0 = sIn[el * 4 + 0], in1 = sIn[el * 4 + 1], in2 = sIn[el * 4 + 2], in3 = sIn[el * 4 + 3];
-        auto both_t = [&](const R* A, const R* N, int v) -> R {
-            const int s0 = Y::tr(el, 0, i, v), s1 = Y::tr(el, 1, j, v);
-            const int s2 = Y::tr(el, 2, P - i, v), s3 = Y::tr(el, 3, P - j, v);
-            return sLm[j] * (A[s0] + (in0 ? N[s0] : R(0))) + sLp[j] * (A[s2] + (in2 ? N[s2] : R(0))) +
-                   sLp[i] * (A[s1] + (in1 ? N[s1] : R(0))) + sLm[i] * (A[s3] + (in3 ? N[s3] : R(0)));
-        };
+        jx = a.Jinv[(int64_t)e * 4]; jy = a.Jinv[(int64_t)e * 4 + 1];
+        kx = a.Jinv[(int64_t)e * 4 + 2]; ky = a.Jinv[(int64_t)e * 4 + 3];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            qb[v] += double(both_t(sAu, sNu, v));
-            const R gbx = Qxb[v] + both_t(sAx, sNx, v), gby = Qyb[v] + both_t(sAy, sNy, v);
-            sW3[ub + v * Y::UV] = jx * gbx + jy * gby;
-            sGx[ub + v * Y::UV] = kx * gbx + ky * gby;
+            if constexpr (!INC) qb[v] = double(sW3[ub + v * Y::UV]);
+            qb[v] += double(trace_t(sFI, v));
+            const R gbx = trace_t(sTGx, v), gby = trace_t(sTGy, v);
+            sW1[ub + v * Y::UV] += jx * gbx + jy * gby;
+            sW2[ub + v * Y::UV] += kx * gbx + ky * gby;
         }
     }
     __syncthreads();
-
     if (a.mub_partial) {
         const double sm = block_reduce_n<OpSum, NTHR / 64>(musum, sRed);
         if (tid == 0) a.mub_partial[tile] += sm;  // summed over the launches since the seed
@@ -1017,12 +1056,7 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
     if (active) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const R* X = sW3 + el * Y::UE + v * Y::UV;
-            const R* H = sGx + el * Y::UE + v * Y::UV;
-            R acc = R(0);
-#pragma unroll
-            for (int m = 0; m < N1; ++m) acc += sD[m * N1 + i] * X[j * N1 + m] + sD[m * N1 + j] * H[m * N1 + i];
-            double out = qb[v] + double(acc);
+            double out = qb[v] + double(grad_t(v));
             if (MODE == MODE_STAGE1) out += a.U0b[v * PS + gi];
             a.Ub_out[v * PS + gi] = out;
         }
@@ -1030,7 +1064,7 @@ __device__ __forceinline__ void visc_vjp_body(const VjpArgs<R>& a, const OpTable
 }
 
 template <typename R, int P, int EPB, int MODE, int NTHR = visc_threads<P, EPB>()>
-__global__ __launch_bounds__(NTHR) void visc_vjp_kernel(const VjpArgs<R> a, const OpTables<R> ops,
+__global__ __launch_bounds__(NTHR, 2) void visc_vjp_kernel(const VjpArgs<R> a, const OpTables<R> ops,
                                                          const ViscParams vp) {
     visc_vjp_body<R, P, EPB, MODE, NTHR>(a, ops, vp, tile_of_block(a.xcd_groups));
 }
@@ -1039,7 +1073,7 @@ __global__ __launch_bounds__(NTHR) void visc_vjp_kernel(const VjpArgs<R> a, cons
 // launch: one work item (member, tile) per workgroup, each member with its own
 // arguments, operator tables and viscous parameters.
 template <typename R, int P, int EPB, int MODE, int NTHR = visc_threads<P, EPB>()>
-__global__ __launch_bounds__(NTHR) void batched_visc_vjp_kernel(const BatchVjpInst<R>* __restrict__ insts,
+__global__ __launch_bounds__(NTHR, 2) void batched_visc_vjp_kernel(const BatchVjpInst<R>* __restrict__ insts,
                                                                  const int2* __restrict__ items) {
     const int2 it = items[blockIdx.x];
     visc_vjp_body<R, P, EPB, MODE, NTHR>(insts[it.x].a, insts[it.x].ops, insts[it.x].vp, it.y);
