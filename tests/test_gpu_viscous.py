@@ -179,3 +179,20 @@ def test_viscous_rejects_unsupported_meshes():
     with pytest.raises(ZJError) as e:
         solver.Solver(t, compat="textbook", positivity=False, viscous=True)
     assert e.value.code == 4
+
+
+@pytest.mark.parametrize("n", [1, 3, 5])
+@pytest.mark.parametrize("p,precision", [(3, "fp64"), (4, "fp64"), (5, "fp64"), (4, "fp32bulk"), (5, "fp32bulk")])
+def test_viscous_step_tiles(p, precision, n):
+    """A step's increment where the traces take the state's place in the tile (FP64 P4, P5: tiles of 10 and 7) and
+    where they do not: part of a tile, a tile and a remainder.  The increment is some 1e-3 of the state, whose
+    rounding (1e-16 FP64) shows in it at 1e-13; FP32-bulk carries the residual's own FP32 error."""
+    say(f"case: viscous step, TGV {n}x{n} P{p} hllc/hu Re 100 {precision}")
+    s, tb, t = _pair(cases.tgv_mesh(n), p, "hllc", "hu", precision=precision)
+    U = _state(t, 20 + n)
+    s.set_state(U)
+    dt = 1e-3
+    s.rk3_step(dt)
+    r = rel(s.get_state() - U, tb.advance(U, dt, False) - U)
+    say(f"  rel L2 of the increment {r:.3e}")
+    assert r < (1e-12 if precision == "fp64" else 1e-5)

@@ -118,6 +118,15 @@ constexpr int visc_threads() {
     return r < BLOCK ? r : BLOCK;
 }
 
+// FP64 P4 and P5: 39 KB of LDS instead of 46, so four workgroups fit on a CU
+// and not three (256x256 P4, four steps with their set-up: 1664 -> 1510 us; a
+// 128x128 P5 stage 55.6 -> 52.9 us).  At P3 four would still not fit (41,312
+// of 40,960 bytes each), and FP32's count is set by its registers.
+template <typename R, int P>
+constexpr bool visc_traces_over_state() {
+    return std::is_same<R, double>::value && P >= 4;
+}
+
 // One tile's viscous stage (the workgroup's NTHR threads, the tile's elements).
 template <typename R, int P, int EPB, int MODE, int NTHR, class SM>
 __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<R>& ops, const ViscParams& vp,
@@ -143,7 +152,12 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
     // 23 instead of 30 KB at P4, 31 instead of 41 KB at P3, so more
     // workgroups fit on a CU).
     constexpr bool ALIAS = PRE && NF <= NTHR;
-    R* const sTr = sm.Tr();
+    // The traces in the state's place (each thread holds its face point's
+    // over the barrier; phase C reads the state again, from cache).
+    constexpr bool TRU = visc_traces_over_state<R, P>();
+    static_assert(!TRU || (ALIAS && Y::TE <= Y::UE), "the traces take the state's place");
+    R* sTr;
+    if constexpr (TRU) sTr = sU; else sTr = sm.Tr();
     R* sTGx = nullptr;
     R* sTGy = nullptr;
     if constexpr (PRE) { sTGx = sm.TGx(); sTGy = sm.TGy(); }
@@ -193,13 +207,20 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
             point_gradient<R, P>(sU + el * Y::UE + v * Y::UV, sD, i, j, jx, jy, kx, ky, sGx[ub + v * Y::UV],
                                  sGy[ub + v * Y::UV]);
     }
-    for (int t = tid; t < NF; t += NTHR) {
+    for (int t0 = 0; t0 < NF; t0 += NTHR) {
+        const int t = t0 + tid;
         const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        if (e0 + el2 < a.E) {
+        const bool item = t < NF && e0 + el2 < a.E;
+        R tu[NV];
+        if (item) {
             const TraceLine tl = trace_line<P>(k, f);
 #pragma unroll
-            for (int v = 0; v < NV; ++v)
-                sTr[Y::tr(el2, k, f, v)] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+            for (int v = 0; v < NV; ++v) tu[v] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+        }
+        if constexpr (TRU) __syncthreads();  // the state is read
+        if (item) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) sTr[Y::tr(el2, k, f, v)] = tu[v];
         }
     }
     __syncthreads();
@@ -320,11 +341,12 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
     __syncthreads();
 
     // ---- C: corrected gradient, viscous and inviscid fluxes at the points
+    double qs[NV] = {0.0, 0.0, 0.0, 0.0};
     if (active) {
         R Uq[NV], Qx[NV], Qy[NV], fx[NV], fy[NV], Fv[NV], Gv[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            Uq[v] = sU[ub + v * Y::UV];
+            if constexpr (TRU) { qs[v] = stage_input(v); Uq[v] = R(qs[v]); } else Uq[v] = sU[ub + v * Y::UV];
             const R cxi = sC[i] * sJ[Y::tr(el, 3, P - j, v)] + sC[N1 + i] * sJ[Y::tr(el, 1, j, v)];
             const R ceta = sC[j] * sJ[Y::tr(el, 0, i, v)] + sC[N1 + j] * sJ[Y::tr(el, 2, P - i, v)];
             Qx[v] = sGx[ub + v * Y::UV] + jx * cxi + kx * ceta;
@@ -379,7 +401,7 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
             const double dt = *a.dt_ptr;
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                const double q = stage_input(v);
+                const double q = TRU ? qs[v] : stage_input(v);
                 const double u0 = HAS_U0 ? a.U0[v * PS + gi] : 0.0;
                 double un;
                 if (MODE == MODE_STAGE1) un = q + dt * res[v];
@@ -433,7 +455,7 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
 }
 
 template <typename R, int P, int EPB, int MODE, int NTHR = visc_threads<P, EPB>()>
-__global__ __launch_bounds__(NTHR) void visc_stage_kernel(const StageArgs<R> a, const OpTables<R> ops,
+__global__ __launch_bounds__(NTHR, (visc_traces_over_state<R, P>() ? 4 : 1)) void visc_stage_kernel(const StageArgs<R> a, const OpTables<R> ops,
                                                           const ViscParams vp) {
     visc_body<R, P, EPB, MODE, NTHR>(a, ops, vp, tile_of_block(a.xcd_groups), threadIdx.x, ViscSmem<R, P, EPB>{});
 }
