@@ -207,20 +207,29 @@ __device__ __forceinline__ void visc_body(const StageArgs<R>& a, const OpTables<
             point_gradient<R, P>(sU + el * Y::UE + v * Y::UV, sD, i, j, jx, jy, kx, ky, sGx[ub + v * Y::UV],
                                  sGy[ub + v * Y::UV]);
     }
-    for (int t0 = 0; t0 < NF; t0 += NTHR) {
-        const int t = t0 + tid;
-        const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
-        const bool item = t < NF && e0 + el2 < a.E;
+    if constexpr (TRU) {
+        const int el2 = tid / (4 * FP), r = tid - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+        const bool item = tid < NF && e0 + el2 < a.E;
         R tu[NV];
         if (item) {
             const TraceLine tl = trace_line<P>(k, f);
 #pragma unroll
             for (int v = 0; v < NV; ++v) tu[v] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
         }
-        if constexpr (TRU) __syncthreads();  // the state is read
+        __syncthreads();  // the state is read
         if (item) {
 #pragma unroll
             for (int v = 0; v < NV; ++v) sTr[Y::tr(el2, k, f, v)] = tu[v];
+        }
+    } else {
+        for (int t = tid; t < NF; t += NTHR) {
+            const int el2 = t / (4 * FP), r = t - el2 * (4 * FP), k = r / FP, f = r - k * FP;
+            if (e0 + el2 < a.E) {
+                const TraceLine tl = trace_line<P>(k, f);
+#pragma unroll
+                for (int v = 0; v < NV; ++v)
+                    sTr[Y::tr(el2, k, f, v)] = trace_point<R, P>(sU + el2 * Y::UE + v * Y::UV, tl, sLm, sLp);
+            }
         }
     }
     __syncthreads();
