@@ -14,7 +14,7 @@ from oracle import tri_oracle as T
 from tests.test_gpu_parity import rel, say
 from tests.test_gpu_tri_viscous import _pair, _state
 from zhijian_amd import cases
-from zhijian_amd.tri import TriSolver
+from zhijian_amd.tri import TriSolver, sp_coords, tri_faces
 
 pytestmark = pytest.mark.gpu
 
@@ -75,6 +75,98 @@ def test_tri_form_by_size(p, n, viscous, precision):
     r = rel(s.residual(), o.residual(U))
     say(f"  rel L2 {r:.3e}, tiles of {s.info()['elems_per_block']}")
     assert r < BAR[precision]
+
+
+@pytest.mark.parametrize("p,n,viscous,precision,corr", [
+    (1, 111, False, "fp64", "ga"), (1, 111, False, "fp32bulk", "hu"), (2, 182, False, "fp64", "sd"),
+    (2, 182, False, "fp32bulk", "ga"), (1, 111, True, "fp64", "hu"), (1, 111, True, "fp32bulk", "ga"),
+    (2, 128, True, "fp32bulk", "dg"), (2, 128, True, "fp64", "sd")])
+def test_tri_large_low_order_steps(p, n, viscous, precision, corr):
+    """Two steps of meshes above those counts: the stage updates, and the traces across tiles that each stage leaves
+    for the next and the first step for the second (set_state forms them only once)."""
+    say(f"case: triangle steps {'viscous' if viscous else 'inviscid'}, {2 * n * n} elements P{p} {precision} hllc/{corr}")
+    m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
+    kw = dict(viscous=True, Re=100.0) if viscous else {}
+    s = TriSolver(m.xy, m.tris, p, periodic=(1.0, 1.0), riemann="hllc", precision=precision, corr=corr, **kw)
+    o = T.TriTextbook(p, m.xy, m.tris, s.faces, s.normals, riemann="hllc", corr=corr)
+    if viscous:
+        o.set_viscous(100.0)
+    U = _state(m, p, n)
+    s.set_state(U)
+    dt = 0.5 * s.dt_cfl(0.5)
+    s.rk3_step(dt)
+    s.rk3_step(dt)
+    r = rel(s.get_state() - U, o.advance(o.advance(U, dt), dt) - U)
+    l2 = abs(s.residual_l2() - np.linalg.norm(s.residual())) / s.residual_l2()
+    say(f"  rel L2 of the increment {r:.3e}, tiles of {s.info()['elems_per_block']}")
+    assert r < BAR[precision]
+    assert l2 < 0.1  # stage 3's residual, a few per cent of a step away from the new state's
+
+
+@pytest.mark.parametrize("p,precision", [(1, "fp64"), (1, "fp32bulk"), (2, "fp64")])
+def test_tri_large_low_order_boundaries(p, precision):
+    """The same with boundary faces (far field, outflow, slip wall and no-slip wall, one type per side)."""
+    n = 111 if p == 1 else 182
+    say(f"case: triangle steps, open mesh, {2 * n * n} elements P{p} {precision} roe")
+    m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
+    faces, nrm = tri_faces(m.xy, m.tris)
+    side = np.where(np.abs(nrm[:, 0]) > 0.5, np.where(nrm[:, 0] > 0, 6, 4), np.where(nrm[:, 1] > 0, 1, 2))
+    bt = np.where(faces[:, 2] < 0, side, 0).astype(np.int32)
+    bmap = np.where(bt == 6, 1, 0).astype(np.int32)
+    bcd = np.array([[1.1, 0.3, 0.1, 2e3, 0, 0, 0, 0], [2e3, 0, 0, 0, 0, 0, 0, 0]], np.float64)
+    s = TriSolver(m.xy, m.tris, p, faces=faces, normals=nrm, bc_type=bt, bc_face_map=bmap, bc_data=bcd, riemann="roe",
+                  precision=precision)
+    o = T.TriTextbook(p, m.xy, m.tris, faces, nrm, riemann="roe", bc_type=bt, bc_face_map=bmap, bc_data=bcd)
+    shp = sp_coords(m.xy, m.tris, p).shape[:2]
+    U = cases.perturb(cases.prim_to_cons(np.full(shp, 1.0), np.full(shp, 0.3), np.full(shp, -0.1), np.full(shp, 2e3), 1.4),
+                      0.05, 4).reshape(-1)
+    s.set_state(U)
+    dt = 0.5 * s.dt_cfl(0.5)
+    s.rk3_step(dt)
+    s.rk3_step(dt)
+    r = rel(s.get_state() - U, o.advance(o.advance(U, dt), dt) - U)
+    say(f"  rel L2 of the increment {r:.3e}")
+    assert r < BAR[precision]
+
+
+@pytest.mark.parametrize("p,n,precision", [(1, 111, "fp64"), (1, 100, "fp32bulk"), (1, 111, "fp32bulk"), (1, 160, "fp32bulk"),
+                                           (2, 100, "fp32bulk"), (2, 128, "fp32bulk")])
+def test_tri_large_low_order_viscous_vjp(p, n, precision):
+    """The adjoint of meshes around those counts, where the stage's tiles and the adjoint's may differ: two steps
+    backwards with dJ/d(dt) (a step's edge cotangents are the next one's input), and the residual's VJP, as
+    test_tri_viscous_vjp_tiles has them.  Rounding is independent of g: in a product with a random g over N >= 240,000
+    values, divided by the factors' norms, an error of 6e-8 (FP32) over some tens of terms a value enters at
+    1e-6 / sqrt(N) = 2e-9, and the difference quotient's 1e-8 at 2e-11."""
+    say(f"case: triangle viscous VJP, {2 * n * n} elements P{p} {precision} roe/hu")
+    s, o, m = _pair(n, p, "roe", "hu", precision=precision, seed=n)
+    U = _state(m, p, 3 + n)
+    s.set_state(U)
+    dt, eps = 0.25 * s.dt_cfl(0.5), 1e-5
+    rng = np.random.default_rng(n)
+    g, v = rng.standard_normal(U.size), rng.standard_normal(U.size) * U
+    bar = 1e-10 if precision == "fp64" else 1e-8
+    scale = np.linalg.norm(g) * np.linalg.norm(v)
+    want = float(g @ (o.residual(U + eps * v) - o.residual(U - eps * v))) / (2 * eps)
+    scale_r = np.linalg.norm(g) * np.linalg.norm(o.residual(U + eps * v) - o.residual(U - eps * v)) / (2 * eps)
+    rr = abs(float(s.residual_vjp(g) @ v) - want) / scale_r
+    U1 = o.advance(U, dt)
+    s.set_state(U1)
+    s.adjoint_set(g)
+    dtb = s.rk3_step_vjp(dt)
+    s.set_state(U)
+    s.rk3_step_vjp(dt, want_dt=False)
+    got = float(s.adjoint_get() @ v)
+
+    def two(X):
+        return o.advance(o.advance(X, dt), dt)
+
+    want = float(g @ (two(U + eps * v) - two(U - eps * v))) / (2 * eps)
+    h = 1e-4 * dt
+    want_dt = float(g @ (o.advance(U1, dt + h) - o.advance(U1, dt - h))) / (2 * h)
+    scale_dt = np.linalg.norm(g) * np.linalg.norm(o.residual(U1))
+    r, rd = abs(got - want) / scale, abs(dtb - want_dt) / scale_dt
+    say(f"  residual {rr:.3e}, two steps {r:.3e}, time step {rd:.3e}")
+    assert rr < bar and r < bar and rd < bar
 
 
 @pytest.mark.parametrize("n", [1, 4, 5])
