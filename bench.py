@@ -378,8 +378,8 @@ def tri_alg_bytes_per_stage(E, p, stage, precision, cross_edges, viscous=False):
     """Algorithmic HBM bytes of one triangle stage launch: the FP64 stage state
     per solution point (stage 1 reads U^n and writes U1; stages 2 and 3 read
     U^n and the intermediate state and write one), 10 geometry words per
-    element (affine metric, three face normals; the kernels' 16 also hold the
-    edges' scale factors, which these determine), 3 int2 links, and the
+    element (affine metric, three face normals; the matrix-core kernels' 6
+    edge factors, which these determine, are not counted), 3 int2 links, and the
     (p+1) x 4 trace of every element edge whose neighbour lies in another tile,
     written once and read once in the compute precision (with the
     Navier-Stokes terms (p+1) x 12: U, dU/dx, dU/dy)."""

@@ -36,9 +36,11 @@
 //            only edges whose neighbour lies in another tile of 64 elements are
 //            written (a neighbour in the same tile is read from LDS), rotating
 //            as the quadrilateral path's: stage 1 T0->T1, 2 T1->T2, 3 T2->T0
-//   geo      [E][16]: r_x, r_y, s_x, s_y, then the face normal (as the face's
-//            left element sees it) of edges 0, 1, 2, |e|/(2J) of each edge and
-//            of the neighbour's side of each (0 on a boundary)
+//   geo      [E][10]: r_x, r_y, s_x, s_y, then the face normal (as the face's
+//            left element sees it) of edges 0, 1, 2
+//   edge     [E][6]: |e|/(2J) of each edge and of the neighbour's side of each
+//            (0 on a boundary), for the matrix-core kernels; apart from geo,
+//            whose words the others read alone
 //   links    [E][3] int2: x = neighbour element (-1 on a boundary), y = packed
 //            neighbour edge (or BC type) | role << 3 | BC data index << 6
 //   ops      constant memory, per order: Dr, Ds [Np][Np], interp [3(p+1)][Np],
@@ -76,8 +78,8 @@ struct TriShape {
 
 constexpr int TILE = BLOCK / NV;  // elements per workgroup (one lane per element and variable)
 constexpr int EB = 16;            // elements per block of the state and trace layouts
-constexpr int GEO = 16;           // geometry words per element
-constexpr int GEO_S = 10, GEO_SN = 13;  // edge factors within them: own, the neighbour's
+constexpr int GEO = 10;           // geometry words per element
+constexpr int EDG = 6;            // edge factors per element: own, then the neighbour's
 
 // Operator tables of order P in constant memory, laid out for wide scalar
 // loads in the kernels' loops:
@@ -190,6 +192,7 @@ struct TriArgs {
     double* U_out;        // stage output (may alias U_in or U0 lane-locally)
     double* R_out;        // residual (MODE_RESIDUAL)
     const R* geo;
+    const R* edge;
     const int2* links;
     const R* T_in;
     R* T_out;
@@ -515,7 +518,7 @@ __global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) voi
         const int nl = Lk.x - e0, ek = link_edge(Lk.y), role = link_role(Lk.y);
         const bool right = role == ROLE_RIGHT, live = e0 + el < a.E, bnd = role == ROLE_BOUNDARY;
         const bool in = !bnd && nl >= 0 && nl < TT;
-        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R ns[4] = {nx, ny, right ? -s : s, right ? sn : -sn};
         store4(sNs + 4 * tid, ns);
         const bool self = !live || !in;
@@ -524,8 +527,8 @@ __global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) voi
         owned = live && !(right && in);
     }
     if (tid < TT) {
-        R w[4];
-        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        const R* Ge = a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO;
+        const R w[4] = {Ge[0], Ge[1], Ge[2], Ge[3]};
         store4(sGeo + 4 * tid, w);
     }
     const unsigned long long own_mask = __ballot(owned);
@@ -810,7 +813,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
         const int nl = Lk.x - e0, ek = link_edge(Lk.y);
         const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
         const bool in = !live || (nl >= 0 && nl < TT);  // beyond the mesh: its own neighbour
-        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
         const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, right ? sn : -sn};
         store4(sEw + 4 * tid, we);
@@ -821,8 +824,8 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
         owned = live && !(right && in);
     }
     if (tid < TT) {
-        R w[4];
-        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        const R* Ge = a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO;
+        const R w[4] = {Ge[0], Ge[1], Ge[2], Ge[3]};
         store4(sGeo + 4 * tid, w);
     }
     const unsigned long long own_mask = __ballot(owned);
@@ -1571,6 +1574,7 @@ struct TriVjpArgs {
     const double* U_in;     // q
     const double* U0;       // U^n (stages 2, 3)
     const R* geo;
+    const R* edge;
     const int2* links;
     const R* T_in;          // traces of q on edges read across tiles
     const double* bc_data;
@@ -2052,7 +2056,7 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
         const int nl = Lk.x - e0, ek = link_edge(Lk.y);
         const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
         const bool in = !live || (nl >= 0 && nl < TT);
-        const R s = Ge[GEO_S + k], sn = Ge[GEO_SN + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
         const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, in ? (right ? sn : -sn) : R(0)};
         store4(sEw + 4 * tid, we);
@@ -2063,8 +2067,8 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
         owned = live && !(right && in);
     }
     if (tid < TT) {
-        R w[4];
-        load4(a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO, w);
+        const R* Ge = a.geo + (int64_t)min(e0 + tid, a.E - 1) * GEO;
+        const R w[4] = {Ge[0], Ge[1], Ge[2], Ge[3]};
         store4(sGeo + 4 * tid, w);
     }
     const unsigned long long own_mask = __ballot(owned);
@@ -2892,6 +2896,7 @@ struct zj_tri {
     double* Rres = nullptr;
     double* aos = nullptr;
     void* geo = nullptr;
+    void* edge = nullptr;
     int2* links = nullptr;
     void* T[3] = {nullptr, nullptr, nullptr};
     double* bc_data = nullptr;
@@ -2960,7 +2965,7 @@ static int tupload_as(zj_tri* h, void** dst, const std::vector<double>& v) {
 static void trelease(zj_tri* h) {
     if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
     if (h->graph) (void)hipGraphDestroy(h->graph);
-    void* bufs[] = {h->U, h->W, h->Rres, h->aos, h->geo, h->links, h->T[0], h->T[1], h->T[2],
+    void* bufs[] = {h->U, h->W, h->Rres, h->aos, h->geo, h->edge, h->links, h->T[0], h->T[1], h->T[2],
                     h->bc_data, h->hcell, h->d_scalars, h->partial, h->partial_dt, h->perm,
                     h->A_Ub, h->A_U0b, h->A_W1, h->A_W2, h->A_dtb, h->A_T[0], h->A_T[1], h->A_T[2],
                     h->A_Tb[0], h->A_Tb[1]};
@@ -3037,14 +3042,15 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
     auto dev = [&](int old) { return inv[(size_t)old]; };
 
     std::vector<int2> links((size_t)E * 3, make_int2(-1, -1));
-    std::vector<double> geo((size_t)E * GEO, 0.0);
+    std::vector<double> geo((size_t)E * GEO, 0.0), edge((size_t)E * EDG, 0.0);
     for (int e = 0; e < E; ++e) {
         const int o = perm.empty() ? e : perm[(size_t)e];
         double* ge = &geo[(size_t)e * GEO];
         for (int c = 0; c < 4; ++c) ge[c] = met[(size_t)o * 4 + c];
-        ge[GEO_S] = std::sqrt(ge[2] * ge[2] + ge[3] * ge[3]);
-        ge[GEO_S + 1] = std::sqrt((ge[0] + ge[2]) * (ge[0] + ge[2]) + (ge[1] + ge[3]) * (ge[1] + ge[3]));
-        ge[GEO_S + 2] = std::sqrt(ge[0] * ge[0] + ge[1] * ge[1]);
+        double* ed = &edge[(size_t)e * EDG];
+        ed[0] = std::sqrt(ge[2] * ge[2] + ge[3] * ge[3]);
+        ed[1] = std::sqrt((ge[0] + ge[2]) * (ge[0] + ge[2]) + (ge[1] + ge[3]) * (ge[1] + ge[3]));
+        ed[2] = std::sqrt(ge[0] * ge[0] + ge[1] * ge[1]);
     }
     std::vector<double> hcd((size_t)E);
     for (int e = 0; e < E; ++e) hcd[(size_t)e] = hc[(size_t)(perm.empty() ? e : perm[(size_t)e])];
@@ -3087,7 +3093,7 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
     for (size_t k = 0; k < links.size(); ++k) {
         if (links[k].y == -1) return tfail(h, ZJ_ERR_ARG, "an element edge has no face");
         if (links[k].x >= 0)
-            geo[k / 3 * GEO + GEO_SN + k % 3] = geo[(size_t)links[k].x * GEO + GEO_S + (links[k].y & 7)];
+            edge[k / 3 * EDG + 3 + k % 3] = edge[(size_t)links[k].x * EDG + (links[k].y & 7)];
     }
 
     ZJ_THIP(h, hipSetDevice(h->device));
@@ -3106,9 +3112,9 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
     for (int k = 0; k < 3; ++k) ZJ_THIP(h, hipMalloc(&h->T[k], eb * NFP * (h->viscous ? TWV : 4) * rsz));
     int rc;
     if (h->prec == ZJ_PREC_FP64) {
-        if ((rc = tupload_as<double>(h, &h->geo, geo))) return rc;
+        if ((rc = tupload_as<double>(h, &h->geo, geo)) || (rc = tupload_as<double>(h, &h->edge, edge))) return rc;
     } else {
-        if ((rc = tupload_as<float>(h, &h->geo, geo))) return rc;
+        if ((rc = tupload_as<float>(h, &h->geo, geo)) || (rc = tupload_as<float>(h, &h->edge, edge))) return rc;
     }
     if ((rc = tupload(h, (void**)&h->links, links))) return rc;
     std::vector<double> bcd;
@@ -3131,6 +3137,7 @@ static TriArgs<R> tri_args(zj_tri* h, int mode) {
     TriArgs<R> a{};
     a.E = h->E;
     a.geo = (const R*)h->geo;
+    a.edge = (const R*)h->edge;
     a.links = h->links;
     a.bc_data = h->bc_data;
     a.dt_ptr = h->d_scalars;
@@ -3416,6 +3423,7 @@ static TriVjpArgs<R> tvjp_args(zj_tri* h) {
     TriVjpArgs<R> a{};
     a.E = h->E;
     a.geo = (const R*)h->geo;
+    a.edge = (const R*)h->edge;
     a.links = h->links;
     a.bc_data = h->bc_data;
     a.dt_ptr = h->d_scalars;
