@@ -22,7 +22,8 @@ BAR = {"fp64": 1e-12, "fp32bulk": 1e-5}
 
 
 @pytest.mark.parametrize("n", [1, 4, 5, 9])
-@pytest.mark.parametrize("p,precision", [(2, "fp64"), (3, "fp64"), (5, "fp64"), (3, "fp32bulk"), (4, "fp32bulk"), (5, "fp32bulk")])
+@pytest.mark.parametrize("p,precision", [(1, "fp64"), (2, "fp64"), (3, "fp64"), (5, "fp64"), (1, "fp32bulk"), (2, "fp32bulk"),
+                                         (3, "fp32bulk"), (4, "fp32bulk"), (5, "fp32bulk")])
 def test_tri_viscous_tiles(p, precision, n):
     corr = {1: "dg", 4: "ga", 5: "hu", 9: "sd"}[n]
     say(f"case: triangle viscous stage, {2 * n * n} elements P{p} {precision} roe/{corr}")

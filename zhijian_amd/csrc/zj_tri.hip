@@ -1523,31 +1523,76 @@ __global__ __launch_bounds__(TT * NV) void tri_visc_scalar_kernel(TriArgs<R> a) 
     }
 }
 
-// Traces of U and grad U on every edge (after a new state is set): one wave
-// per four elements.
+// The traces of a new state, below: waves of G groups of four elements, four
+// waves a workgroup.
+constexpr int TRACE_G = 2, TRACE_TILE = BLOCK / 64 * 4 * TRACE_G;
+
+// Traces of U and grad U on every edge (after a new state is set).  Bound by
+// writing them: 1.1 KB an element at P3 FP64 against 0.3 read.  The operator
+// tables are read into LDS once for 32 elements, and a group's rows leave
+// through LDS in whole lines; with the tables from memory and 32-byte pieces
+// stored from the products, set_state took, us, one lane per element and
+// variable with scalar operands / that / this, at 500,000 elements: P3 FP64
+// 312 / 350 / 214, P1 FP64 112 / 142 / 98, P5 FP64 544 / 638 / 424, P3 FP32
+// 245 / 220 / 158.
+// The bound of two waves per SIMD keeps the products' results out of the
+// accumulation registers: with some of them there, hipcc 7.2 merged their LDS
+// stores with the others' at wrong offsets (FP32).
 template <typename R, int P>
-__global__ __launch_bounds__(BLOCK) void tri_visc_trace_kernel(int E, const double* U, const R* geo, R* T_out) {
+__global__ __launch_bounds__(BLOCK, 2) void tri_visc_trace_kernel(int E, const double* U, const R* geo, R* T_out) {
     using FO = tri::FragOps<R, P>;
-    constexpr int NP = FO::NP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB;
-    const R* const ops = frag_ops<R>() + tri::frag_offset<R>(P);
-    const int lane = threadIdx.x & 63, row = lane >> 4, v = lane & 3;
-    const int e = (blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * 4 + ((lane >> 2) & 3);
-    const bool live = e < E;
-    R u[1][PB], t[1][FB], tg[1][2 * FB];
+    constexpr int NP = FO::NP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB, G = TRACE_G;
+    __shared__ R ops[FO::F - FO::I];  // the operator tables I, G
+    __shared__ R sOut[BLOCK / 64 * 4 * NFP * TWV];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4, v = lane & 3;
+    const int e0 = blockIdx.x * TRACE_TILE;
+    auto elg = [&](int q) { return e0 + (wave * G + q) * 4 + ((lane >> 2) & 3); };
+    const PointRows<NP, G> rows(e0, wave, lane, E);
+    double u0[G][PB];
+    R ge[G][4];
 #pragma unroll
-    for (int b = 0; b < PB; ++b) u[0][b] = live && 4 * b + row < NP ? R(U[blk(e, 4 * b + row, NP) + v]) : R(0);
-    tri::frag_mma<true, R, 1, FB, PB>(ops + FO::I, u, t);
-    tri::frag_mma<true, R, 1, 2 * FB, PB>(ops + FO::G, u, tg);
-    if (!live) return;
-    const R* Ge = geo + (int64_t)e * GEO;
-    const R rx = Ge[0], ry = Ge[1], sx = Ge[2], sy = Ge[3];
+    for (int q = 0; q < G; ++q) {
 #pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        if (4 * b + row >= NFP) continue;
-        R* T = T_out + ((int64_t)e * NFP + 4 * b + row) * TWV + v;
-        T[0] = t[0][b];
-        T[NV] = rx * tg[0][b] + sx * tg[0][FB + b];
-        T[2 * NV] = ry * tg[0][b] + sy * tg[0][FB + b];
+        for (int b = 0; b < PB; ++b) u0[q][b] = *rows.at(U, q, b);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) ge[q][c] = geo[(int64_t)min(elg(q), E - 1) * GEO + c];
+    }
+    {
+        const R* const src = frag_ops<R>() + tri::frag_offset<R>(P) + FO::I;
+        for (int t = 4 * threadIdx.x; t < FO::F - FO::I; t += 4 * BLOCK) {
+            R w[4];
+            load4(src + t, w);
+            store4(ops + t, w);
+        }
+    }
+    R u[G][PB], tu[G][FB], tg[G][2 * FB];
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) u[q][b] = 4 * b + row < NP ? R(u0[q][b]) : R(0);
+    __syncthreads();
+    tri::frag_mma<true, R, G, FB, PB>(ops, u, tu);
+    tri::frag_mma<true, R, G, 2 * FB, PB>(ops + (FO::G - FO::I), u, tg);
+    // a group's rows are one run of memory: through LDS, so that a store's lanes write whole lines of it
+    R* const out = sOut + wave * (4 * NFP * TWV);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+        const int first = e0 + (wave * G + q) * 4;
+        tri::wave_lds_fence();
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            if (4 * b + row >= NFP) continue;
+            R* T = out + (((lane >> 2) & 3) * NFP + 4 * b + row) * TWV + v;
+            T[0] = tu[q][b];
+            T[NV] = ge[q][0] * tg[q][b] + ge[q][2] * tg[q][FB + b];
+            T[2 * NV] = ge[q][1] * tg[q][b] + ge[q][3] * tg[q][FB + b];
+        }
+        tri::wave_lds_fence();
+        const int n = min(4, E - first) * NFP * TWV;  // words; none beyond the mesh
+        using V = typename std::conditional<sizeof(R) == 8, double2, float4>::type;  // one lane's 16 bytes
+        constexpr int W = sizeof(V) / sizeof(R);
+        for (int t = W * lane; t < n; t += W * 64)
+            *reinterpret_cast<V*>(T_out + (int64_t)first * NFP * TWV + t) = *reinterpret_cast<const V*>(out + t);
     }
 }
 
@@ -2640,8 +2685,7 @@ hipError_t tri_visc_launch(int P, int mode, const TriArgs<R>& a, hipStream_t s) 
 
 template <typename R>
 hipError_t tri_visc_trace(int P, int E, const double* U, const R* geo, R* T, hipStream_t s) {
-    constexpr int PER = BLOCK / 64 * 4;  // elements per workgroup
-    const int grid = (std::max(E, 1) + PER - 1) / PER;
+    const int grid = (std::max(E, 1) + TRACE_TILE - 1) / TRACE_TILE;
     switch (P) {
     case 1: tri_visc_trace_kernel<R, 1><<<grid, BLOCK, 0, s>>>(E, U, geo, T); break;
     case 2: tri_visc_trace_kernel<R, 2><<<grid, BLOCK, 0, s>>>(E, U, geo, T); break;
