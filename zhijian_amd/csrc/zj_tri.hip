@@ -1523,8 +1523,8 @@ __global__ __launch_bounds__(TT * NV) void tri_visc_scalar_kernel(TriArgs<R> a) 
     }
 }
 
-// The traces of a new state, below: waves of G groups of four elements, four
-// waves a workgroup.
+// The traces of a new state and the completion of a cotangent, below: waves of
+// G groups of four elements, four waves a workgroup.
 constexpr int TRACE_G = 2, TRACE_TILE = BLOCK / 64 * 4 * TRACE_G;
 
 // Traces of U and grad U on every edge (after a new state is set).  Bound by
@@ -2506,7 +2506,14 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
 // Completion of a cotangent with the Navier-Stokes terms: U_bar plus the
 // transposed traces of U and of its gradient for the cross-tile edge
 // cotangents (12 words per point) that the last adjoint launch left (tiles of
-// TT elements).  One wave per four elements.
+// TT elements).  Without any (Tb null) a copy.  Every load that does not hang
+// on another goes out first, and 32 elements share the tables in LDS: with
+// tables and links read where they are used, and for the copy too,
+// adjoint_get_device of 500,000 elements at P3 FP64 with cotangents pending
+// took 295 us, this 178, one lane per element and variable 183; at P5 FP32
+// 348, 298 and 336.  At P1 and P2, where a wave has little to share, the form
+// below is the quicker: 500,000 elements FP64, this / that, P1 78 / 67, P2
+// 133 / 126, and 33,800 elements P2 FP32 12.8 / 11.9.
 template <typename R, int P, int TT>
 __global__ __launch_bounds__(BLOCK) void tri_visc_complete_kernel(int E, const int2* __restrict__ links,
                                                                   const R* __restrict__ geo,
@@ -2514,35 +2521,122 @@ __global__ __launch_bounds__(BLOCK) void tri_visc_complete_kernel(int E, const i
                                                                   const R* __restrict__ Tb,
                                                                   double* __restrict__ out) {
     using FO = tri::FragOps<R, P>;
-    constexpr int NP = FO::NP, FP = FO::FP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB;
-    const R* const ops = frag_ops<R>() + tri::frag_offset<R>(P) + FO::ADJ0;
-    const int lane = threadIdx.x & 63, row = lane >> 4, v = lane & 3;
-    const int e = (blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * 4 + ((lane >> 2) & 3), ec = min(e, E - 1);
-    R f[1][3 * FB], acc[1][PB];
-    const R* Ge = geo + (int64_t)ec * GEO;
-    const R rx = Ge[0], ry = Ge[1], sx = Ge[2], sy = Ge[3];
+    constexpr int NP = FO::NP, FP = FO::FP, NFP = FO::NFP, PB = FO::PB, FB = FO::FB, G = TRACE_G;
+    __shared__ R ops[FO::DT - FO::GT];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4, v = lane & 3;
+    const int e0 = blockIdx.x * TRACE_TILE;
+    auto elg = [&](int q) { return e0 + (wave * G + q) * 4 + ((lane >> 2) & 3); };
+    const PointRows<NP, G> rows(e0, wave, lane, E);
+    double o[G][PB];
 #pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        const int j = 4 * b + row;
-        f[0][b] = f[0][FB + b] = f[0][2 * FB + b] = R(0);
-        if (Tb && j < NFP) {
-            const int n = links[(int64_t)ec * 3 + j / FP].x;
-            if (n / TT != ec / TT) {
-                const R* T = Tb + ((int64_t)ec * NFP + j) * TWV + v;
-                f[0][b] = T[0];
-                f[0][FB + b] = rx * T[NV] + ry * T[2 * NV];
-                f[0][2 * FB + b] = sx * T[NV] + sy * T[2 * NV];
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b) o[q][b] = *rows.at(Ub, q, b);
+    if (Tb) {
+        const R* const src = frag_ops<R>() + tri::frag_offset<R>(P) + FO::ADJ0 + FO::GT;
+        for (int t = 4 * threadIdx.x; t < FO::DT - FO::GT; t += 4 * BLOCK) {
+            R w[4];
+            load4(src + t, w);
+            store4(ops + t, w);
+        }
+        R f[G][3 * FB], acc[G][PB];
+        int n[G][3];
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) n[q][k] = links[(int64_t)min(elg(q), E - 1) * 3 + k].x;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int e = min(elg(q), E - 1);
+            const R* Ge = geo + (int64_t)e * GEO;
+            const R rx = Ge[0], ry = Ge[1], sx = Ge[2], sy = Ge[3];
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                // slots across tiles (the others read the first row in common)
+                const int j = 4 * b + row, k = min(j, NFP - 1) / FP;
+                const bool on = j < NFP && (k == 0 ? n[q][0] : (k == 1 ? n[q][1] : n[q][2])) / TT != e / TT;
+                const R* T = Tb + (on ? (int64_t)e * NFP + j : (int64_t)0) * TWV + v;
+                const R tb = T[0], xb = T[NV], yb = T[2 * NV];
+                f[q][b] = on ? tb : R(0);
+                f[q][FB + b] = on ? rx * xb + ry * yb : R(0);
+                f[q][2 * FB + b] = on ? sx * xb + sy * yb : R(0);
             }
         }
-    }
-    tri::frag_mma<true, R, 1, PB, 3 * FB>(ops + FO::GT, f, acc);
-    if (e >= E) return;
+        __syncthreads();
+        tri::frag_mma<true, R, G, PB, 3 * FB>(ops, f, acc);
 #pragma unroll
-    for (int b = 0; b < PB; ++b)
-        if (4 * b + row < NP) {
-            const int64_t gi = blk(e, 4 * b + row, NP) + v;
-            out[gi] = Ub[gi] + double(acc[0][b]);
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int b = 0; b < PB; ++b) o[q][b] += double(acc[q][b]);
+    }
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int b = 0; b < PB; ++b)
+            if (4 * b + row < NP && elg(q) < E) *rows.at(out, q, b) = o[q][b];
+}
+
+// The same at P1 and P2, one lane per element and variable.
+template <typename R, int P, int TT>
+__global__ __launch_bounds__(TT * NV) void tri_visc_complete_scalar_kernel(int E, const int2* __restrict__ links,
+                                                                           const R* __restrict__ geo,
+                                                                           const double* __restrict__ Ub,
+                                                                           const R* __restrict__ Tb,
+                                                                           double* __restrict__ out, int xcd_groups) {
+    using S = TriShape<P>;
+    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
+    constexpr int O0 = ops_offset(P), CA = TriOps<P>::CA, OI = O0 + TriOps<P>::C;
+    const int tid = threadIdx.x, el = tid >> 2, v = tid & 3;
+    const int e0 = tile_of_block(xcd_groups) * TT, e = e0 + el;
+    if (e >= E) return;
+    const int64_t base = blk(e, 0, NP) + v;
+    double acc[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) acc[i] = Ub[base + (int64_t)i * EB * NV];
+    if (Tb) {
+        R tu[NFP], tx[NFP], ty[NFP];
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk) {
+            const int2 Lk = links[(int64_t)e * 3 + kk];
+            const int nl = Lk.x - e0;
+            const bool cross = !(nl >= 0 && nl < TT);
+#pragma unroll
+            for (int f = 0; f < FP; ++f) {
+                const int j = kk * FP + f;
+                const R* T = Tb + ((int64_t)e * NFP + j) * TWV;
+                tu[j] = cross ? T[v] : R(0);
+                tx[j] = cross ? T[NV + v] : R(0);
+                ty[j] = cross ? T[2 * NV + v] : R(0);
+            }
         }
+        const R* G = geo + (int64_t)e * GEO;
+        const R rx = G[0], ry = G[1], sx = G[2], sy = G[3];
+        R grb[NP], gsb[NP];
+#pragma unroll
+        for (int m = 0; m < NP; ++m) {
+            R su = R(0), qx = R(0), qy = R(0);
+#pragma unroll
+            for (int j = 0; j < NFP; ++j) {
+                const R w = cop<R>(OI + j * NP + m);
+                su = fmaR(w, tu[j], su);
+                qx = fmaR(w, tx[j], qx);
+                qy = fmaR(w, ty[j], qy);
+            }
+            acc[m] += double(su);
+            grb[m] = rx * qx + ry * qy;
+            gsb[m] = sx * qx + sy * qy;
+        }
+#pragma unroll
+        for (int m = 0; m < NP; ++m) {
+            R s = R(0);
+#pragma unroll
+            for (int i = 0; i < NP; ++i)
+                s = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], s));
+            acc[m] += double(s);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) out[base + (int64_t)i * EB * NV] = acc[i];
 }
 
 // Traces of U on every edge (after a new state is set).
@@ -2795,22 +2889,24 @@ hipError_t tri_visc_vjp(int P, int mode, const TriVjpArgs<R>& a, hipStream_t s) 
 
 template <typename R, int P>
 hipError_t tri_visc_complete_p(int E, const int2* links, const R* geo, const double* Ub, const R* Tb, double* out,
-                               hipStream_t s) {
-    constexpr int PER = BLOCK / 64 * 4;  // elements per workgroup
-    tri_visc_complete_kernel<R, P, TriViscVjpTile<R, P>::value>
-        <<<(std::max(E, 1) + PER - 1) / PER, BLOCK, 0, s>>>(E, links, geo, Ub, Tb, out);
+                               int xcd, hipStream_t s) {
+    constexpr int TT = TriViscVjpTile<R, P>::value;
+    if constexpr (P <= 2)
+        tri_visc_complete_scalar_kernel<R, P, TT><<<(std::max(E, 1) + TT - 1) / TT, TT * NV, 0, s>>>(E, links, geo, Ub, Tb, out, xcd);
+    else
+        tri_visc_complete_kernel<R, P, TT><<<(std::max(E, 1) + TRACE_TILE - 1) / TRACE_TILE, BLOCK, 0, s>>>(E, links, geo, Ub, Tb, out);
     return hipGetLastError();
 }
 
 template <typename R>
 hipError_t tri_visc_complete(int P, int E, const int2* links, const R* geo, const double* Ub, const R* Tb, double* out,
-                             hipStream_t s) {
+                             int xcd, hipStream_t s) {
     switch (P) {
-    case 1: return tri_visc_complete_p<R, 1>(E, links, geo, Ub, Tb, out, s);
-    case 2: return tri_visc_complete_p<R, 2>(E, links, geo, Ub, Tb, out, s);
-    case 3: return tri_visc_complete_p<R, 3>(E, links, geo, Ub, Tb, out, s);
-    case 4: return tri_visc_complete_p<R, 4>(E, links, geo, Ub, Tb, out, s);
-    default: return tri_visc_complete_p<R, 5>(E, links, geo, Ub, Tb, out, s);
+    case 1: return tri_visc_complete_p<R, 1>(E, links, geo, Ub, Tb, out, xcd, s);
+    case 2: return tri_visc_complete_p<R, 2>(E, links, geo, Ub, Tb, out, xcd, s);
+    case 3: return tri_visc_complete_p<R, 3>(E, links, geo, Ub, Tb, out, xcd, s);
+    case 4: return tri_visc_complete_p<R, 4>(E, links, geo, Ub, Tb, out, xcd, s);
+    default: return tri_visc_complete_p<R, 5>(E, links, geo, Ub, Tb, out, xcd, s);
     }
 }
 
@@ -3567,9 +3663,9 @@ extern "C" int zj_tri_adjoint_get_device(zj_tri_handle h, double* d_ubar_aos, vo
     if (h->viscous)
         e = h->prec == ZJ_PREC_FP64
                 ? tri_visc_complete<double>(h->P, h->E, h->links, (const double*)h->geo, h->A_Ub, (const double*)tb,
-                                            h->Rres, s)
+                                            h->Rres, h->xcd_groups, s)
                 : tri_visc_complete<float>(h->P, h->E, h->links, (const float*)h->geo, h->A_Ub, (const float*)tb,
-                                           h->Rres, s);
+                                           h->Rres, h->xcd_groups, s);
     else
         e = h->prec == ZJ_PREC_FP64
                 ? tri_complete<double>(h->P, h->E, h->links, h->A_Ub, (const double*)tb, h->Rres, h->xcd_groups, s)
@@ -3625,7 +3721,7 @@ static hipError_t tri_residual_vjp(zj_tri* h, hipStream_t s) {
     a.Tb_out = tb;
     if (h->viscous) {
         if ((e = tri_visc_vjp<R>(h->P, MODE_RESIDUAL, a, s)) != hipSuccess) return e;
-        return tri_visc_complete<R>(h->P, h->E, h->links, geo, h->Rres, tb, h->W, s);
+        return tri_visc_complete<R>(h->P, h->E, h->links, geo, h->Rres, tb, h->W, h->xcd_groups, s);
     }
     if ((e = tri_vjp<R>(h->P, MODE_RESIDUAL, a, s)) != hipSuccess) return e;
     return tri_complete<R>(h->P, h->E, h->links, h->Rres, tb, h->W, h->xcd_groups, s);
