@@ -171,7 +171,8 @@ def test_tri_large_low_order_viscous_vjp(p, n, precision):
 
 
 @pytest.mark.parametrize("n", [1, 4, 5])
-@pytest.mark.parametrize("p,precision", [(1, "fp64"), (2, "fp64"), (5, "fp64"), (2, "fp32bulk"), (4, "fp32bulk")])
+@pytest.mark.parametrize("p,precision", [(1, "fp64"), (2, "fp64"), (5, "fp64"), (1, "fp32bulk"), (2, "fp32bulk"),
+                                         (4, "fp32bulk")])
 def test_tri_viscous_vjp_tiles(p, precision, n):
     """One step backwards with dJ/d(dt) at the adjoint's tile edges (32 elements; 64 at P1, 16 at FP64 P5):
     <g, dU1/dU v> and <g, dU1/d(dt)> against central differences of the oracle's step.  The difference

@@ -1635,6 +1635,7 @@ struct TriVjpArgs {
     int xcd_groups;
     int lift_off;
     double mu, kappa, eta;  // Navier-Stokes terms (tri_visc_vjp_kernel)
+    int lf_off;
     int family;             // of the correction: DG, SD = GA, HU
     const double* R_in;     // residual at q, with dtb_partial (tri_visc_vjp_kernel)
 };
@@ -2023,7 +2024,12 @@ __global__ __launch_bounds__(BLOCK) void tri_complete_kernel(int E, const int2* 
 template <typename R, int P> struct TriViscVjpTile {
     static constexpr int NP = (P + 1) * (P + 2) / 2, NFP = 3 * (P + 1), PB = (NP + 3) / 4, FB = (NFP + 3) / 4;
     static constexpr bool BIG = sizeof(R) == 8 && P == 5;
-    static constexpr int G = BIG ? 1 : 2, WV = P == 1 ? 8 : 4, value = 4 * G * WV;
+    static constexpr int G = BIG ? 1 : 2, WV = P == 1 ? 8 : 4;
+    // FP32 meshes of at least this many elements have tiles of 64, as the scalar stage form has (so that no trace
+    // is formed again), and take the scalar form below: P1 always, P2 where dJ/d(dt) is asked for (else eight
+    // waves of the matrix-core form)
+    static constexpr int LARGE_FROM = sizeof(R) == 8 || P > 2 ? INT_MAX : P == 1 ? 16384 : 24576;
+    static constexpr int tile(int E) { return E >= LARGE_FROM ? TILE : 4 * G * WV; }
     // waves per SIMD asked for: in FP64 the face points' VJPs take more than the 256 VGPRs of two (P2:
     // 584 us a step at one wave, 707 at two with scratch), P5's LDS allows one workgroup
     static constexpr int WPE = (sizeof(R) == 8 ? P == 1 : P < 5) ? 2 : 1;
@@ -2034,13 +2040,13 @@ template <typename R, int P> struct TriViscVjpTile {
     static constexpr int ESF = tri::elem_stride<R>(4 * FB), ESX = tri::elem_stride<R>(ROWS);
 };
 
-template <typename R, int P, int MODE>
-__global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R, P>::WPE)) void tri_visc_vjp_kernel(TriVjpArgs<R> a) {
+template <typename R, int P, int MODE, int NWV>
+__global__ __launch_bounds__(64 * NWV, (TriViscVjpTile<R, P>::WPE)) void tri_visc_vjp_kernel(TriVjpArgs<R> a) {
     using S = TriShape<P>;
     using TV = TriViscVjpTile<R, P>;
     using FO = tri::FragOps<R, P>;
     constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP, PB = FO::PB, FB = FO::FB;
-    constexpr int G = TV::G, NWV = TV::WV, NB = 64 * NWV, TT = TV::value, ESF = TV::ESF, ESX = TV::ESX;
+    constexpr int G = TV::G, NB = 64 * NWV, TT = 4 * G * NWV, ESF = TV::ESF, ESX = TV::ESX;
     constexpr int RU = TV::RU, RA = 2 * NP, RB = 3 * NP;       // point rows
     constexpr int RY = NFP, RO = 2 * NFP, RD = 3 * NFP;         // trace rows
     constexpr double ca = MODE == MODE_STAGE2 ? 0.75 : (MODE == MODE_STAGE3 ? 1.0 / 3.0 : 0.0);
@@ -2503,6 +2509,626 @@ __global__ __launch_bounds__((64 * TriViscVjpTile<R, P>::WV), (TriViscVjpTile<R,
         }
 }
 
+// The same VJP of large FP32 meshes (TriViscVjpTile): lanes and operators as in
+// tri_visc_scalar_kernel, whose reasons hold here too, and the residual formed
+// along with the rest, where the matrix-core form takes a launch of its own
+// for it.  A step backwards, us, matrix cores / this: P1 without and with
+// dJ/d(dt) 500,000 elements 1247 / 966 and 1592 / 1021, 39,200 elements
+// 120 / 96 and 171 / 110, 25,088 elements 84 / 80 and 127 / 95; P2 with
+// dJ/d(dt) 500,000 elements 2776 / 2161, 32,768 elements 224 / 155, 25,088
+// elements 187 / 154 (without, eight waves against four: 2113 / 1909,
+// 156 / 130 and 126 / 126).
+// Per lane (element, variable) unless stated, after the forward values:
+//   R1  cotangent of u_out, the RK combination
+//   R2, R4  the lifting, the divergence and the normal fluxes transposed;
+//       then one lane per point
+//   R5  the corrected gradient's lifted jumps transposed: each edge point's
+//       jump cotangent
+//   R3  per solved face point; then the face liftings transposed, gathered
+//       over the edge's points
+//   R6  the traces and the gradient transposed: cotangent of q
+template <typename R, int P, int MODE>
+__global__ __launch_bounds__(BLOCK) void tri_visc_vjp_scalar_kernel(TriVjpArgs<R> a) {
+    using S = TriShape<P>;
+    constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
+    constexpr int TT = TILE, NB = BLOCK, NWV = NB / 64;
+    using OP = TriOps<P>;
+    constexpr int O0 = ops_offset(P), CA = OP::CA, OI = O0 + OP::C;
+    constexpr int XW = 2 * (NP > NFP ? NP : NFP);  // the point fluxes, later the jump cotangents
+    constexpr double ca = MODE == MODE_STAGE2 ? 0.75 : (MODE == MODE_STAGE3 ? 1.0 / 3.0 : 0.0);
+    constexpr double cb = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
+    constexpr double cc = MODE == MODE_STAGE2 ? 0.25 : (MODE == MODE_STAGE3 ? 2.0 / 3.0 : 1.0);
+    const int OLT = O0 + a.lift_off;
+    const int LFO = lf_offset(P) + a.lf_off;
+    __shared__ R sTu[TT * NFP * NV];   // traces of U
+    __shared__ R sTx[TT * NFP * NV];   // traces of the gradient, then their cotangents
+    __shared__ R sTy[TT * NFP * NV];
+    __shared__ R sD[TT * NFP * NV];    // flux differences, their cotangents, then the U traces' cotangents
+    __shared__ R sU[TT * NP * NV];     // q, then the flux VJPs' cotangents of U at the points
+    __shared__ R sQx[TT * NP * NV];    // corrected gradient, then its cotangent
+    __shared__ R sQy[TT * NP * NV];
+    __shared__ R sX[TT * XW * NV];     // contravariant point fluxes, then their x / y cotangents;
+                                       // later the jump cotangents and the face liftings' seeds
+    __shared__ double sred[NWV];
+    __shared__ R sEdge[TT * 3];
+    __shared__ int2 sLink[TT * 3];
+    __shared__ R sNrm[TT * 3 * 2];
+    __shared__ unsigned char sList[TT * 3];
+    __shared__ int sCnt[NWV];
+    R* const sFR = sX;
+    R* const sFS = sX + TT * NP * NV;
+    R* const sJ = sX;
+    R* const sC = sX + TT * NFP * NV;
+
+    const int tid = threadIdx.x, el = tid >> 2, v = tid & 3;
+    const int tile = tile_of_block(a.xcd_groups);
+    const int e0 = tile * TT, e = e0 + el;
+    const bool live = e < a.E;
+    const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
+    const int64_t base = blk(e, 0, NP) + v;
+    auto sl = [](int elx, int j, int w) { return (elx * NFP + j) * NV + w; };
+    auto sp = [](int elx, int m, int w) { return (elx * NP + m) * NV + w; };
+
+    // ---- forward 0: state, gradient, traces of U and of the gradient
+    R rx = R(0), ry = R(0), sx = R(0), sy = R(0);
+    R jwx[3] = {R(0), R(0), R(0)}, jwy[3] = {R(0), R(0), R(0)};  // each edge's jump weights
+    int2 L[3] = {make_int2(0, 0), make_int2(0, 0), make_int2(0, 0)};
+    if (live) {
+#pragma unroll
+        for (int m = 0; m < NP; ++m) sU[sp(el, m, v)] = R(a.U_in[base + (int64_t)m * EB * NV]);
+        const R* G = a.geo + (int64_t)e * GEO;
+        rx = G[0]; ry = G[1]; sx = G[2]; sy = G[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) L[k] = a.links[(int64_t)e * 3 + k];
+        R se[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const R ax = k == 0 ? sx : (k == 1 ? rx + sx : rx), ay = k == 0 ? sy : (k == 1 ? ry + sy : ry);
+            se[k] = sqrtR(ax * ax + ay * ay);
+            const R sg = link_role(L[k].y) == ROLE_RIGHT ? R(-1) : R(1);
+            jwx[k] = sg * se[k] * G[4 + 2 * k];
+            jwy[k] = sg * se[k] * G[5 + 2 * k];
+        }
+        if (v < 3) {
+            sEdge[el * 3 + v] = se[v];
+            sLink[el * 3 + v] = L[v];
+            sNrm[(el * 3 + v) * 2] = G[4 + 2 * v];
+            sNrm[(el * 3 + v) * 2 + 1] = G[5 + 2 * v];
+        }
+        R gr[NP], gs[NP];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) { gr[i] = R(0); gs[i] = R(0); }
+#pragma unroll
+        for (int m = 0; m < NP; ++m) {
+            const R um = sU[sp(el, m, v)];
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                gr[i] = fmaR(cop<R>(O0 + m * CA + i), um, gr[i]);
+                gs[i] = fmaR(cop<R>(O0 + m * CA + NP + i), um, gs[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            sQx[sp(el, i, v)] = rx * gr[i] + sx * gs[i];
+            sQy[sp(el, i, v)] = ry * gr[i] + sy * gs[i];
+        }
+#pragma unroll 1
+        for (int j = 0; j < NFP; ++j) {
+            R tu = R(0), tx = R(0), ty = R(0);
+#pragma unroll
+            for (int m = 0; m < NP; ++m) {
+                const R w = cop<R>(OI + j * NP + m);
+                tu = fmaR(w, sU[sp(el, m, v)], tu);
+                tx = fmaR(w, sQx[sp(el, m, v)], tx);
+                ty = fmaR(w, sQy[sp(el, m, v)], ty);
+            }
+            sTu[sl(el, j, v)] = tu;
+            sTx[sl(el, j, v)] = tx;
+            sTy[sl(el, j, v)] = ty;
+        }
+    }
+    bool owned = false;
+    if (live && v < 3) {
+        const int2 Lv = v == 0 ? L[0] : (v == 1 ? L[1] : L[2]);
+        const int nl = Lv.x - e0;
+        owned = !(link_role(Lv.y) == ROLE_RIGHT && nl >= 0 && nl < TT);
+    }
+    const unsigned long long own_mask = __ballot(owned);
+    const int lane = tid & 63, wave = tid >> 6;
+    if (lane == 0) sCnt[wave] = __popcll(own_mask);
+    __syncthreads();
+
+    // ---- forward 1: corrected gradient
+    if (live) {
+        R jx[NFP], jy[NFP];
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk) {
+            const int2 Lk = L[kk];
+            const int nl = Lk.x - e0;
+            const bool in = nl >= 0 && nl < TT;
+            const int ek = link_edge(Lk.y);
+#pragma unroll
+            for (int f = 0; f < FP; ++f) {
+                const int j = kk * FP + f, oj = ek * FP + (P - f);
+                const R own = sTu[sl(el, j, v)];
+                R oth;
+                if (in) oth = sTu[sl(nl, oj, v)];
+                else oth = a.T_in[((int64_t)Lk.x * NFP + oj) * TWV + v];
+                const R jmp = R(0.5) * (own + oth) - own;
+                jx[j] = jwx[kk] * jmp;
+                jy[j] = jwy[kk] * jmp;
+            }
+        }
+#pragma unroll 1
+        for (int i = 0; i < NP; ++i) {
+            R qx = sQx[sp(el, i, v)], qy = sQy[sp(el, i, v)];
+#pragma unroll
+            for (int j = 0; j < NFP; ++j) {
+                const R l = cop<R>(OLT + j * NP + i);
+                qx = fmaR(l, jx[j], qx);
+                qy = fmaR(l, jy[j], qy);
+            }
+            sQx[sp(el, i, v)] = qx;
+            sQy[sp(el, i, v)] = qy;
+        }
+    }
+    if (owned) {
+        int pos = __popcll(own_mask & ((1ull << lane) - 1));
+        for (int w = 0; w < wave; ++w) pos += sCnt[w];
+        sList[pos] = (unsigned char)(el * 3 + v);
+    }
+    __syncthreads();
+
+    // ---- forward 2: contravariant total fluxes at the points (points v, v + 4,
+    // ... of the element, four variables each), then this lane's divergence
+    // and interpolated normal fluxes
+    constexpr int MPL = (NP + NV - 1) / NV;
+    if (live) {
+#pragma unroll 1
+        for (int q = 0; q < MPL; ++q) {
+            const int m = v + NV * q;
+            if (m >= NP) break;
+            R U4[NV], X4[NV], Y4[NV];
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                U4[w] = sU[sp(el, m, w)];
+                X4[w] = sQx[sp(el, m, w)];
+                Y4[w] = sQy[sp(el, m, w)];
+            }
+            const R inv = fast_rcp(U4[0]);
+            const R ux = U4[1] * inv, uy = U4[2] * inv;
+            const R p = (g - R(1)) * (U4[3] - R(0.5) * (U4[1] * ux + U4[2] * uy));
+            R Fv[NV], Gv[NV];
+            visc_flux(U4, X4, Y4, g, mu, kappa, Fv, Gv);
+            const R fx[NV] = {U4[1], U4[1] * ux + p, U4[1] * uy, (U4[3] + p) * ux};
+            const R fy[NV] = {U4[2], U4[2] * ux, U4[2] * uy + p, (U4[3] + p) * uy};
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                const R Fx = fx[w] - Fv[w], Fy = fy[w] - Gv[w];
+                sFR[sp(el, m, w)] = rx * Fx + ry * Fy;
+                sFS[sp(el, m, w)] = sx * Fx + sy * Fy;
+            }
+        }
+    }
+    __syncthreads();
+    R div[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) div[i] = R(0);
+    if (live) {
+        R fn[NFP];
+#pragma unroll
+        for (int j = 0; j < NFP; ++j) fn[j] = R(0);
+#pragma unroll 1
+        for (int m = 0; m < NP; ++m) {
+            const R fr = sFR[sp(el, m, v)], fs = sFS[sp(el, m, v)], frs = fr + fs;
+#pragma unroll
+            for (int i = 0; i < NP; ++i)
+                div[i] = fmaR(cop<R>(O0 + m * CA + NP + i), fs, fmaR(cop<R>(O0 + m * CA + i), fr, div[i]));
+#pragma unroll
+            for (int j = 0; j < NFP; ++j)
+                fn[j] = fmaR(cop<R>(O0 + m * CA + 2 * NP + j), j < FP ? fs : (j < 2 * FP ? frs : fr), fn[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < NFP; ++j) sD[sl(el, j, v)] = (j >= FP && j < 2 * FP) ? fn[j] : -fn[j];
+    }
+    __syncthreads();
+    int nsolved = 0;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) nsolved += sCnt[w];
+
+    // the values of one solved face point (slot j of element elt, edge kk):
+    // both sides' traces, edge factors, the face liftings of the jumps and
+    // the averaged state and BR2 gradient
+    struct Face {
+        int elt, kk, j, ek, oj, nl;
+        bool in, right;
+        int2 Lk;
+        R nx, ny, so, sn;
+        R own[NV], oth[NV], Uc[NV], Qbx[NV], Qby[NV];
+    };
+    auto face_at = [&](int t, Face& F) __attribute__((always_inline)) {
+        const int c = sList[t / FP], f = t - (t / FP) * FP;
+        F.elt = c / 3;
+        F.kk = c - F.elt * 3;
+        F.j = F.kk * FP + f;
+        F.Lk = sLink[F.elt * 3 + F.kk];
+        F.right = link_role(F.Lk.y) == ROLE_RIGHT;
+        F.nx = sNrm[(F.elt * 3 + F.kk) * 2];
+        F.ny = sNrm[(F.elt * 3 + F.kk) * 2 + 1];
+        F.ek = link_edge(F.Lk.y);
+        F.oj = F.ek * FP + (P - f);
+        F.nl = F.Lk.x - e0;
+        F.in = F.nl >= 0 && F.nl < TT;
+        const R* Tn = a.T_in + (int64_t)F.Lk.x * NFP * TWV;
+        R gxo[NV], gyo[NV], gxn[NV], gyn[NV];
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            F.own[w] = sTu[sl(F.elt, F.j, w)];
+            gxo[w] = sTx[sl(F.elt, F.j, w)];
+            gyo[w] = sTy[sl(F.elt, F.j, w)];
+        }
+        if (F.in) {
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                F.oth[w] = sTu[sl(F.nl, F.oj, w)];
+                gxn[w] = sTx[sl(F.nl, F.oj, w)];
+                gyn[w] = sTy[sl(F.nl, F.oj, w)];
+            }
+            F.sn = sEdge[F.nl * 3 + F.ek];
+        } else {
+            load4(Tn + (int64_t)F.oj * TWV, F.oth);
+            load4(Tn + (int64_t)F.oj * TWV + NV, gxn);
+            load4(Tn + (int64_t)F.oj * TWV + 2 * NV, gyn);
+            const R* Gn = a.geo + (int64_t)F.Lk.x * GEO;
+            const R ax = F.ek == 0 ? Gn[2] : (F.ek == 1 ? Gn[0] + Gn[2] : Gn[0]);
+            const R ay = F.ek == 0 ? Gn[3] : (F.ek == 1 ? Gn[1] + Gn[3] : Gn[1]);
+            F.sn = sqrtR(ax * ax + ay * ay);
+        }
+        F.so = sEdge[F.elt * 3 + F.kk];
+        R lo[NV] = {R(0), R(0), R(0), R(0)}, ln[NV] = {R(0), R(0), R(0), R(0)};
+#pragma unroll 1
+        for (int f2 = 0; f2 < FP; ++f2) {
+            const int j2 = F.kk * FP + f2, o2 = F.ek * FP + (P - f2);
+            R uo[NV], un[NV];
+#pragma unroll
+            for (int w = 0; w < NV; ++w) uo[w] = sTu[sl(F.elt, j2, w)];
+            if (F.in) {
+#pragma unroll
+                for (int w = 0; w < NV; ++w) un[w] = sTu[sl(F.nl, o2, w)];
+            } else {
+                load4(Tn + (int64_t)o2 * TWV, un);
+            }
+            const R wo = clf<R>(LFO + (F.kk * FP + f) * FP + f2);
+            const R wn = clf<R>(LFO + (F.ek * FP + (P - f)) * FP + (P - f2));
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                const R jo = R(0.5) * (uo[w] + un[w]) - uo[w];
+                lo[w] = fmaR(wo, jo, lo[w]);
+                ln[w] = fmaR(wn, jo, ln[w]);
+            }
+        }
+        const R sg = F.right ? R(-1) : R(1);
+        const R nox = sg * F.nx, noy = sg * F.ny;
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            F.Uc[w] = R(0.5) * (F.own[w] + F.oth[w]);
+            F.Qbx[w] = R(0.5) * ((gxo[w] + eta * F.so * nox * lo[w]) + (gxn[w] + eta * F.sn * nox * ln[w]));
+            F.Qby[w] = R(0.5) * ((gyo[w] + eta * F.so * noy * lo[w]) + (gyn[w] + eta * F.sn * noy * ln[w]));
+        }
+    };
+
+    // ---- forward 3: flux differences of both sides of every solved face point
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
+        Face F;
+        face_at(t, F);
+        R UL[NV], UR[NV], Fc[NV], Fv[NV], Gv[NV];
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            UL[w] = F.right ? F.oth[w] : F.own[w];
+            UR[w] = F.right ? F.own[w] : F.oth[w];
+        }
+        visc_flux(F.Uc, F.Qbx, F.Qby, g, mu, kappa, Fv, Gv);
+        riemann_by_kind(a.riemann, UL, UR, F.nx, F.ny, g, Fc);
+        const R sc = F.right ? -F.so : F.so;
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            const R fi = Fc[w] - (Fv[w] * F.nx + Gv[w] * F.ny);
+            sD[sl(F.elt, F.j, w)] = sc * fi - sD[sl(F.elt, F.j, w)];
+            if (F.in) sD[sl(F.nl, F.oj, w)] = -F.sn * fi - sD[sl(F.nl, F.oj, w)];
+        }
+    }
+    __syncthreads();
+
+    // ---- forward 4 and R1: residual; cotangent of u_out, RK combination
+    double rsum = 0.0;
+    R divb[NP];
+    double qb[NP];
+    if (live) {
+#pragma unroll 1
+        for (int j = 0; j < NFP; ++j) {
+            const R d = sD[sl(el, j, v)];
+#pragma unroll
+            for (int i = 0; i < NP; ++i) div[i] = fmaR(cop<R>(OLT + j * NP + i), d, div[i]);
+        }
+        double unb[NP];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) unb[i] = a.Ub_in[base + (int64_t)i * EB * NV];
+        if (MODE != MODE_RESIDUAL && a.Tb_in) {
+            // edge cotangents of u_out's traces (U, gradient) left on this element's cross-tile edges
+            R tu[NFP], tx[NFP], ty[NFP];
+            bool any = false;
+#pragma unroll
+            for (int kk = 0; kk < 3; ++kk) {
+                const int nl = L[kk].x - e0;
+                const bool cross = !(nl >= 0 && nl < TT);
+                any = any || cross;
+#pragma unroll
+                for (int f = 0; f < FP; ++f) {
+                    const int j = kk * FP + f;
+                    const R* Tb = a.Tb_in + ((int64_t)e * NFP + j) * TWV;
+                    tu[j] = cross ? Tb[v] : R(0);
+                    tx[j] = cross ? Tb[NV + v] : R(0);
+                    ty[j] = cross ? Tb[2 * NV + v] : R(0);
+                }
+            }
+            if (any) {
+                R grb[NP], gsb[NP];
+#pragma unroll
+                for (int m = 0; m < NP; ++m) {
+                    R su = R(0), qx = R(0), qy = R(0);
+#pragma unroll
+                    for (int j = 0; j < NFP; ++j) {
+                        const R w = cop<R>(OI + j * NP + m);
+                        su = fmaR(w, tu[j], su);
+                        qx = fmaR(w, tx[j], qx);
+                        qy = fmaR(w, ty[j], qy);
+                    }
+                    unb[m] += double(su);
+                    grb[m] = rx * qx + ry * qy;
+                    gsb[m] = sx * qx + sy * qy;
+                }
+#pragma unroll
+                for (int m = 0; m < NP; ++m) {
+                    R acc = R(0);
+#pragma unroll
+                    for (int i = 0; i < NP; ++i)
+                        acc = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], acc));
+                    unb[m] += double(acc);
+                }
+            }
+        }
+        const double dt = MODE == MODE_RESIDUAL ? 0.0 : *a.dt_ptr;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int64_t gi = base + (int64_t)i * EB * NV;
+            double rb;
+            if (MODE == MODE_RESIDUAL) {
+                rb = unb[i];
+                qb[i] = 0.0;
+            } else {
+                if (MODE == MODE_STAGE3) a.U0b[gi] = ca * unb[i];
+                if (MODE == MODE_STAGE2) a.U0b[gi] += ca * unb[i];
+                qb[i] = cb * unb[i];
+                rb = cc * dt * unb[i];
+                rsum += cc * (-double(div[i])) * unb[i];
+            }
+            divb[i] = R(-rb);  // R = -div
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) { divb[i] = R(0); qb[i] = 0.0; }
+    }
+    if (a.dtb_partial) {
+        const double s2 = block_reduce_n<OpSum, NWV>(rsum, sred);
+        if (tid == 0) a.dtb_partial[tile] = s2;
+    }
+    __syncthreads();
+
+    // ---- R2, R4: the lifting transposed; the divergence and normal fluxes
+    // transposed to the x / y flux cotangents at the points
+    if (live) {
+#pragma unroll 1
+        for (int j = 0; j < NFP; ++j) {
+            R acc = R(0);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) acc = fmaR(cop<R>(OLT + j * NP + i), divb[i], acc);
+            sD[sl(el, j, v)] = acc;
+        }
+#pragma unroll 1
+        for (int m = 0; m < NP; ++m) {
+            R frb = R(0), fsb = R(0);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                frb = fmaR(cop<R>(O0 + m * CA + i), divb[i], frb);
+                fsb = fmaR(cop<R>(O0 + m * CA + NP + i), divb[i], fsb);
+            }
+#pragma unroll
+            for (int j = 0; j < NFP; ++j) {
+                // d = sc F^I - Fn with Fn = -fn (edges 0, 2), +fn (edge 1); fn_j
+                // interpolates fs, fr + fs, fr on edges 0, 1, 2
+                const R im = cop<R>(O0 + m * CA + 2 * NP + j);
+                const R db = sD[sl(el, j, v)];
+                const R fnb = (j >= FP && j < 2 * FP) ? -db : db;
+                if (j >= FP) frb = fmaR(im, fnb, frb);
+                if (j < 2 * FP) fsb = fmaR(im, fnb, fsb);
+            }
+            sFR[sp(el, m, v)] = rx * frb + sx * fsb;  // cotangent of F_x = f_x - F_v
+            sFS[sp(el, m, v)] = ry * frb + sy * fsb;  // and of F_y
+        }
+    }
+    __syncthreads();
+    if (live) {
+#pragma unroll 1
+        for (int q = 0; q < MPL; ++q) {
+            const int m = v + NV * q;
+            if (m >= NP) break;
+            R U4[NV], X4[NV], Y4[NV], A4[NV], B4[NV], Fb[NV], Gb[NV];
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                U4[w] = sU[sp(el, m, w)];
+                X4[w] = sQx[sp(el, m, w)];
+                Y4[w] = sQy[sp(el, m, w)];
+                A4[w] = sFR[sp(el, m, w)];
+                B4[w] = sFS[sp(el, m, w)];
+                Fb[w] = -A4[w];
+                Gb[w] = -B4[w];
+            }
+            R Ub4[NV] = {R(0), R(0), R(0), R(0)}, Xb4[NV] = {R(0), R(0), R(0), R(0)},
+              Yb4[NV] = {R(0), R(0), R(0), R(0)};
+            euler_flux_vjp(U4, g, A4, B4, Ub4);
+            visc_flux_vjp(U4, X4, Y4, g, mu, kappa, Fb, Gb, Ub4, Xb4, Yb4);
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                sU[sp(el, m, w)] = Ub4[w];
+                sQx[sp(el, m, w)] = Xb4[w];
+                sQy[sp(el, m, w)] = Yb4[w];
+            }
+        }
+    }
+    __syncthreads();
+
+    // ---- R5: the corrected gradient's lifted jumps transposed
+    if (live) {
+#pragma unroll 1
+        for (int j = 0; j < NFP; ++j) {
+            R bx = R(0), by = R(0);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                const R l = cop<R>(OLT + j * NP + i);
+                bx = fmaR(l, sQx[sp(el, i, v)], bx);
+                by = fmaR(l, sQy[sp(el, i, v)], by);
+            }
+            const int kk = j / FP;
+            sJ[sl(el, j, v)] = (kk == 0 ? jwx[0] : (kk == 1 ? jwx[1] : jwx[2])) * bx +
+                               (kk == 0 ? jwy[0] : (kk == 1 ? jwy[1] : jwy[2])) * by;
+        }
+    }
+    __syncthreads();
+
+    // ---- R3: every solved face point backwards
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
+        Face F;
+        face_at(t, F);
+        R UL[NV], UR[NV], Fcb[NV], Fvb[NV], Gvb[NV];
+        const R sc = F.right ? -F.so : F.so;
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            UL[w] = F.right ? F.oth[w] : F.own[w];
+            UR[w] = F.right ? F.own[w] : F.oth[w];
+            R fb = sc * sD[sl(F.elt, F.j, w)];
+            if (F.in) fb += -F.sn * sD[sl(F.nl, F.oj, w)];
+            Fcb[w] = fb;
+            Fvb[w] = -fb * F.nx;
+            Gvb[w] = -fb * F.ny;
+        }
+        R ULb[NV] = {R(0), R(0), R(0), R(0)}, URb[NV] = {R(0), R(0), R(0), R(0)};
+        riemann_by_kind_vjp(a.riemann, UL, UR, F.nx, F.ny, g, Fcb, ULb, URb);
+        R Ucb[NV] = {R(0), R(0), R(0), R(0)}, Qxb[NV] = {R(0), R(0), R(0), R(0)}, Qyb[NV] = {R(0), R(0), R(0), R(0)};
+        visc_flux_vjp(F.Uc, F.Qbx, F.Qby, g, mu, kappa, Fvb, Gvb, Ucb, Qxb, Qyb);
+        const R sg = F.right ? R(-1) : R(1);
+        const R nox = sg * F.nx, noy = sg * F.ny;
+        R ownb[NV], othb[NV];
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+            const R jo = sJ[sl(F.elt, F.j, w)], jn = F.in ? sJ[sl(F.nl, F.oj, w)] : R(0);
+            ownb[w] = (F.right ? URb[w] : ULb[w]) + R(0.5) * Ucb[w] - R(0.5) * jo + R(0.5) * jn;
+            othb[w] = (F.right ? ULb[w] : URb[w]) + R(0.5) * Ucb[w] + R(0.5) * jo - R(0.5) * jn;
+            Qxb[w] *= R(0.5);
+            Qyb[w] *= R(0.5);
+            sC[sl(F.elt, F.j, w)] = eta * (nox * Qxb[w] + noy * Qyb[w]);
+            sD[sl(F.elt, F.j, w)] = ownb[w];
+            sTx[sl(F.elt, F.j, w)] = Qxb[w];
+            sTy[sl(F.elt, F.j, w)] = Qyb[w];
+        }
+        if (F.in) {
+#pragma unroll
+            for (int w = 0; w < NV; ++w) {
+                sD[sl(F.nl, F.oj, w)] = othb[w];
+                sTx[sl(F.nl, F.oj, w)] = Qxb[w];
+                sTy[sl(F.nl, F.oj, w)] = Qyb[w];
+            }
+        } else {
+            R* Tb = a.Tb_out + ((int64_t)F.Lk.x * NFP + F.oj) * TWV;
+            store4(Tb, othb);
+            store4(Tb + NV, Qxb);
+            store4(Tb + 2 * NV, Qyb);
+        }
+    }
+    __syncthreads();
+    // the face liftings transposed: the jump at this point from every point's
+    // lifting cotangents (the seeds c, times each side's edge factor)
+#pragma unroll 1
+    for (int t = tid; t < nsolved * FP; t += NB) {
+        const int c = sList[t / FP], f = t - (t / FP) * FP;
+        const int elt = c / 3, kk = c - elt * 3, j = kk * FP + f;
+        const int2 Lk = sLink[elt * 3 + kk];
+        const int ek = link_edge(Lk.y), oj = ek * FP + (P - f), nl = Lk.x - e0;
+        const bool in = nl >= 0 && nl < TT;
+        const R so = sEdge[elt * 3 + kk];
+        R sn;
+        if (in) {
+            sn = sEdge[nl * 3 + ek];
+        } else {
+            const R* Gn = a.geo + (int64_t)Lk.x * GEO;
+            const R ax = ek == 0 ? Gn[2] : (ek == 1 ? Gn[0] + Gn[2] : Gn[0]);
+            const R ay = ek == 0 ? Gn[3] : (ek == 1 ? Gn[1] + Gn[3] : Gn[1]);
+            sn = sqrtR(ax * ax + ay * ay);
+        }
+        R jb[NV] = {R(0), R(0), R(0), R(0)};
+#pragma unroll 1
+        for (int f1 = 0; f1 < FP; ++f1) {
+            const R w1 = so * clf<R>(LFO + (kk * FP + f1) * FP + f) +
+                         sn * clf<R>(LFO + (ek * FP + (P - f1)) * FP + (P - f));
+#pragma unroll
+            for (int w = 0; w < NV; ++w) jb[w] = fmaR(w1, sC[sl(elt, kk * FP + f1, w)], jb[w]);
+        }
+        // jump = (u_n - u_o) / 2 at this point
+#pragma unroll
+        for (int w = 0; w < NV; ++w) sD[sl(elt, j, w)] -= R(0.5) * jb[w];
+        if (in) {
+#pragma unroll
+            for (int w = 0; w < NV; ++w) sD[sl(nl, oj, w)] += R(0.5) * jb[w];
+        } else {
+            R* Tb = a.Tb_out + ((int64_t)Lk.x * NFP + oj) * TWV;
+#pragma unroll
+            for (int w = 0; w < NV; ++w) Tb[w] += R(0.5) * jb[w];
+        }
+    }
+    __syncthreads();
+
+    // ---- R6: traces and gradient transposed; cotangent of q
+    if (!live) return;
+    R grb[NP], gsb[NP];
+    double out[NP];
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {
+        R su = R(0), qx = sQx[sp(el, m, v)], qy = sQy[sp(el, m, v)];
+#pragma unroll
+        for (int j = 0; j < NFP; ++j) {
+            const R w = cop<R>(OI + j * NP + m);
+            su = fmaR(w, sD[sl(el, j, v)], su);
+            qx = fmaR(w, sTx[sl(el, j, v)], qx);
+            qy = fmaR(w, sTy[sl(el, j, v)], qy);
+        }
+        out[m] = qb[m] + double(sU[sp(el, m, v)]) + double(su);
+        grb[m] = rx * qx + ry * qy;
+        gsb[m] = sx * qx + sy * qy;
+    }
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {
+        R acc = R(0);
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+            acc = fmaR(cop<R>(O0 + m * CA + NP + i), gsb[i], fmaR(cop<R>(O0 + m * CA + i), grb[i], acc));
+        const int64_t gi = base + (int64_t)m * EB * NV;
+        double o = out[m] + double(acc);
+        if (MODE == MODE_STAGE1) o += a.U0b[gi];
+        a.Ub_out[gi] = o;
+    }
+}
+
 // Completion of a cotangent with the Navier-Stokes terms: U_bar plus the
 // transposed traces of U and of its gradient for the cross-tile edge
 // cotangents (12 words per point) that the last adjoint launch left (tiles of
@@ -2847,15 +3473,20 @@ hipError_t tri_complete(int P, int E, const int2* links, const double* Ub, const
     return hipGetLastError();
 }
 
-// The BR2 adjoint's elements per workgroup for an order and precision.
-int tri_visc_vjp_tile(int P, bool fp64) {
+// The BR2 adjoint's elements per workgroup for an order, precision and mesh size.
+int tri_visc_vjp_tile(int P, bool fp64, int E) {
     switch (P) {
-    case 1: return fp64 ? TriViscVjpTile<double, 1>::value : TriViscVjpTile<float, 1>::value;
-    case 2: return fp64 ? TriViscVjpTile<double, 2>::value : TriViscVjpTile<float, 2>::value;
-    case 3: return fp64 ? TriViscVjpTile<double, 3>::value : TriViscVjpTile<float, 3>::value;
-    case 4: return fp64 ? TriViscVjpTile<double, 4>::value : TriViscVjpTile<float, 4>::value;
-    default: return fp64 ? TriViscVjpTile<double, 5>::value : TriViscVjpTile<float, 5>::value;
+    case 1: return fp64 ? TriViscVjpTile<double, 1>::tile(E) : TriViscVjpTile<float, 1>::tile(E);
+    case 2: return fp64 ? TriViscVjpTile<double, 2>::tile(E) : TriViscVjpTile<float, 2>::tile(E);
+    case 3: return fp64 ? TriViscVjpTile<double, 3>::tile(E) : TriViscVjpTile<float, 3>::tile(E);
+    case 4: return fp64 ? TriViscVjpTile<double, 4>::tile(E) : TriViscVjpTile<float, 4>::tile(E);
+    default: return fp64 ? TriViscVjpTile<double, 5>::tile(E) : TriViscVjpTile<float, 5>::tile(E);
     }
+}
+
+// Whether the VJP of a mesh forms the residual itself for dJ/d(dt).
+template <typename R> bool tri_visc_vjp_has_residual(int P, int E) {
+    return E >= (P == 1 ? TriViscVjpTile<R, 1>::LARGE_FROM : P == 2 ? TriViscVjpTile<R, 2>::LARGE_FROM : INT_MAX);
 }
 
 template <typename R, int P>
@@ -2863,14 +3494,29 @@ hipError_t tri_visc_vjp_p(int mode, const TriVjpArgs<R>& a, hipStream_t s) {
     if constexpr (std::is_same<R, double>::value && P == 4) {
         return hipErrorInvalidValue;  // refused when the handle is made
     } else {
-        constexpr int TT = TriViscVjpTile<R, P>::value;
-        const int grid = (std::max(a.E, 1) + TT - 1) / TT;
-        const dim3 blk(64 * TriViscVjpTile<R, P>::WV);
+        using TV = TriViscVjpTile<R, P>;
+        const int TT = TV::tile(a.E), grid = (std::max(a.E, 1) + TT - 1) / TT;
+        auto launch = [&](auto m) {
+            constexpr int MODE = decltype(m)::value;
+            if constexpr (TV::LARGE_FROM < INT_MAX)
+                if (a.E >= TV::LARGE_FROM) {
+                    if constexpr (P == 2) {
+                        if (MODE == MODE_RESIDUAL || !a.dtb_partial) {
+                            klaunch(tri_visc_vjp_kernel<R, P, MODE, 2 * TV::WV>, grid, dim3(128 * TV::WV), 0, s, a);
+                            return;
+                        }
+                    }
+                    if constexpr (P == 1 || MODE != MODE_RESIDUAL)
+                        klaunch(tri_visc_vjp_scalar_kernel<R, P, MODE>, grid, dim3(BLOCK), 0, s, a);
+                    return;
+                }
+            klaunch(tri_visc_vjp_kernel<R, P, MODE, TV::WV>, grid, dim3(64 * TV::WV), 0, s, a);
+        };
         switch (mode) {
-        case MODE_RESIDUAL: klaunch(tri_visc_vjp_kernel<R, P, MODE_RESIDUAL>, grid, blk, 0, s, a); break;
-        case MODE_STAGE1: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE1>, grid, blk, 0, s, a); break;
-        case MODE_STAGE2: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE2>, grid, blk, 0, s, a); break;
-        default: klaunch(tri_visc_vjp_kernel<R, P, MODE_STAGE3>, grid, blk, 0, s, a); break;
+        case MODE_RESIDUAL: launch(std::integral_constant<int, MODE_RESIDUAL>{}); break;
+        case MODE_STAGE1: launch(std::integral_constant<int, MODE_STAGE1>{}); break;
+        case MODE_STAGE2: launch(std::integral_constant<int, MODE_STAGE2>{}); break;
+        default: launch(std::integral_constant<int, MODE_STAGE3>{}); break;
         }
         return hipGetLastError();
     }
@@ -2890,11 +3536,21 @@ hipError_t tri_visc_vjp(int P, int mode, const TriVjpArgs<R>& a, hipStream_t s) 
 template <typename R, int P>
 hipError_t tri_visc_complete_p(int E, const int2* links, const R* geo, const double* Ub, const R* Tb, double* out,
                                int xcd, hipStream_t s) {
-    constexpr int TT = TriViscVjpTile<R, P>::value;
-    if constexpr (P <= 2)
-        tri_visc_complete_scalar_kernel<R, P, TT><<<(std::max(E, 1) + TT - 1) / TT, TT * NV, 0, s>>>(E, links, geo, Ub, Tb, out, xcd);
-    else
-        tri_visc_complete_kernel<R, P, TT><<<(std::max(E, 1) + TRACE_TILE - 1) / TRACE_TILE, BLOCK, 0, s>>>(E, links, geo, Ub, Tb, out);
+    using TV = TriViscVjpTile<R, P>;
+    if constexpr (P <= 2) {
+        auto launch = [&](auto tile) {
+            constexpr int TT = decltype(tile)::value;
+            tri_visc_complete_scalar_kernel<R, P, TT><<<(std::max(E, 1) + TT - 1) / TT, TT * NV, 0, s>>>(E, links, geo, Ub, Tb, out, xcd);
+        };
+        if constexpr (TV::LARGE_FROM < INT_MAX)
+            if (E >= TV::LARGE_FROM) {
+                launch(std::integral_constant<int, TILE>{});
+                return hipGetLastError();
+            }
+        launch(std::integral_constant<int, TV::tile(1)>{});
+    } else {
+        tri_visc_complete_kernel<R, P, TV::tile(1)><<<(std::max(E, 1) + TRACE_TILE - 1) / TRACE_TILE, BLOCK, 0, s>>>(E, links, geo, Ub, Tb, out);
+    }
     return hipGetLastError();
 }
 
@@ -3545,7 +4201,7 @@ extern "C" int zj_tri_get_info(zj_tri_handle h, int64_t* n_dof, int* elems_per_b
 static int tensure_adjoint(zj_tri* h) {
     if (h->A_Ub) return ZJ_OK;
     int tt = TILE;
-    if (h->viscous) tt = tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64);
+    if (h->viscous) tt = tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64, h->E);
     ZJ_THIP(h, hipSetDevice(h->device));
     h->A_blk = (h->E + tt - 1) / tt;
     const size_t eb = ((size_t)h->E + EB - 1) / EB * EB;
@@ -3574,6 +4230,7 @@ static TriVjpArgs<R> tvjp_args(zj_tri* h) {
     a.mu = h->mu;
     a.kappa = h->kappa;
     a.eta = h->eta;
+    a.lf_off = lf_family(h->corr) * lf_words(h->P);
     a.family = lf_family(h->corr);
     return a;
 }
@@ -3590,7 +4247,7 @@ static hipError_t tri_adjoint_step(zj_tri* h, bool want_dt, hipStream_t s) {
     // kernel, whose traces (T[0] of the state, then each recomputed stage's)
     // cover the edges across them; else every edge's traces are formed after
     // each stage.
-    const bool same = h->viscous && tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64) % h->epb == 0;
+    const bool same = h->viscous && tri_visc_vjp_tile(h->P, h->prec == ZJ_PREC_FP64, h->E) % h->epb == 0;
     const bool retrace = h->viscous && !same;
     const R* T[3] = {same ? (const R*)h->T[0] : AT[0], AT[1], AT[2]};
     hipError_t e = hipSuccess;
@@ -3618,7 +4275,8 @@ static hipError_t tri_adjoint_step(zj_tri* h, bool want_dt, hipStream_t s) {
         a.Tb_out = Tb[1 - h->A_cur];
         a.U0b = h->A_U0b;
         a.dtb_partial = want_dt ? h->A_dtb + (size_t)(3 - st) * h->A_blk : nullptr;
-        if (h->viscous && want_dt) {  // the residual at q, of which the time step's cotangent is made
+        if (h->viscous && want_dt && !tri_visc_vjp_has_residual<R>(h->P, h->E)) {
+            // the residual at q, of which the time step's cotangent is made
             f = tri_args<R>(h, MODE_RESIDUAL);
             f.U_in = a.U_in; f.T_in = a.T_in; f.l2_partial = nullptr;
             if ((e = tri_visc_launch<R>(h->P, MODE_RESIDUAL, f, s)) != hipSuccess) return e;
