@@ -58,12 +58,13 @@ def test_tri_euler_tiles(p, precision, n):
 
 
 @pytest.mark.parametrize("p,n,viscous,precision", [(1, 110, False, "fp64"), (1, 111, False, "fp64"), (1, 110, True, "fp64"),
-                                                   (1, 111, True, "fp64"), (2, 127, True, "fp32bulk"),
+                                                   (1, 111, True, "fp64"), (1, 90, True, "fp64"), (1, 91, True, "fp64"),
+                                                   (2, 127, True, "fp32bulk"),
                                                    (2, 128, True, "fp32bulk"), (2, 180, False, "fp64"),
                                                    (2, 182, False, "fp64")])
 def test_tri_form_by_size(p, n, viscous, precision):
-    """Both sides of the element counts (24,576 at P1, 32,768 and 65,536 at P2) from which large meshes take
-    the scalar form of the stage kernels."""
+    """Both sides of the element counts (24,576 at P1, 16,384 there with the BR2 terms in FP64, 32,768 and 65,536 at
+    P2) from which large meshes take the scalar form of the stage kernels."""
     say(f"case: triangle stage {'viscous' if viscous else 'inviscid'}, {2 * n * n} elements P{p} {precision}")
     m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
     kw = dict(viscous=True, Re=100.0) if viscous else {}
@@ -81,7 +82,7 @@ def test_tri_form_by_size(p, n, viscous, precision):
 @pytest.mark.parametrize("p,n,viscous,precision,corr", [
     (1, 111, False, "fp64", "ga"), (1, 111, False, "fp32bulk", "hu"), (2, 182, False, "fp64", "sd"),
     (2, 182, False, "fp32bulk", "ga"), (1, 111, True, "fp64", "hu"), (1, 111, True, "fp32bulk", "ga"),
-    (2, 128, True, "fp32bulk", "dg"), (2, 128, True, "fp64", "sd")])
+    (2, 128, True, "fp32bulk", "dg"), (2, 128, True, "fp64", "sd"), (1, 91, True, "fp64", "dg")])
 def test_tri_large_low_order_steps(p, n, viscous, precision, corr):
     """Two steps of meshes above those counts: the stage updates, and the traces across tiles that each stage leaves
     for the next and the first step for the second (set_state forms them only once)."""

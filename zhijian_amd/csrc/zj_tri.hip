@@ -741,8 +741,9 @@ template <typename R, int P> struct TriViscTile {
     static constexpr bool BIG = sizeof(R) == 8 && P == 5;
     static constexpr int G = BIG ? 1 : 2, WV = BIG ? 8 : 4;
     static constexpr int value = 4 * G * WV;
-    // P1 and FP32 P2 meshes of at least this many elements take the scalar form, in tiles of 64
-    static constexpr int SCALAR_FROM = P == 1 ? 24576 : (P == 2 && sizeof(R) == 4 ? 32768 : INT_MAX);
+    // P1 and FP32 P2 meshes of at least this many elements take the scalar form, in tiles of 64 (FP64 P1: two
+    // workgroups fit on a CU, so at 32 elements each the 256 CUs hold 16,384 elements at a time)
+    static constexpr int SCALAR_FROM = P == 1 ? (sizeof(R) == 8 ? 16384 : 24576) : (P == 2 && sizeof(R) == 4 ? 32768 : INT_MAX);
     static constexpr int tile(int E) { return E >= SCALAR_FROM ? TILE : value; }
     // rows of an element's region: Q_x, then F_r, at 0; Q_y, then F_s, at NP; U at RU; then the
     // gradient traces x (later the common fluxes) at 0 and y at NFP, the partner's U traces at
@@ -1120,7 +1121,8 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
 // scalar operands.  A point has few operator entries there, and padding to
 // blocks of four costs the matrix-core form a third of its rows; but its
 // tiles of 64 leave a small mesh's CUs idle.  us a stage, this / matrix cores:
-// P1 FP64 32,768 elements 13 / 17, 16,200 10.5 / 9.5, 7,200 10 / 7; P1 FP32
+// P1 FP64 32,768 elements 13 / 17, 16,200 10.5 / 9.5, 7,200 10 / 7 (a whole
+// step at 24,200 elements 43 / 47, at 20,000 42 / 45.5, at 16,200 35 / 32); P1 FP32
 // 80,000 20 / 22, 16,200 9 / 7; P2 FP32 80,000 36 / 37, 32,768 16.7 / 17.1,
 // 16,200 14 / 10 (P2 FP64 80,000 85 / 59).  The point values (U, then Q) live
 // in LDS, each lane reads a point's four variables there.
