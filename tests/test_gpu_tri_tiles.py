@@ -82,9 +82,11 @@ def test_tri_form_by_size(p, n, viscous, precision):
 @pytest.mark.parametrize("p,n,viscous,precision,corr", [
     (1, 111, False, "fp64", "ga"), (1, 111, False, "fp32bulk", "hu"), (2, 182, False, "fp64", "sd"),
     (2, 182, False, "fp32bulk", "ga"), (1, 111, True, "fp64", "hu"), (1, 111, True, "fp32bulk", "ga"),
-    (2, 128, True, "fp32bulk", "dg"), (2, 128, True, "fp64", "sd"), (1, 91, True, "fp64", "dg")])
+    (2, 128, True, "fp32bulk", "dg"), (2, 128, True, "fp64", "sd"), (1, 91, True, "fp64", "dg"),
+    (2, 148, False, "fp64", "dg"), (2, 156, False, "fp32bulk", "hu"), (2, 158, False, "fp64", "dg")])
 def test_tri_large_low_order_steps(p, n, viscous, precision, corr):
-    """Two steps of meshes above those counts: the stage updates, and the traces across tiles that each stage leaves
+    """Two steps of meshes above those counts (and of P2 Euler meshes of 43,808 to 49,928 elements, on both sides of
+    the count that the tiles of 64 divide evenly over the CUs): the stage updates, and the traces across tiles that each stage leaves
     for the next and the first step for the second (set_state forms them only once)."""
     say(f"case: triangle steps {'viscous' if viscous else 'inviscid'}, {2 * n * n} elements P{p} {precision} hllc/{corr}")
     m = cases.split_tri_mesh(n, jitter=0.2, seed=n)

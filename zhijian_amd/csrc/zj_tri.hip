@@ -456,11 +456,22 @@ template <typename R, int P> struct TriTile {
     static constexpr int PB = (NP + 3) / 4, FB = (NFP + 3) / 4, CB = (2 * NP + 3) / 4;
     static constexpr bool BIG = sizeof(R) == 8 && P == 5;
     static constexpr int G = BIG ? 1 : 2, WV = BIG ? 8 : 4, value = 4 * G * WV, WPE = sizeof(R) == 8 && P >= 4 ? 2 : 3;
+    // P1 and P2 meshes of at least SCALAR_FROM elements take the scalar form.  So do P2 meshes from HALF_FROM to
+    // HALF_TO elements where it gives the busiest of the 256 CUs half as many of its tiles of 64 as the matrix-core
+    // form gives of 32: only a last round of fewer makes the latter the quicker there.  us a step, scalar / matrix
+    // cores: FP64 26,912 elements 45.5 / 46.2 (2 against 4 tiles), 39,200 56.4 / 54.6 (3, 5), 43,808 57.9 / 61.8
+    // (3, 6), 49,928 76.8 / 69.0 (4, 7), 60,552 81.3 / 76.6 (4, 8); FP32 39,200 41.7 / 37.9, 43,808 42.8 / 44.5,
+    // 52,488 48.7 / 49.1, 60,552 50.5 / 52.9
+    static constexpr int SCALAR_FROM = P == 1 ? 24576 : (P == 2 ? 65536 : INT_MAX);
+    static constexpr int HALF_FROM = P == 2 ? (sizeof(R) == 8 ? 24576 : 40960) : INT_MAX;
+    static constexpr int HALF_TO = sizeof(R) == 8 ? 49152 : SCALAR_FROM;
+    static constexpr int per_cu(int E, int t) { return ((E + t - 1) / t + 255) / 256; }
+    static constexpr bool scalar(int E) {
+        return E >= SCALAR_FROM || (E >= HALF_FROM && E <= HALF_TO && 2 * per_cu(E, TILE) <= per_cu(E, value));
+    }
+    static constexpr int tile(int E) { return scalar(E) ? TILE : value; }
     // rows of an element: traces of U; then U, later F_r, and F_s, later the common fluxes and the
     // other tiles' traces
-    // P1 and P2 meshes of at least this many elements take the scalar form
-    static constexpr int SCALAR_FROM = P == 1 ? 24576 : (P == 2 ? 65536 : INT_MAX);
-    static constexpr int tile(int E) { return E >= SCALAR_FROM ? TILE : value; }
     static constexpr int RU = 4 * FB, RO = RU + NFP;
     static constexpr int ROWS = RU + 4 * CB > RO + 4 * FB ? RU + 4 * CB : RO + 4 * FB;
     static constexpr int ESX = tri::elem_stride<R>(ROWS);
@@ -3342,7 +3353,7 @@ hipError_t tri_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
     auto launch = [&](auto m) {
         constexpr int MODE = decltype(m)::value;
         if constexpr (TV::SCALAR_FROM < INT_MAX)
-            if (a.E >= TV::SCALAR_FROM) {
+            if (TV::scalar(a.E)) {
                 klaunch(tri_scalar_kernel<R, P, MODE>, grid, dim3(BLOCK), 0, s, a);
                 return;
             }
