@@ -107,6 +107,40 @@ def test_tri_large_low_order_steps(p, n, viscous, precision, corr):
     assert l2 < 0.1  # stage 3's residual, a few per cent of a step away from the new state's
 
 
+@pytest.mark.parametrize("p,n,precision", [(1, 91, "fp32bulk"), (2, 158, "fp64"), (2, 160, "fp32bulk"), (3, 317, "fp64"),
+                                           (3, 317, "fp32bulk"), (5, 224, "fp64"), (5, 317, "fp32bulk")])
+def test_tri_large_residual(p, n, precision):
+    """A residual alone of meshes whose stages take the matrix-core form, in the scalar form with its tiles of 64: the
+    traces that steps left for tiles of 32 suffice, and the norm counts the residual's own tiles.  Against the stage
+    form's values on the same state and mesh, by the difference a vanishing step makes: dU = dt R to the rounding of
+    the state, 1e-16 |U| / (dt |R|)."""
+    say(f"case: triangle residual after a step, {2 * n * n} elements P{p} {precision} hllc/ga")
+    m = cases.split_tri_mesh(n, jitter=0.2, seed=n)
+    s = TriSolver(m.xy, m.tris, p, periodic=(1.0, 1.0), riemann="hllc", precision=precision, corr="ga")
+    assert s.info()["elems_per_block"] == 32
+    U = _state(m, p, n)
+    s.set_state(U)
+    dt = 0.5 * s.dt_cfl(0.5)
+    s.rk3_step(dt)
+    U1 = s.get_state()
+    R = s.residual()
+    assert abs(s.residual_l2() / np.linalg.norm(R) - 1) < 1e-12
+    s.rk3_step(1e-3 * dt)
+    d = rel((s.get_state() - U1) / (1e-3 * dt), R)
+    rounding = 4e-16 * np.linalg.norm(U1) / (1e-3 * dt * np.linalg.norm(R))
+    say(f"  rel L2 {d:.3e}, rounding {rounding:.3e}")
+    # the step's own curvature is 1e-3 dt / 2 times the residual's rate of change, of the CFL number's order
+    assert d < 5e-4 + rounding + BAR[precision]
+    r2 = rel(_residual_of(s, U1), R)
+    say(f"  after a trace of every edge {r2:.3e}")
+    assert r2 < 1e-13 if precision == "fp64" else r2 < 1e-6
+
+
+def _residual_of(s, U):
+    s.set_state(U)
+    return s.residual()
+
+
 @pytest.mark.parametrize("p,precision", [(1, "fp64"), (1, "fp32bulk"), (2, "fp64")])
 def test_tri_large_low_order_boundaries(p, precision):
     """The same with boundary faces (far field, outflow, slip wall and no-slip wall, one type per side)."""

@@ -222,12 +222,13 @@ template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return _
 
 // The stage of large meshes at P1 and P2: lanes one per (element, variable),
 // the operators as scalar operands (see the file's head); higher orders and
-// small meshes take tri_stage_kernel below.  us a stage, this / that: P1 FP64
+// small meshes take tri_stage_kernel below (TriTile has the rules; residuals
+// alone come here at other orders, too).  us a stage, this / that: P1 FP64
 // 51,200 elements 11.7 / 15.7, 16,200 7.6 / 7.2, 7,200 7.5 / 5.5; P2 FP64
 // 500,000 166 / 182, 51,200 24 / 21; P2 FP32 80,000 17 / 18, 51,200 14 / 14,
 // 32,768 11 / 9.5.
 template <typename R, int P, int MODE>
-__global__ __launch_bounds__(BLOCK) void tri_scalar_kernel(TriArgs<R> a) {
+__global__ __launch_bounds__(BLOCK, (sizeof(R) == 8 && P == 3 ? 3 : 1)) void tri_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
     constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
     constexpr int NW = NP > NFP ? NP : NFP;
@@ -470,6 +471,15 @@ template <typename R, int P> struct TriTile {
         return E >= SCALAR_FROM || (E >= HALF_FROM && E <= HALF_TO && 2 * per_cu(E, TILE) <= per_cu(E, value));
     }
     static constexpr int tile(int E) { return scalar(E) ? TILE : value; }
+    // A residual alone reads no U^n, which is what the scalar form's FP64 stages 2 and 3 wait for: large meshes
+    // take it for that (its tiles of 64 are whole tiles of the other's, so the traces it needs are there).  us, with
+    // the conversion of the result, scalar / matrix cores: P1 FP32 20,000 elements 9.5 / 10.0; P2 FP64 60,552
+    // 27.7 / 30.6, FP32 52,488 21.1 / 22.4; P3 FP32 500,000 166 / 175, 180,000 64 / 63; P5 FP64 500,000 635 / 722
+    // (572 in builds whose operator table falls well into the scalar cache), 180,000 248 / 267, 80,000 115 / 115; P5 FP32 500,000 380 / 410, 259,200 221 / 224; P4 500,000 434 / 424
+    static constexpr int RESIDUAL_FROM =
+        P == 1 ? 16384 : P == 2 ? HALF_FROM : P == 3 ? 200000 : P == 5 ? (sizeof(R) == 8 ? 100000 : 200000) : INT_MAX;
+    static constexpr bool scalar_residual(int E) { return scalar(E) || E >= RESIDUAL_FROM; }
+    static constexpr int residual_tile(int E) { return scalar_residual(E) ? TILE : value; }
     // rows of an element: traces of U; then U, later F_r, and F_s, later the common fluxes and the
     // other tiles' traces
     static constexpr int RU = 4 * FB, RO = RU + NFP;
@@ -3349,11 +3359,12 @@ __global__ __launch_bounds__(BLOCK) void tri_dt_kernel(const double* __restrict_
 template <typename R, int P>
 hipError_t tri_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
     using TV = TriTile<R, P>;
-    const int TT = TV::tile(a.E), grid = (std::max(a.E, 1) + TT - 1) / TT;
     auto launch = [&](auto m) {
         constexpr int MODE = decltype(m)::value;
-        if constexpr (TV::SCALAR_FROM < INT_MAX)
-            if (TV::scalar(a.E)) {
+        const int TT = MODE == MODE_RESIDUAL ? TV::residual_tile(a.E) : TV::tile(a.E);
+        const int grid = (std::max(a.E, 1) + TT - 1) / TT;
+        if constexpr ((MODE == MODE_RESIDUAL ? TV::RESIDUAL_FROM : TV::SCALAR_FROM) < INT_MAX)
+            if (TT == TILE) {
                 klaunch(tri_scalar_kernel<R, P, MODE>, grid, dim3(BLOCK), 0, s, a);
                 return;
             }
@@ -3446,6 +3457,16 @@ int tri_tile(int P, bool fp64, int E) {
     case 3: return fp64 ? TriTile<double, 3>::tile(E) : TriTile<float, 3>::tile(E);
     case 4: return fp64 ? TriTile<double, 4>::tile(E) : TriTile<float, 4>::tile(E);
     default: return fp64 ? TriTile<double, 5>::tile(E) : TriTile<float, 5>::tile(E);
+    }
+}
+
+int tri_residual_tile(int P, bool fp64, int E) {
+    switch (P) {
+    case 1: return fp64 ? TriTile<double, 1>::residual_tile(E) : TriTile<float, 1>::residual_tile(E);
+    case 2: return fp64 ? TriTile<double, 2>::residual_tile(E) : TriTile<float, 2>::residual_tile(E);
+    case 3: return fp64 ? TriTile<double, 3>::residual_tile(E) : TriTile<float, 3>::residual_tile(E);
+    case 4: return fp64 ? TriTile<double, 4>::residual_tile(E) : TriTile<float, 4>::residual_tile(E);
+    default: return fp64 ? TriTile<double, 5>::residual_tile(E) : TriTile<float, 5>::residual_tile(E);
     }
 }
 
@@ -3985,7 +4006,11 @@ static hipError_t tenqueue(zj_tri* h, int mode, hipStream_t s) {
     else
         e = h->prec == ZJ_PREC_FP64 ? tri_launch<double>(h->P, mode, tri_args<double>(h, mode), s)
                                     : tri_launch<float>(h->P, mode, tri_args<float>(h, mode), s);
-    if (e == hipSuccess && (mode == MODE_RESIDUAL || mode == MODE_STAGE3)) h->l2_blocks = h->nblk;
+    if (e == hipSuccess && mode == MODE_STAGE3) h->l2_blocks = h->nblk;
+    if (e == hipSuccess && mode == MODE_RESIDUAL) {
+        const int tt = h->viscous ? h->epb : tri_residual_tile(h->P, h->prec == ZJ_PREC_FP64, h->E);
+        h->l2_blocks = (h->E + tt - 1) / tt;
+    }
     return e;
 }
 
