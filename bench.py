@@ -459,8 +459,7 @@ def time_tri(n, p, steps, warmup, err_steps, stream, hiprt, cpu_seconds, Re=None
         ms_adj = e0.elapsed_ms(e1) / k
         out[name]["adjoint"] = dict(
             adj_ms_per_step=ms_adj, adjoint_over_forward=ms_adj / out[name]["ms_per_step"],
-            note="adjoint step = traces of U^n " + ("and of the two recomputed stages " if Re else "")
-                 + "+ stages 1-2 recomputed + 3 VJP launches")
+            note="adjoint step = " + ("" if Re else "traces of U^n + ") + "stages 1-2 recomputed + 3 VJP launches")
     for s in sols.values():
         s.close()
     if cpu_seconds > 0:

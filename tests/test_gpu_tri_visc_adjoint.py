@@ -132,7 +132,7 @@ def test_tri_viscous_vjp_numbering_independent():
 
 
 def test_tri_viscous_vjp_fp64_p5():
-    """FP64 P5: the adjoint's 16-element tile takes 91 KiB of LDS (one
+    """FP64 P5: the adjoint's 16-element tile takes 146 KiB of LDS (one
     workgroup per CU); residual and one step against the oracle."""
     say("case: triangle viscous FP64 P5 residual and step VJP, periodic 6x6 roe/dg Re 100")
     s, o, m = _pair(6, 5, "roe", seed=5)

@@ -33,9 +33,10 @@
 //            lanes of a wave (16 elements x 4 variables) touch 512 contiguous
 //            bytes per solution point (W = U1, then U2 in place)
 //   T[3]     flux-point traces [E][3(p+1)][4] in the compute precision;
-//            only edges whose neighbour lies in another tile of 64 elements are
-//            written (a neighbour in the same tile is read from LDS), rotating
-//            as the quadrilateral path's: stage 1 T0->T1, 2 T1->T2, 3 T2->T0
+//            only edges whose neighbour lies in another tile (of 32 elements,
+//            64 in the scalar forms) are written (a neighbour in the same tile
+//            is read from LDS), rotating as the quadrilateral path's: stage 1
+//            T0->T1, 2 T1->T2, 3 T2->T0
 //   geo      [E][10]: r_x, r_y, s_x, s_y, then the face normal (as the face's
 //            left element sees it) of edges 0, 1, 2
 //   edge     [E][6]: |e|/(2J) of each edge and of the neighbour's side of each
@@ -118,14 +119,15 @@ __constant__ float c_ops32[OPS_TOTAL];
 
 // BR2 face liftings, per order and correction family (DG, SD = GA, HU):
 // LF_k = interp(edge k rows) . lift(edge k columns), [3][FP][FP] -- the lifting
-// of one edge's jumps evaluated at that edge's own flux points.
+// of one edge's jumps evaluated at that edge's own flux points.  For the scalar
+// forms, which exist at P1 and P2.
 constexpr int lf_words(int P) { return 9 * (P + 1) * (P + 1); }
 constexpr int lf_offset(int P) {
     int o = 0;
     for (int q = 1; q < P; ++q) o += 3 * lf_words(q);
     return o;
 }
-constexpr int LF_TOTAL = lf_offset(6);
+constexpr int LF_ORDERS = 2, LF_TOTAL = lf_offset(LF_ORDERS + 1);
 inline int lf_family(int corr) { return corr == ZJ_CORR_DG ? 0 : (corr == ZJ_CORR_HU ? 2 : 1); }
 __constant__ double c_lf64[LF_TOTAL];
 __constant__ float c_lf32[LF_TOTAL];
@@ -511,7 +513,7 @@ __global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) voi
     const int e0 = tile * TT;
     const R g = R(a.gamma);
     auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };  // this lane's element of group q
-        auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };
+    auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };
 
     const PointRows<NP, G> rows(e0, wave, lane, a.E);
 
@@ -740,8 +742,8 @@ __global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) voi
 // takes one lane per point or face point through LDS.  Traces across tiles
 // carry 12 words per flux point ([E][3(p+1)][12]: U, dU/dx, dU/dy).
 //
-// What bounds it is the latency of LDS and memory at two (FP64) to four
-// waves per SIMD, then VALU issue (about 1,400 instructions per wave of
+// What bounds it is the latency of LDS and memory at two (FP64) or three
+// (FP32 P2, P3) waves per SIMD, then VALU issue (about 1,400 instructions per wave of
 // eight elements) beside 4,400 (FP64) cycles of matrix-core work.  Hence no
 // branches around loads (rows in excess, in-tile edges and elements beyond
 // the mesh read a valid address and select afterwards: branches had split
@@ -805,7 +807,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
     const int e0 = tile * TT;
     const R g = R(a.gamma), mu = R(a.mu), kappa = R(a.kappa), eta = R(a.eta);
     auto elg = [&](int q) { return (wave * G + q) * 4 + ((lane >> 2) & 3); };  // this lane's element of group q
-        auto st = [](int elx, int j) { return elx * ESF + j * NV; };               // trace slots
+    auto st = [](int elx, int j) { return elx * ESF + j * NV; };                 // trace slots
     auto sx_ = [](int elx, int r) { return elx * ESX + r * NV; };              // rows of the other region
 
     const PointRows<NP, G> rows(e0, wave, lane, a.E);
@@ -1147,12 +1149,12 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
 // 80,000 20 / 22, 16,200 9 / 7; P2 FP32 80,000 36 / 37, 32,768 16.7 / 17.1,
 // 16,200 14 / 10 (P2 FP64 80,000 85 / 59).  The point values (U, then Q) live
 // in LDS, each lane reads a point's four variables there.
-template <typename R, int P, int MODE, int TT>
-__global__ __launch_bounds__(TT * NV) void tri_visc_scalar_kernel(TriArgs<R> a) {
+template <typename R, int P, int MODE>
+__global__ __launch_bounds__(BLOCK) void tri_visc_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
     constexpr int NP = S::NP, FP = S::FP, NFP = S::NFP;
-    constexpr int NB = TT * NV, NWV = NB / 64;
-    static_assert(NB % 64 == 0 && 2 * NP >= NFP, "tile and point-array layout");
+    constexpr int TT = TILE, NB = BLOCK, NWV = NB / 64;
+    static_assert(2 * NP >= NFP, "point-array layout");
     using OP = TriOps<P>;
     constexpr int O0 = ops_offset(P), CA = OP::CA, OI = O0 + OP::C;
     const int OLT = O0 + a.lift_off;
@@ -1622,7 +1624,7 @@ __global__ __launch_bounds__(BLOCK, 2) void tri_visc_trace_kernel(int E, const d
 // ------------------------------------------------------------ adjoint
 // Vector-Jacobian product of one triangle stage u_n = a U^n + b q + c dt R(q)
 // (MODE_STAGE1..3), or of the residual alone (MODE_RESIDUAL).  The forward
-// values are recomputed as tri_stage_kernel forms them; then, per lane
+// values are recomputed as tri_scalar_kernel forms them; then, per lane
 // (element, variable):
 //   R1  cotangent of u_out: its partial value plus the transposed trace
 //       operator on the edge cotangents other tiles left (cross-tile edges);
@@ -2054,7 +2056,9 @@ template <typename R, int P> struct TriViscVjpTile {
     static constexpr int LARGE_FROM = sizeof(R) == 8 || P > 2 ? INT_MAX : P == 1 ? 16384 : 24576;
     static constexpr int tile(int E) { return E >= LARGE_FROM ? TILE : 4 * G * WV; }
     // waves per SIMD asked for: in FP64 the face points' VJPs take more than the 256 VGPRs of two (P2:
-    // 584 us a step at one wave, 707 at two with scratch), P5's LDS allows one workgroup
+    // 584 us a step at one wave, 707 at two with scratch), P5's LDS allows one workgroup.  FP64 P1 at two keeps 180
+    // bytes a lane in scratch and is the quicker of them on large meshes: 500,000 elements 2139 us a step, tiles of
+    // 32 at one wave without scratch 2522 (80,000 322 / 383, 16,200 77 / 79, 800 58 / 44)
     static constexpr int WPE = (sizeof(R) == 8 ? P == 1 : P < 5) ? 2 : 1;
     // rows of an element's region: Q_x, Q_y, the point fluxes' cotangents x, y, U (RU); later the
     // gradient traces x and y, the partner's U traces and the flux differences' cotangents
@@ -3401,7 +3405,7 @@ hipError_t tri_visc_launch_p(int mode, const TriArgs<R>& a, hipStream_t s) {
             constexpr int MODE = decltype(m)::value;
             if constexpr (TV::SCALAR_FROM < INT_MAX)
                 if (a.E >= TV::SCALAR_FROM) {
-                    klaunch(tri_visc_scalar_kernel<R, P, MODE, TILE>, grid, dim3(BLOCK), 0, s, a);
+                    klaunch(tri_visc_scalar_kernel<R, P, MODE>, grid, dim3(BLOCK), 0, s, a);
                     return;
                 }
             klaunch(tri_visc_stage_kernel<R, P, MODE>, grid, dim3(64 * TV::WV), 0, s, a);
@@ -3672,7 +3676,7 @@ hipError_t load_tri_ops(int device) {
         !frags(std::integral_constant<int, 5>{}))
         return hipErrorInvalidValue;
     std::vector<double> lf((size_t)LF_TOTAL, 0.0);
-    for (int P = 1; P <= 5; ++P) {
+    for (int P = 1; P <= LF_ORDERS; ++P) {
         for (int fam = 0; fam < 3; ++fam) {
             tri::Operators O;
             if (!tri::operators(P, O, fam == 0 ? ZJ_CORR_DG : (fam == 1 ? ZJ_CORR_SD : ZJ_CORR_HU)))

@@ -120,7 +120,8 @@ constexpr int visc_threads() {
 
 // FP64 P4 and P5: 39 KB of LDS instead of 46, so four workgroups fit on a CU
 // and not three (256x256 P4, four steps with their set-up: 1664 -> 1510 us; a
-// 128x128 P5 stage 55.6 -> 52.9 us).  At P3 four would still not fit (41,312
+// 128x128 P5 stage 55.6 -> 52.9 us; a step at 60x60 and below, where a CU gets
+// two workgroups or fewer, is 1 to 2% longer: P4 35.0 -> 35.3 and 48.9 -> 49.6).  At P3 four would still not fit (41,312
 // of 40,960 bytes each), and FP32's count is set by its registers.
 template <typename R, int P>
 constexpr bool visc_traces_over_state() {
@@ -589,9 +590,9 @@ __global__ __launch_bounds__(BLOCK) void visc_trace_kernel(int E, const double* 
 // what counts is the waves per SIMD.  Four point and four trace arrays whose
 // roles follow one another (66 KB at FP64 P3) let two workgroups share a CU
 // where one array per quantity (123 KB) let one; the registers are held to
-// the same (256) by reading a face's traces again behind its Riemann VJP and
-// by keeping the cotangent of q in LDS over R4.  Solving an in-tile face once
-// halves R4's flux VJPs.  128x128 P3 FP64, a checkpointed gradient over 32
+// the same (256; P4 and P5 keep 12 bytes a lane in scratch) by reading a face's
+// traces again behind its Riemann VJP and by keeping the cotangent of q in LDS
+// over R4.  Solving an in-tile face once halves R4's flux VJPs.  128x128 P3 FP64, a checkpointed gradient over 32
 // steps (96 forward stages and 96 of these): 9.40 -> 7.09 ms.  A step
 // backwards at 128x128, us, P1..P5: FP64 143, 273, 297, 500, 694 -> 118, 209,
 // 228, 383, 506; FP32-bulk 105, 234, 167, 287, 377 -> 91, 153, 163, 247, 318.
