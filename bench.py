@@ -629,6 +629,47 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
+# Sections of the record of which the output line holds the figures alone.
+DETAIL = ("adjoint", "batched", "textbook", "navier_stokes", "triangles", "gpu_api", "vortex", "io")
+FIGURES = ("ms_per_step", "dof_updates_per_s", "frac", "adj_ms_per_step", "adjoint_over_forward",
+           "gradient_over_forward", "gradient_ms", "rel_l2", "ms", "save_gbps", "load_gbps", "value")
+LINE_MAX = 8000  # characters: a reader of the output's end gets the line whole
+
+
+def figures(x):
+    """A section's figures: its named numbers, nested as it is, without workloads, notes and lists."""
+    out = {}
+    for k, v in x.items():
+        if isinstance(v, dict):
+            f = figures(v)
+            if f:
+                out[k] = f
+        elif k in FIGURES and isinstance(v, (int, float)):
+            out[k] = v
+    return out
+
+
+def rounded(x, digits):
+    if isinstance(x, float):
+        return float(f"{x:.{digits}g}")
+    if isinstance(x, dict):
+        return {k: rounded(v, digits) for k, v in x.items()}
+    return [rounded(v, digits) for v in x] if isinstance(x, list) else x
+
+
+def output_line(record):
+    """The one line of standard output: the record with its sections' figures in five digits, and without
+    the longest sections should it still exceed LINE_MAX (the whole record goes to standard error)."""
+    out = {k: rounded(figures(v), 5) if k in DETAIL and v else v for k, v in record.items()}
+    line = json.dumps(out)
+    for k in sorted((k for k in DETAIL if out.get(k)), key=lambda k: -len(json.dumps(out[k]))):
+        if len(line) <= LINE_MAX:
+            break
+        out[k] = "on standard error"
+        line = json.dumps(out)
+    return line
+
+
 def time_precision(sol, U0, dt, steps, warmup, stream, hiprt):
     """Graph-replayed steps and per-stage kernel times (ms)."""
     sol.set_state(U0)
@@ -979,7 +1020,8 @@ def main():
         "io": io_res,
         "copy_kernel_gbps": copy_gbps,
     }
-    print(json.dumps(out), flush=True)
+    log("record: " + json.dumps(out))
+    print(output_line(out), flush=True)
 
 
 def reap_children():
