@@ -39,7 +39,7 @@
 //            T0->T1, 2 T1->T2, 3 T2->T0
 //   geo      [E][10]: r_x, r_y, s_x, s_y, then the face normal (as the face's
 //            left element sees it) of edges 0, 1, 2
-//   edge     [E][6]: |e|/(2J) of each edge and of the neighbour's side of each
+//   edge     [E][3][2]: |e|/(2J) of each edge and of the neighbour's side of it
 //            (0 on a boundary), for the matrix-core kernels; apart from geo,
 //            whose words the others read alone
 //   links    [E][3] int2: x = neighbour element (-1 on a boundary), y = packed
@@ -80,7 +80,7 @@ struct TriShape {
 constexpr int TILE = BLOCK / NV;  // elements per workgroup (one lane per element and variable)
 constexpr int EB = 16;            // elements per block of the state and trace layouts
 constexpr int GEO = 10;           // geometry words per element
-constexpr int EDG = 6;            // edge factors per element: own, then the neighbour's
+constexpr int EDG = 6;            // edge factors per element: own and the neighbour's, edge by edge
 
 // Operator tables of order P in constant memory, laid out for wide scalar
 // loads in the kernels' loops:
@@ -541,7 +541,7 @@ __global__ __launch_bounds__((64 * TriTile<R, P>::WV), (TriTile<R, P>::WPE)) voi
         const int nl = Lk.x - e0, ek = link_edge(Lk.y), role = link_role(Lk.y);
         const bool right = role == ROLE_RIGHT, live = e0 + el < a.E, bnd = role == ROLE_BOUNDARY;
         const bool in = !bnd && nl >= 0 && nl < TT;
-        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + 2 * k], sn = a.edge[(int64_t)e * EDG + 2 * k + 1], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R ns[4] = {nx, ny, right ? -s : s, right ? sn : -sn};
         store4(sNs + 4 * tid, ns);
         const bool self = !live || !in;
@@ -837,7 +837,7 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
         const int nl = Lk.x - e0, ek = link_edge(Lk.y);
         const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
         const bool in = !live || (nl >= 0 && nl < TT);  // beyond the mesh: its own neighbour
-        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + 2 * k], sn = a.edge[(int64_t)e * EDG + 2 * k + 1], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
         const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, right ? sn : -sn};
         store4(sEw + 4 * tid, we);
@@ -2134,7 +2134,7 @@ __global__ __launch_bounds__(64 * NWV, (TriViscVjpTile<R, P>::WPE)) void tri_vis
         const int nl = Lk.x - e0, ek = link_edge(Lk.y);
         const bool right = link_role(Lk.y) == ROLE_RIGHT, live = e0 + el < a.E;
         const bool in = !live || (nl >= 0 && nl < TT);
-        const R s = a.edge[(int64_t)e * EDG + k], sn = a.edge[(int64_t)e * EDG + 3 + k], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
+        const R s = a.edge[(int64_t)e * EDG + 2 * k], sn = a.edge[(int64_t)e * EDG + 2 * k + 1], nx = Ge[4 + 2 * k], ny = Ge[5 + 2 * k];
         const R w = right ? -s : s, wn = right ? -eta * sn : eta * sn;
         const R we[4] = {w * nx, w * ny, wn * nx, wn * ny}, ns[4] = {nx, ny, w, in ? (right ? sn : -sn) : R(0)};
         store4(sEw + 4 * tid, we);
@@ -3883,8 +3883,8 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
         for (int c = 0; c < 4; ++c) ge[c] = met[(size_t)o * 4 + c];
         double* ed = &edge[(size_t)e * EDG];
         ed[0] = std::sqrt(ge[2] * ge[2] + ge[3] * ge[3]);
-        ed[1] = std::sqrt((ge[0] + ge[2]) * (ge[0] + ge[2]) + (ge[1] + ge[3]) * (ge[1] + ge[3]));
-        ed[2] = std::sqrt(ge[0] * ge[0] + ge[1] * ge[1]);
+        ed[2] = std::sqrt((ge[0] + ge[2]) * (ge[0] + ge[2]) + (ge[1] + ge[3]) * (ge[1] + ge[3]));
+        ed[4] = std::sqrt(ge[0] * ge[0] + ge[1] * ge[1]);
     }
     std::vector<double> hcd((size_t)E);
     for (int e = 0; e < E; ++e) hcd[(size_t)e] = hc[(size_t)(perm.empty() ? e : perm[(size_t)e])];
@@ -3927,7 +3927,7 @@ static int tbuild(zj_tri* h, const zj_tri_desc* m, const zj_params* p) {
     for (size_t k = 0; k < links.size(); ++k) {
         if (links[k].y == -1) return tfail(h, ZJ_ERR_ARG, "an element edge has no face");
         if (links[k].x >= 0)
-            edge[k / 3 * EDG + 3 + k % 3] = edge[(size_t)links[k].x * EDG + (links[k].y & 7)];
+            edge[k * 2 + 1] = edge[(size_t)links[k].x * EDG + 2 * (links[k].y & 7)];
     }
 
     ZJ_THIP(h, hipSetDevice(h->device));
