@@ -1144,11 +1144,14 @@ __global__ __launch_bounds__((64 * TriViscTile<R, P>::WV), 2) void tri_visc_stag
 // scalar operands.  A point has few operator entries there, and padding to
 // blocks of four costs the matrix-core form a third of its rows; but its
 // tiles of 64 leave a small mesh's CUs idle.  us a stage, this / matrix cores:
-// P1 FP64 32,768 elements 13 / 17, 16,200 10.5 / 9.5, 7,200 10 / 7 (a whole
-// step at 24,200 elements 43 / 47, at 20,000 42 / 45.5, at 16,200 35 / 32); P1 FP32
+// P1 FP64 32,768 elements 13 / 17, 16,200 10.5 / 9.5, 7,200 10 / 7; P1 FP32
 // 80,000 20 / 22, 16,200 9 / 7; P2 FP32 80,000 36 / 37, 32,768 16.7 / 17.1,
-// 16,200 14 / 10 (P2 FP64 80,000 85 / 59).  The point values (U, then Q) live
-// in LDS, each lane reads a point's four variables there.
+// 16,200 14 / 10 (P2 FP64 80,000 85 / 59).  Whole steps: P1 FP64 24,200
+// elements 43 / 47, 20,000 42 / 45.5, 16,200 35 / 32; P1 FP32 24,200 35.4 /
+// 32.9, 25,088 35.0 / 35.7, 51,200 44 / 56; P2 FP32 32,768 54.9 / 56.5, 51,200
+// 96 / 84, 125,000 164 / 171, 500,000 634 / 623: within 5% on either side
+// but for 50,000 to 65,000 elements.  The point values (U, then Q) live in
+// LDS, each lane reads a point's four variables there.
 template <typename R, int P, int MODE>
 __global__ __launch_bounds__(BLOCK) void tri_visc_scalar_kernel(TriArgs<R> a) {
     using S = TriShape<P>;
